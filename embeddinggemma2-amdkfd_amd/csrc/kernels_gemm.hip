@@ -43,10 +43,10 @@
 
 #include "eg2_device.hpp"
 #include "eg2_kernels.hpp"
+#include "gemm_narrow.hpp"
 
 namespace eg2 {
 
-typedef int intx4 __attribute__((ext_vector_type(4)));
 typedef int intx16 __attribute__((ext_vector_type(16)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -54,8 +54,6 @@ constexpr int kXcds = 8;     // MI355X: 8 XCDs of 32 CUs, each with its own L2
 constexpr int kDepth = 3;    // blocks in flight per wave in gemm_q8_kernel (93 VGPRs: five waves per SIMD)
 constexpr int kUnroll = 6;   // its loop's unrolling: slots rotate mod kDepth, MFMA results mod 2
 constexpr int kTile = 1024;  // one 32 x 32 int8 operand block
-constexpr float kMagic = 12582912.0f;         // 1.5 * 2^23
-constexpr int kMagicBits = 0x4B400000;
 
 extern __shared__ __align__(16) unsigned char gemm_lds[];
 
@@ -366,12 +364,39 @@ static hipError_t launch_gemm_kernel(dim3 grid, size_t lds, hipStream_t st, cons
 // 4 GiB - 1 bytes (the executor's arrays take a few hundred KB).
 inline bool scales_fit(int k, int ld) { return (uint64_t)(k / kQK) * (uint64_t)ld * 4u <= 0xFFFFFFFFull; }
 
+// Where the narrow kernels (gemm_narrow.hpp) end, measured per launch inside
+// a graph over 24 weight sets (so each launch finds its weights outside the
+// L2, as in the forward), wide / narrow in us:
+//   gemm m 768, k 768:   n 1 5.3 / 2.6, 128 6.5 / 3.2, 512 7.1 / 5.3, 700 6.9 / 7.0
+//   gemm m 768, k 1152:  n 1 7.8 / 3.1, 512 8.9 / 7.0, 700 8.8 / 9.5
+//   gemm m 2304, k 768:  n 192 6.8 / 6.1, 256 7.2 / 7.2
+//   gemm m 768, k 3072:  n 16 17.5 / 5.5, 512 18.5 / 15.6
+// The narrow kernel's time grows with its workgroups (one per 16 x 16 tile,
+// 24 to 48 KB of LDS each), the wide one's hardly until its tiles fill the
+// chip, so the line is a number of tiles.
+constexpr int kNarrowTiles = 1792;
+// gate|up + GeGLU: n 32 8.4 / 5.9, 96 8.7 / 6.1, 192 8.5 / 8.1, 256 8.7 / 10.6
+// (36 workgroups of 53 KB per 16 rows).
+constexpr int kNarrowGegluRows = 192;
+// Q|K|V: the fused kernel gives a head's 256 columns to one workgroup, so 32
+// rows run on 5 CUs; below this the narrow projection (80 workgroups per 16
+// rows) followed by the standalone QK-norm / RoPE in place is faster: n 1
+// 8.3 / 5.1, 64 9.1 / 6.2, 256 9.3 / 8.2, 352 9.3 / 9.7. Same bits.
+constexpr int kNarrowQkvRows = 256;
+
 hipError_t launch_gemm_q8(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd, int ldw,
                           float* y, int n, int m, int k, int ldy, hipStream_t st) {
   if (n <= 0 || m <= 0 || k <= 0 || k % kQK != 0 || ldy < m || ldx < n || ldw < m) return hipErrorInvalidValue;
   if (!scales_fit(k, ldx) || !scales_fit(k, ldw)) return hipErrorInvalidValue;
-  return launch_gemm_kernel<false>(gemm_grid(n, m, true), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, k / kQK, ldy,
-                                   nullptr, nullptr);
+  const int nb = k / kQK;
+  if ((int64_t)((n + 15) / 16) * ((m + 15) / 16) <= kNarrowTiles) {
+    const dim3 grid((m + 15) / 16, (n + 15) / 16);
+    auto* kernel = nb <= 24 ? gemm_q8_narrow_kernel<6> : nb <= 36 ? gemm_q8_narrow_kernel<9> : gemm_q8_narrow_kernel<12>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb, ldy);
+    return hipGetLastError();
+  }
+  return launch_gemm_kernel<false>(gemm_grid(n, m, true), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb, ldy, nullptr,
+                                   nullptr);
 }
 
 hipError_t launch_gemm_q8_geglu(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd, int ldw,
@@ -380,6 +405,11 @@ hipError_t launch_gemm_q8_geglu(const int8_t* xq, const float* xd, int ldx, cons
   if (n <= 0 || ff <= 0 || ff % kQK != 0 || k <= 0 || k % kQK != 0 || ldx < n || ldw < m || ldg < n)
     return hipErrorInvalidValue;
   if (!scales_fit(k, ldx) || !scales_fit(k, ldw)) return hipErrorInvalidValue;
+  if (n <= kNarrowGegluRows) {
+    hipLaunchKernelGGL(gemm_q8_geglu_narrow_kernel, dim3(ff / kQK, (n + 15) / 16), dim3(512), 0, st, xq, xd, ldx, wq, wd,
+                       ldw, n, ff, k / kQK, gq, gd, ldg);
+    return hipGetLastError();
+  }
   // LDS: the epilogue's gate and up tiles
   constexpr size_t lds = 2 * 2 * 32 * kGPitch * sizeof(float);
   return launch_gemm_kernel<true>(gemm_grid(n, m), lds, st, xq, xd, ldx, wq, wd, ldw, nullptr, n, m, k / kQK, ldg, gq,
@@ -516,6 +546,11 @@ hipError_t launch_gemm_q8_qkv_rope(const int8_t* xq, const float* xd, int ldx, c
                                    const int32_t* pos, float eps, float* out, hipStream_t st) {
   if (n <= 0 || k <= 0 || k % kQK != 0 || ldx < n || ldw < kQKVCols) return hipErrorInvalidValue;
   if (!scales_fit(k, ldx) || !scales_fit(k, ldw)) return hipErrorInvalidValue;
+  if (n <= kNarrowQkvRows) {
+    const hipError_t e = launch_gemm_q8(xq, xd, ldx, wq, wd, ldw, out, n, kQKVCols, k, kQKVCols, st);
+    if (e != hipSuccess) return e;
+    return launch_qk_norm_rope(out, q_w, k_w, rope, pos, eps, out, n, st);
+  }
   const XcdRegions reg = xcd_split((n + 31) / 32, kQkvHeads);
   const dim3 grid(kXcds * reg.rows * reg.cols);
   const int nb = k / kQK;
