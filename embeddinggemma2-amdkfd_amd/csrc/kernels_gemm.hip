@@ -28,8 +28,8 @@
 // Work: a workgroup of 4 waves computes a 64 x 64 output tile, wave w the
 // 32 x 32 quarter at rows 32 (w >> 1), columns 32 (w & 1). Each wave loads
 // its own activation and weight blocks and their scales straight into
-// registers by buffer loads, three blocks ahead (93 VGPRs, five waves per
-// SIMD: the 4,608 waves of gate|up all resident), with no LDS and no barrier
+// registers by buffer loads, three blocks ahead (90-95 VGPRs, five waves per
+// SIMD: the 4,608 waves of gate|up all resident), with no barrier
 // (an LDS ring shared by the four waves, with a barrier per block, was no
 // faster: the loop is bound by each wave's instruction stream, 24 or 36
 // blocks of one MFMA and 48 VALU operations, not by its loads). Per block:
@@ -37,7 +37,7 @@
 // adds, then the refill of kb's registers with block kb + 3. In the MFMA
 // 32x32 output layout a lane holds one column and 16 rows; each row's
 // activation scale reaches it through a DPP row broadcast folded into the
-// multiply.
+// multiply, or (gate|up) a small LDS ring of the wave's own (q8_block_loop).
 #include <algorithm>
 #include <utility>
 
@@ -63,20 +63,20 @@ __device__ __forceinline__ float row_bcast(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x150 + V, 0xf, 0xf, true));
 }
 
-// t[v] = (dot[v] * d_w) * d_x(row v) from the biased MFMA result; the
-// lane's 16 output rows take their activation scales from lanes 0..15 of
-// its 16-lane row. The two phases are kept apart so 16 independent
-// operations separate each dependent pair; accumulate_products then adds
-// t to acc (the third phase), after the next block's MFMA is issued.
-template <int... V>
-__device__ __forceinline__ floatx16 scale_products(const intx16& biased, float dw, float dxv,
+// t[v] = (dot[v] * d_w) * d_x(row v) from the biased MFMA result, the
+// activation scale of the lane's output row v given by dx(v). The two phases
+// are kept apart so 16 independent operations separate each dependent pair;
+// accumulate_products then adds t to acc (the third phase), after the next
+// block's MFMA is issued.
+template <typename Dx, int... V>
+__device__ __forceinline__ floatx16 scale_products(const intx16& biased, float dw, Dx dx,
                                                    std::integer_sequence<int, V...>) {
   const float bias = dw * -kMagic;
   const floatx16 f = __builtin_bit_cast(floatx16, biased);
   floatx16 t;
   ((t[V] = __builtin_fmaf(f[V], dw, bias)), ...);
   __builtin_amdgcn_sched_barrier(0);
-  ((t[V] = t[V] * row_bcast<V>(dxv)), ...);
+  ((t[V] = t[V] * dx(std::integral_constant<int, V>{})), ...);
   return t;
 }
 template <int... V>
@@ -215,8 +215,17 @@ __device__ __forceinline__ void geglu_epilogue(const floatx16& acc, int tr, int 
 // projection kernels: the activation block tile atile (1 KB per block, nb
 // blocks) and its scales xd[kb * ldx + xoff / 4] (n rows), the weight block
 // tile btile and its scales wd[kb * ldw + woff / 4] (m rows), xoff being
-// the row whose scale this lane feeds to the DPP broadcast (srow) and woff
-// the lane's column. Operands go straight to registers (the row-tile
+// the row whose scale this lane loads (srow) and woff the lane's column.
+// The scale multiply takes a lane's 16 row scales from a DPP row broadcast,
+// or (LDS) as plain registers read through a 256-byte ring of the wave's own
+// (dx_ring): a SIMD issues a plain v_mul_f32 in 2.4 cycles and a DPP one in
+// 4.3 (measured, four waves), so block and wave cost 145 cycles instead of
+// 193 when the arithmetic bounds. gate|up, whose 4.5 waves per SIMD do fill
+// it, takes the ring: 18.0 -> 16.9 us at 2048 rows, one 16 x 128 wave 2.26
+// -> 2.21 ms. O, down and Q|K|V, with one or two waves per SIMD, keep the
+// DPP: alone they gain 0-5%, but with four waves in flight the step got 1.5%
+// slower (their LDS round trips then sit on the chain and on the LDS that
+// the other waves' attention uses). Operands go straight to registers (the row-tile
 // layout is the MFMA's register order: lane L's 16 bytes of a block are
 // one load at 16 L) by buffer loads with a scalar offset per block, kDepth
 // blocks ahead, with no LDS and no barrier: the waves of a workgroup never
@@ -226,10 +235,10 @@ __device__ __forceinline__ void geglu_epilogue(const floatx16& acc, int tr, int 
 // scalar multiply each rather than a new 64-bit base and descriptor (12
 // scalar instructions fewer per block and wave). Returns the tile in the
 // 32x32 MFMA output layout.
-template <bool TAIL>
+template <bool TAIL, bool LDS>
 __device__ __forceinline__ floatx16 q8_block_loop(const int8_t* atile, const float* __restrict__ xd, int ldx, int n,
                                                   uint32_t xoff, const int8_t* btile, const float* __restrict__ wd,
-                                                  int ldw, int m, uint32_t woff, int nb, int lane) {
+                                                  int ldw, int m, uint32_t woff, int nb, int lane, float* dx_ring) {
   // Buffer loads: the per-block advance is a scalar offset, so no vector
   // address is kept per block in flight.
   const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(atile, (uint32_t)nb * kTile);
@@ -262,6 +271,13 @@ __device__ __forceinline__ floatx16 q8_block_loop(const int8_t* atile, const flo
   }
   intx16 d[2];
   d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[0].a, f[0].b, magic, 0, 0, 0);
+  // LDS: the wave's scales of block kb go into slot kb % 2 of its ring when
+  // they have arrived (before the MFMA of kb) and come back as the lane's 16
+  // rows just before they are used, into the registers of the idle MFMA
+  // result; a wave's LDS accesses stay in order, so no barrier.
+  float* put = dx_ring + (lane & 31);
+  const float* get = dx_ring + 4 * (lane >> 5);
+  if constexpr (LDS) put[0] = f[0].dx;
   floatx16 acc = floatx16{};
   // One block: j = kb % kUnroll (a constant after unrolling, so the
   // fragment slot j % kDepth and the MFMA result register j % 2 are fixed
@@ -269,9 +285,24 @@ __device__ __forceinline__ floatx16 q8_block_loop(const int8_t* atile, const flo
   // adds, then the slot refilled with block kb + kDepth.
   auto step = [&](int j, int kb) {
     const int cur = j & 1, nxt = cur ^ 1, slot = j % kDepth;
-    const floatx16 t = scale_products(d[cur], f[slot].dw, f[slot].dx, std::make_integer_sequence<int, 16>{});
+    floatx16 t;
+    if constexpr (LDS) {
+      float dx[16];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 d4 = *reinterpret_cast<const float4*>(get + 32 * cur + 8 * i);
+        dx[4 * i] = d4.x, dx[4 * i + 1] = d4.y, dx[4 * i + 2] = d4.z, dx[4 * i + 3] = d4.w;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      t = scale_products(d[cur], f[slot].dw, [&](auto v) { return dx[v()]; }, std::make_integer_sequence<int, 16>{});
+    } else {
+      const float dx = f[slot].dx;
+      t = scale_products(d[cur], f[slot].dw, [&](auto v) { return row_bcast<v()>(dx); },
+                         std::make_integer_sequence<int, 16>{});
+    }
     __builtin_amdgcn_sched_barrier(0);
     d[nxt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[(j + 1) % kDepth].a, f[(j + 1) % kDepth].b, magic, 0, 0, 0);
+    if constexpr (LDS) put[32 * nxt] = f[(j + 1) % kDepth].dx;
     __builtin_amdgcn_sched_barrier(0);
     accumulate_products(acc, t, std::make_integer_sequence<int, 16>{});
     __builtin_amdgcn_sched_barrier(0);
@@ -326,14 +357,16 @@ gemm_q8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xd, int 
   // tile), weight columns 64 tc + 32 wc; scales clamped to the last row
   // and column.
   const int wr = w >> 1, wc = w & 1, g = lane >> 5;
-  // Row whose scale this lane supplies to the DPP broadcast: lane 16r + v
-  // carries the scale of output register v for the lanes of 16-lane row r.
-  const int srow = 8 * ((lane & 15) >> 2) + 4 * g + (lane & 3);
-  const floatx16 acc = q8_block_loop<TAIL>(
+  // Row whose scale this lane loads: row lane % 32 for the LDS ring; for the
+  // DPP broadcast lane 16r + v carries the scale of output register v for
+  // the lanes of 16-lane row r.
+  __shared__ __align__(16) float dx_ring[GEGLU ? 4 : 1][2 * 32];
+  const int srow = GEGLU ? lane & 31 : 8 * ((lane & 15) >> 2) + 4 * g + (lane & 3);
+  const floatx16 acc = q8_block_loop<TAIL, GEGLU>(
       xq + (size_t)min(2 * tr + wr, (n + 31) / 32 - 1) * nb * kTile, xd, ldx, n,
       4u * (uint32_t)min(64 * tr + 32 * wr + srow, n - 1),
       wq + (size_t)min(2 * tc + wc, (m + 31) / 32 - 1) * nb * kTile, wd, ldw, m,
-      4u * (uint32_t)min(64 * tc + 32 * wc + (lane & 31), m - 1), nb, lane);
+      4u * (uint32_t)min(64 * tc + 32 * wc + (lane & 31), m - 1), nb, lane, dx_ring[GEGLU ? w : 0]);
   if constexpr (GEGLU) {
     geglu_epilogue(acc, tr, tc, wr, wc, n, m / 64, gq, gd, ldy);
   } else {
@@ -455,10 +488,10 @@ gemm_q8_qkv_rope_kernel(const int8_t* __restrict__ xq, const float* __restrict__
   // barrier).
   const int g = lane >> 5;
   const int srow = 8 * ((lane & 15) >> 2) + 4 * g + (lane & 3);
-  const floatx16 acc = q8_block_loop<TAIL>(
+  const floatx16 acc = q8_block_loop<TAIL, false>(
       xq + (size_t)tr * nb * kTile, xd, ldx, n, 4u * (uint32_t)min(32 * tr + srow, n - 1),
       wq + (size_t)(8 * hc + w) * nb * kTile, wd, ldw, kQKVCols,
-      4u * (uint32_t)(kHeadDim * hc + 32 * w + (lane & 31)), nb, lane);
+      4u * (uint32_t)(kHeadDim * hc + 32 * w + (lane & 31)), nb, lane, nullptr);
   // The epilogue runs on the tile in two halves of 16 token rows through a
   // 16-row LDS tile (17 KB per workgroup, not 34 KB). Its global inputs go
   // out now, so their latency overlaps the tile's trip through LDS and the
