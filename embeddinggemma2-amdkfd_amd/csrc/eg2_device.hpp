@@ -10,6 +10,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "eg2_libm.hpp"
 
 namespace eg2 {
@@ -152,11 +154,21 @@ __device__ __forceinline__ float rows4_sum(float v) {
   return rows4_reduce(v, [](float x, float y) { return x + y; });
 }
 
-// Max over the 32 lanes of each half-wave (lanes 0-31 and 32-63 separately).
+// Max over the 32 lanes of each half-wave (lanes 0-31 and 32-63 separately),
+// all 64 lanes active: DPP within the 16-lane rows, then the other row by
+// v_permlane16_swap (five LDS shuffles, some 120 cycles each, sat on the
+// chain of the kernels that quantize a value per lane).
 __device__ __forceinline__ float half_wave_max(float v) {
-#pragma unroll
-  for (int m = 16; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
+  auto move = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float,
+                              __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v = fmaxf(v, move(v, std::integral_constant<int, 0xB1>{}));   // quad_perm [1,0,3,2]
+  v = fmaxf(v, move(v, std::integral_constant<int, 0x4E>{}));   // quad_perm [2,3,0,1]
+  v = fmaxf(v, move(v, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+  v = fmaxf(v, move(v, std::integral_constant<int, 0x140>{}));  // row_mirror
+  const auto other = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(other[0]), __uint_as_float(other[1]));
 }
 
 // Quantizes one Q8_0 block whose 32 values sit one per lane in a half-wave
@@ -414,6 +426,15 @@ __device__ __forceinline__ float sum_squares_sse2(const float* row, int n) {
 // (kernels.c:144, :154, :165).
 __device__ __forceinline__ float rms_inverse(float ss, int n, float eps) {
   return 1.0f / __builtin_sqrtf(ss / (float)n + eps);
+}
+
+// Key range of query token t in its sequence [lo, hi) (kernels.c:330-336
+// in packed coordinates): the sequence, or |t - kt| <= window/2.
+__host__ __device__ inline void key_range(uint32_t t, uint32_t lo, uint32_t hi, int window, uint32_t& first,
+                                          uint32_t& last) {
+  const uint32_t half = window > 0 ? (uint32_t)(window / 2) : 0u;
+  first = window > 0 && t - lo > half ? t - half : lo;
+  last = window > 0 && t + half + 1 < hi ? t + half + 1 : hi;
 }
 
 }  // namespace eg2

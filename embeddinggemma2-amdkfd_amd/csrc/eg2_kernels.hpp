@@ -103,4 +103,19 @@ constexpr int kAttentionGrid = 1024;
 hipError_t launch_attention_static(const float* qkv, const uint32_t* offsets, int batch, int window, int rows,
                                    int8_t* cq, float* cd, hipStream_t st);
 
+// The fused kernels of a short wave's layer (short_wave.hpp), for waves of
+// 16 or 32 rows (short_wave): the residual update and norms with the next
+// projection, and attention from the raw Q|K|V rows. tok: the plan's token
+// records. x_out must not be x. Bit-identical to the separate kernels.
+bool short_wave(int rows);
+hipError_t launch_residual_qkv(const float* x, const float* h, const float* post_w, const float* next_w, float eps,
+                               const int8_t* wq, const float* wd, int ldw, float* x_out, float* out, int rows,
+                               hipStream_t st);
+hipError_t launch_residual_geglu(const float* x, const float* h, const float* post_w, const float* next_w, float eps,
+                                 const int8_t* wq, const float* wd, int ldw, float* x_out, int8_t* gq, float* gd,
+                                 int rows, hipStream_t st);
+hipError_t launch_short_attention(const float* qkv, const uint32_t* tok, const float* q_w, const float* k_w,
+                                  const float* rope, const int32_t* pos, float eps, int window, int rows, int8_t* cq,
+                                  float* cd, hipStream_t st);
+
 }  // namespace eg2

@@ -12,8 +12,8 @@
 // 2048-token workspace.
 //
 // Batch (src/gemma2_kfd.cpp:268-353): validate, build per-token metadata
-// (sequence bounds, positions), pad the wave to a multiple of 32 rows with a
-// dummy sequence, run the layer stack -- captured once per padded wave size
+// (sequence bounds, positions), pad the wave to a multiple of 32 rows (16 for up
+// to 16 tokens) with a dummy sequence, run the layer stack -- captured once per padded wave size
 // as a hipGraph -- then pooling, the optional dense head and L2, and copy the
 // [batch][768] embeddings back. Every call is serialised; a device failure
 // poisons the context (src/gemma2_kfd.cpp:190-191, 214-215, 270).
@@ -60,6 +60,8 @@ inline unsigned attention_form(unsigned longest) {
   return bound[softmax_form(longest)];
 }
 inline unsigned graph_key(unsigned rows, unsigned longest) { return 4 * rows + softmax_form(longest); }
+// Rows of a wave of n tokens: a multiple of 32, or 16 for up to 16 tokens.
+inline unsigned padded_rows(unsigned n) { return n <= 16 ? 16 : (n + 31) / 32 * 32; }
 constexpr int kEmbd = 768, kFF = 1152, kHeadDim = 256, kQKV = 768 + 2 * 256, kDenseFF = 3072;
 constexpr int kVocab = 262144;
 constexpr double kTimeoutSeconds = 30.0;  // src/gemma2_kfd.cpp:21
@@ -224,6 +226,7 @@ struct Lane {
   hipStream_t stream = nullptr;
   std::mutex mutex;
   float *x, *h, *xd, *cd, *pooled, *mid, *mid_d;
+  float* x2;  // the residual stream's second buffer in a short wave (32 rows)
   int8_t *xq, *cq, *mid_q;
   float* qkv;     // [rows][q0 q1 q2 | k | v] after QK-norm / RoPE
   float* scores;  // attention scratch: 1/sum per (token, head), then a score row per (token, head)
@@ -350,6 +353,7 @@ class Backend {
   // event after it on the lane's stream under `name`.
   void launch(Lane& L, const char* name, hipError_t e);
   void record_layers(Lane& L, unsigned rows, unsigned longest);
+  void record_short_layers(Lane& L, unsigned rows);
   void record_head(Lane& L, int batch);
   void gemm(Lane& L, const char* name, const int8_t* xq, const float* xd, const DevMat& w, float* y, int n, int ldy,
             hipStream_t s);
@@ -531,6 +535,7 @@ void Backend::alloc_lane(Lane& L) {
   check(hipExtStreamCreateWithCUMask(&L.stream, (uint32_t)mask.size(), mask.data()), "hipExtStreamCreateWithCUMask");
   L.x = dalloc<float>((size_t)kCap * kEmbd);
   L.h = dalloc<float>((size_t)kCap * kEmbd);
+  L.x2 = dalloc<float>(32 * (size_t)kEmbd);
   L.xq = dalloc<int8_t>(eg2_q8_tile_bytes(kCap, kFF));
   L.xd = dalloc<float>((size_t)kCap * (kFF / 32));
   L.cq = dalloc<int8_t>(eg2_q8_tile_bytes(kCap, kEmbd));
@@ -594,6 +599,10 @@ void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
   const int n = (int)rows;
   launch(ln, "embed", eg2::launch_embed_norm_quant(token_embd_, ln.ids_d, n, std::sqrt((float)kEmbd),
                                                    layers_[0].attn_norm, eps_, ln.x, ln.xq, ln.xd, s));
+  if (eg2::short_wave(n)) {
+    record_short_layers(ln, rows);
+    return;
+  }
   for (size_t il = 0; il < layers_.size(); ++il) {
     const Layer& L = layers_[il];
     // Q|K|V projection with QK-norm / RoPE in its epilogue: the attention
@@ -619,14 +628,50 @@ void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
   launch(ln, "output_norm", eg2::launch_rms_norm_rows(ln.x, output_norm_, eps_, n, s));
 }
 
+// The layers of a short wave (eg2::short_wave: 16 or 32 rows) after the
+// embedding, five kernels per layer: each residual update runs at the head
+// of the projection that consumes it, from one buffer of the residual stream
+// to the other, and attention is one kernel from the raw Q|K|V rows.
+void Backend::record_short_layers(Lane& ln, unsigned rows) {
+  hipStream_t s = ln.stream;
+  const int n = (int)rows;
+  float *x = ln.x, *other = ln.x2;
+  for (size_t il = 0; il < layers_.size(); ++il) {
+    const Layer& L = layers_[il];
+    if (il == 0) {
+      gemm(ln, "gemm_qkv", ln.xq, ln.xd, L.qkv, ln.qkv, n, kQKV, s);
+    } else {
+      launch(ln, "residual_gemm_qkv",
+             eg2::launch_residual_qkv(x, ln.h, layers_[il - 1].post_ffw, L.attn_norm, eps_, L.qkv.q, L.qkv.d, L.qkv.ld,
+                                      other, ln.qkv, n, s));
+      std::swap(x, other);
+    }
+    launch(ln, "attention", eg2::launch_short_attention(ln.qkv, ln.tok_d, L.q_norm, L.k_norm, L.rope, ln.pos_d, eps_,
+                                                        L.window, n, ln.cq, ln.cd, s));
+    gemm(ln, "gemm_o", ln.cq, ln.cd, L.o, ln.h, n, kEmbd, s);
+    launch(ln, "residual_gemm_gate_up_geglu",
+           eg2::launch_residual_geglu(x, ln.h, L.post_attn, L.ffn_norm, eps_, L.gu.q, L.gu.d, L.gu.ld, other, ln.xq,
+                                      ln.xd, n, s));
+    std::swap(x, other);
+    gemm(ln, "gemm_down", ln.xq, ln.xd, L.down, ln.h, n, kEmbd, s);
+  }
+  // An odd number of updates so far (two per layer but one): x is x2, and
+  // the last update and the output norm stay in place there.
+  launch(ln, "residual", eg2::launch_residual_norm_quant(x, ln.h, layers_.back().post_ffw, nullptr, eps_, nullptr,
+                                                         nullptr, n, s));
+  launch(ln, "output_norm", eg2::launch_rms_norm_rows(x, output_norm_, eps_, n, s));
+}
+
 // kernels.c:417-427 (mean + L2 per sequence) and the dense head.
 void Backend::record_head(Lane& ln, int B) {
   hipStream_t s = ln.stream;
+  // A short wave leaves its rows in the second buffer (record_short_layers).
+  const float* x = eg2::short_wave((int)ln.staged_rows) ? ln.x2 : ln.x;
   if (dense_) {
     // EXTRACTION.md:178-181: dense_2 then dense_3 on the mean pool
     // (kernels.c:417-425 without its L2), each input Q8_0-quantized,
     // then the L2 of kernels.c:393-396.
-    launch(ln, "pool", eg2::launch_pool_mean(ln.x, ln.off_d, ln.pooled, B, s));
+    launch(ln, "pool", eg2::launch_pool_mean(x, ln.off_d, ln.pooled, B, s));
     launch(ln, "dense_quant", eg2::launch_quantize_rows(ln.pooled, kEmbd, ln.cq, ln.cd, B, s));
     gemm(ln, "dense_2", ln.cq, ln.cd, dense2_, ln.mid, B, kDenseFF, s);
     launch(ln, "dense_quant", eg2::launch_quantize_rows(ln.mid, kDenseFF, ln.mid_q, ln.mid_d, B, s));
@@ -636,10 +681,10 @@ void Backend::record_head(Lane& ln, int B) {
     // One workgroup per sequence reads it through one CU; past 256
     // tokens the mean spreads over 12 workgroups per sequence and the
     // L2 follows (the same result, bit for bit).
-    launch(ln, "pool", eg2::launch_pool_mean(ln.x, ln.off_d, ln.pooled, B, s));
+    launch(ln, "pool", eg2::launch_pool_mean(x, ln.off_d, ln.pooled, B, s));
     launch(ln, "pool_l2", eg2::launch_l2_prefix(ln.pooled, kEmbd, kEmbd, B, s));
   } else {
-    launch(ln, "pool", eg2::launch_pool_l2(ln.x, ln.off_d, ln.pooled, B, s));
+    launch(ln, "pool", eg2::launch_pool_l2(x, ln.off_d, ln.pooled, B, s));
   }
 }
 
@@ -705,7 +750,7 @@ void Backend::stage(Lane& ln, const int32_t* ids, const size_t* offsets, size_t 
   device_step([&] { wait(ln, "HIP previous wave"); });
 
   // Metadata; rows [n, rows) form one dummy sequence that is never pooled.
-  const unsigned rows = (n + 31) / 32 * 32;
+  const unsigned rows = padded_rows(n);
   for (size_t s = 0; s < batch; ++s)
     for (size_t t = offsets[s]; t < offsets[s + 1]; ++t) {
       ln.ids_h[t] = ids[t];

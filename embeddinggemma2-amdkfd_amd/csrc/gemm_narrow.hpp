@@ -34,33 +34,50 @@ struct NarrowFrag {
   float dx, dw;
 };
 
-// The addresses of one wave's 16 x 16 tile: activation rows 16 tr .., weight
-// rows 16 tc .. (rows past n or m repeat the last one's scale; the row tiles
-// are padded to 32).
-struct NarrowTile {
-  __amdgpu_buffer_rsrc_t ra, rb, rx, rw;
-  uint32_t lane_off, xoff, woff, ldx4, ldw4;
+// Byte offset of the lane's 8 values inside the 16-row half of a 1 KB block.
+__device__ __forceinline__ uint32_t narrow_lane_offset() {
+  const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+  return (uint32_t)((g >> 1) * 512 + r * 16 + (g & 1) * 8);
+}
+
+// One wave's 16 weight rows 16 tc .. (rows past m repeat the last one's
+// scale; the row tiles are padded to 32).
+struct NarrowWeights {
+  __amdgpu_buffer_rsrc_t rb, rw;
+  uint32_t lane_off, woff, ldw4;
   int nb;
 
-  __device__ __forceinline__ NarrowTile(const int8_t* xq, const float* xd, int ldx, int n, int tr, const int8_t* wq,
-                                        const float* wd, int ldw, int m, int tc, int blocks)
-      : nb(blocks) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-    ra = buffer_rsrc(xq + (size_t)(tr >> 1) * nb * kTileBytes + (tr & 1) * 256, (uint32_t)nb * kTileBytes - (tr & 1) * 256);
-    rb = buffer_rsrc(wq + (size_t)(tc >> 1) * nb * kTileBytes + (tc & 1) * 256, (uint32_t)nb * kTileBytes - (tc & 1) * 256);
-    rx = buffer_rsrc(xd, 4u * ((uint32_t)(nb - 1) * (uint32_t)ldx + (uint32_t)n));
+  __device__ __forceinline__ NarrowWeights(const int8_t* wq, const float* wd, int ldw, int m, int tc, int blocks)
+      : lane_off(narrow_lane_offset()), ldw4(4u * (uint32_t)ldw), nb(blocks) {
+    const uint32_t skip = (tc & 1) * 256;
+    rb = buffer_rsrc(wq + (size_t)(tc >> 1) * nb * kTileBytes + skip, (uint32_t)nb * kTileBytes - skip);
     rw = buffer_rsrc(wd, 4u * ((uint32_t)(nb - 1) * (uint32_t)ldw + (uint32_t)m));
-    lane_off = (uint32_t)((g >> 1) * 512 + r * 16 + (g & 1) * 8);
-    xoff = 4u * (uint32_t)min(16 * tr + 4 * g + (lane & 3), n - 1);
-    woff = 4u * (uint32_t)min(16 * tc + r, m - 1);
-    ldx4 = 4u * (uint32_t)ldx;
-    ldw4 = 4u * (uint32_t)ldw;
+    woff = 4u * (uint32_t)min(16 * tc + (int)(threadIdx.x & 15), m - 1);
   }
   __device__ __forceinline__ void load(NarrowFrag& f, int kb) const {  // kb uniform; past the end: the last block
     kb = min(kb, nb - 1);
     f.b = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(rb, lane_off, kb * kTileBytes, 0));
-    f.a = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(ra, lane_off, kb * kTileBytes, 0));
     f.dw = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, woff, (uint32_t)kb * ldw4, 0));
+  }
+};
+
+// One wave's 16 activation rows 16 tr .., as NarrowWeights (n rows).
+struct NarrowRows {
+  __amdgpu_buffer_rsrc_t ra, rx;
+  uint32_t lane_off, xoff, ldx4;
+  int nb;
+
+  __device__ __forceinline__ NarrowRows(const int8_t* xq, const float* xd, int ldx, int n, int tr, int blocks)
+      : lane_off(narrow_lane_offset()), ldx4(4u * (uint32_t)ldx), nb(blocks) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t skip = (tr & 1) * 256;
+    ra = buffer_rsrc(xq + (size_t)(tr >> 1) * nb * kTileBytes + skip, (uint32_t)nb * kTileBytes - skip);
+    rx = buffer_rsrc(xd, 4u * ((uint32_t)(nb - 1) * (uint32_t)ldx + (uint32_t)n));
+    xoff = 4u * (uint32_t)min(16 * tr + 4 * (lane >> 4) + (lane & 3), n - 1);
+  }
+  __device__ __forceinline__ void load(NarrowFrag& f, int kb) const {
+    kb = min(kb, nb - 1);
+    f.a = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(ra, lane_off, kb * kTileBytes, 0));
     f.dx = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, xoff, (uint32_t)kb * ldx4, 0));
   }
 };
@@ -123,13 +140,17 @@ gemm_q8_narrow_kernel(const int8_t* __restrict__ xq, const float* __restrict__ x
   __builtin_amdgcn_s_setprio(1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tc = (int)blockIdx.x, tr = (int)blockIdx.y;
-  const NarrowTile tile(xq, xd, ldx, n, tr, wq, wd, ldw, m, tc, nb);
+  const NarrowWeights weights(wq, wd, ldw, m, tc, nb);
+  const NarrowRows rows(xq, xd, ldx, n, tr, nb);
   const int o = (int)threadIdx.x;
   float sum = 0.0f;
   for (int c0 = 0; c0 < nb; c0 += kChunk) {
     NarrowFrag f[NBW];
 #pragma unroll
-    for (int i = 0; i < NBW; ++i) tile.load(f[i], c0 + w * NBW + i);
+    for (int i = 0; i < NBW; ++i) {
+      weights.load(f[i], c0 + w * NBW + i);
+      rows.load(f[i], c0 + w * NBW + i);
+    }
     if (c0) __syncthreads();  // the previous chunk's terms are no longer read
     narrow_put<NBW>(f, w, terms);
     __syncthreads();
@@ -137,6 +158,18 @@ gemm_q8_narrow_kernel(const int8_t* __restrict__ xq, const float* __restrict__ x
   }
   const int row = 16 * tr + 4 * (o >> 6) + (o & 3), col = 16 * tc + ((o >> 2) & 15);
   if (row < n && col < m) y[(size_t)row * ldy + col] = sum;
+}
+
+// The GeGLU of one R x 32 tile, gu = [row][gate 0..31 | up 0..31], by the
+// first 32 R threads, and its Q8_0: block tc of rows t0 .. t0 + R - 1.
+constexpr int kGuPitch = 65;
+__device__ __forceinline__ void narrow_geglu_store(const float* gu, int t0, int tc, int n, int nbf,
+                                                   int8_t* __restrict__ gq, float* __restrict__ gd, int ldg) {
+  const int row = (int)threadIdx.x >> 5, col = (int)threadIdx.x & 31, t = t0 + row;
+  const Q8Lane q = q8_quantize_lane(gelu_mul(gu[row * kGuPitch + col], gu[row * kGuPitch + 32 + col]));
+  if (t >= n) return;
+  gq[q8_tile_offset(t, 32 * tc + col, nbf)] = (int8_t)q.q;
+  if (col == 0) gd[(size_t)tc * ldg + t] = q.d;
 }
 
 // gate|up + GeGLU + Q8_0: a workgroup of 8 waves computes 16 rows x one
@@ -154,13 +187,14 @@ __global__ void __launch_bounds__(512)
 gemm_q8_geglu_narrow_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xd, int ldx,
                             const int8_t* __restrict__ wq, const float* __restrict__ wd, int ldw, int n, int ff,
                             int nb, int8_t* __restrict__ gq, float* __restrict__ gd, int ldg) {
-  constexpr int NBW = kNarrowGegluBlocks, kHalf = NBW, kPitch = 65;
+  constexpr int NBW = kNarrowGegluBlocks, kHalf = NBW;
   __shared__ __align__(16) float4 terms[4][kHalf * 64];  // [tile][block of the half chunk][lane]
-  __shared__ float gu[16 * kPitch];                      // [row][gate 0..31 | up 0..31]
+  __shared__ float gu[16 * kGuPitch];                    // [row][gate 0..31 | up 0..31]
   __builtin_amdgcn_s_setprio(1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ti = w & 3, ks = w >> 2;
   const int tc = (int)blockIdx.x, tr = (int)blockIdx.y;
-  const NarrowTile tile(xq, xd, ldx, n, tr, wq, wd, ldw, 2 * ff, 4 * tc + ti, nb);
+  const NarrowWeights weights(wq, wd, ldw, 2 * ff, 4 * tc + ti, nb);
+  const NarrowRows rows(xq, xd, ldx, n, tr, nb);
   const int so = (int)threadIdx.x >> 8, o = (int)threadIdx.x & 255;  // this thread adds output o of tiles so, so + 2
   float gate = 0.0f, up = 0.0f;
   for (int c0 = 0; c0 < nb; c0 += 2 * kHalf) {
@@ -168,7 +202,10 @@ gemm_q8_geglu_narrow_kernel(const int8_t* __restrict__ xq, const float* __restri
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
-      for (int i = 0; i < NBW / 2; ++i) tile.load(f[p][i], c0 + p * kHalf + ks * (NBW / 2) + i);
+      for (int i = 0; i < NBW / 2; ++i) {
+        weights.load(f[p][i], c0 + p * kHalf + ks * (NBW / 2) + i);
+        rows.load(f[p][i], c0 + p * kHalf + ks * (NBW / 2) + i);
+      }
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       if (c0 + p) __syncthreads();  // the previous half's terms are no longer read
@@ -179,15 +216,11 @@ gemm_q8_geglu_narrow_kernel(const int8_t* __restrict__ xq, const float* __restri
       up = narrow_sum<kHalf>(reinterpret_cast<const float*>(terms[so + 2]), o, cnt, up);
     }
   }
-  float* mine = gu + (4 * (o >> 6) + (o & 3)) * kPitch + 16 * so + ((o >> 2) & 15);
+  float* mine = gu + (4 * (o >> 6) + (o & 3)) * kGuPitch + 16 * so + ((o >> 2) & 15);
   mine[0] = gate;
   mine[32] = up;
   __syncthreads();
-  const int row = (int)threadIdx.x >> 5, col = (int)threadIdx.x & 31, t = 16 * tr + row;
-  const Q8Lane q = q8_quantize_lane(gelu_mul(gu[row * kPitch + col], gu[row * kPitch + 32 + col]));
-  if (t >= n) return;
-  gq[q8_tile_offset(t, 32 * tc + col, ff / kQK)] = (int8_t)q.q;
-  if (col == 0) gd[(size_t)tc * ldg + t] = q.d;
+  narrow_geglu_store(gu, 16 * tr, tc, n, ff / kQK, gq, gd, ldg);
 }
 
 }  // namespace eg2

@@ -112,15 +112,6 @@ constexpr size_t item_bound(size_t tokens, size_t batch) {
 __host__ __device__ inline uint32_t score_pitch(uint32_t len) { return (len + 3u) & ~3u; }
 __host__ __device__ inline size_t inv_floats(size_t rows) { return (3 * rows + 3) & ~(size_t)3; }
 
-// Key range of query token t in its sequence [lo, hi) (kernels.c:330-336
-// in packed coordinates): the sequence, or |t - kt| <= window/2.
-__host__ __device__ inline void key_range(uint32_t t, uint32_t lo, uint32_t hi, int window, uint32_t& first,
-                                          uint32_t& last) {
-  const uint32_t half = window > 0 ? (uint32_t)(window / 2) : 0u;
-  first = window > 0 && t - lo > half ? t - half : lo;
-  last = window > 0 && t + half + 1 < hi ? t + half + 1 : hi;
-}
-
 // ----------------------------------------------------------------- scores
 
 // The scores' staging: per item, eight stages of 32 dimensions, each a

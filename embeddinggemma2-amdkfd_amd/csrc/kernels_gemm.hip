@@ -44,6 +44,7 @@
 #include "eg2_device.hpp"
 #include "eg2_kernels.hpp"
 #include "gemm_narrow.hpp"
+#include "short_wave.hpp"
 
 namespace eg2 {
 
@@ -594,6 +595,36 @@ hipError_t launch_gemm_q8_qkv_rope(const int8_t* xq, const float* xd, int ldx, c
   else
     hipLaunchKernelGGL(gemm_q8_qkv_rope_kernel<true>, grid, dim3(512), lds, st, xq, xd, ldx, wq, wd, ldw, n, nb, q_w,
                        k_w, rope, pos, eps, out);
+  return hipGetLastError();
+}
+
+// The short wave's fused kernels (short_wave.hpp).
+bool short_wave(int rows) { return rows <= kShortRows && rows % 16 == 0; }
+
+hipError_t launch_residual_qkv(const float* x, const float* h, const float* post_w, const float* next_w, float eps,
+                               const int8_t* wq, const float* wd, int ldw, float* x_out, float* out, int rows,
+                               hipStream_t st) {
+  if (rows <= 0 || !short_wave(rows) || x == x_out || ldw < kQKVCols) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(residual_qkv_kernel, dim3(kQKVCols / 32, rows / kShortTile), dim3(kShortThreads), 0, st, x, h, post_w, next_w, eps,
+                     wq, wd, ldw, x_out, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_residual_geglu(const float* x, const float* h, const float* post_w, const float* next_w, float eps,
+                                 const int8_t* wq, const float* wd, int ldw, float* x_out, int8_t* gq, float* gd,
+                                 int rows, hipStream_t st) {
+  if (rows <= 0 || !short_wave(rows) || x == x_out || ldw < 2 * kFF) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(residual_geglu_kernel, dim3(kFF / kQK, rows / kShortTile), dim3(kShortThreads), 0, st, x, h, post_w,
+                     next_w, eps, wq, wd, ldw, x_out, gq, gd, rows);
+  return hipGetLastError();
+}
+
+hipError_t launch_short_attention(const float* qkv, const uint32_t* tok, const float* q_w, const float* k_w,
+                                  const float* rope, const int32_t* pos, float eps, int window, int rows, int8_t* cq,
+                                  float* cd, hipStream_t st) {
+  if (rows <= 0 || !short_wave(rows) || window < 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(short_attention_kernel, dim3(kHeads, rows / kShortQueries), dim3(1024), 0, st, qkv,
+                     reinterpret_cast<const uint4*>(tok), q_w, k_w, rope, pos, eps, window, rows, cq, cd);
   return hipGetLastError();
 }
 

@@ -1,0 +1,352 @@
+// The layer of a short wave (at most kShortRows rows, a multiple of 16) in
+// five kernels instead of nine:
+//   residual_qkv      residual + norms + Q8_0, then the Q|K|V projection
+//   short_attention   QK-norm / RoPE, scores, softmax, context, Q8_0
+//   (O projection     gemm_q8_narrow_kernel)
+//   residual_geglu    residual + norms + Q8_0, then gate|up + GeGLU + Q8_0
+//   (down projection  gemm_q8_narrow_kernel)
+// A short wave is a chain of latencies: each kernel boundary costs about 1.5
+// us and empties the L2, and a 16-row residual kernel or a 3-head attention
+// occupies a handful of CUs. So every workgroup of a projection repeats its
+// rows' residual update and norms itself (the chip is idle anyway) while its
+// weights are on their way, and one workgroup per (head, few query rows)
+// takes attention from the raw projection to the quantized context with all
+// keys and values in LDS. The same operations in the same order as the
+// kernels they replace: the same bits. One query of 11
+// tokens through 24 layers: 1,119 -> 737 us.
+#pragma once
+
+#include "eg2_device.hpp"
+#include "gemm_narrow.hpp"
+#include "row_device.hpp"
+
+namespace eg2 {
+
+// Orders a wave's LDS writes before its reads of them by other lanes (the
+// wave's LDS accesses execute in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// A residual + projection workgroup: 12 waves, kShortTile rows. Thread (wave
+// w, lane) holds columns 256 (w % 3) + 4 lane .. + 3 of rows w / 3 and
+// w / 3 + 4, so a norm weight vector is read once per workgroup, not once per
+// row. What a CU has to read bounds the start of these kernels (64 B per
+// cycle: with 16 rows and a row per wave, 96 KB of rows and 96 KB of norm
+// weights took 5,700 cycles of 18,700), hence also 8 rows rather than 16 per
+// workgroup; the MFMA tile's other 8 rows repeat them and are not stored.
+constexpr int kShortTile = 8;
+constexpr int kShortWaves = 12, kShortThreads = 64 * kShortWaves;
+constexpr int kShortStride = 8 * kTPitch + 4;  // staged squares per row: 8 rows read at once on distinct banks
+
+// The LDS of such a workgroup: the rows' staged squares, then the terms of
+// TILES 16-column tiles, their 24 blocks split over 12 / TILES waves; the
+// quantized rows [block][2][8 rows][16] and their scales [block][8 rows].
+template <int TILES>
+struct ShortLds {
+  static constexpr int kSplit = kShortWaves / TILES, kPer = kBlocks / kSplit;
+  static_assert(kSplit * kPer == kBlocks, "24 blocks split evenly");
+  union alignas(16) {
+    float squares[kShortTile * kShortStride];
+    float4 terms[TILES][kBlocks * 32];  // lanes 0 .. 31: rows 0 .. 7
+  };
+  alignas(16) int8_t aq[kBlocks * 32 * kShortTile];
+  float dxs[kBlocks * kShortTile];
+  float inv[2][kShortTile];
+};
+
+// residual_norm_quant_kernel's work on the workgroup's rows, then the
+// projection onto weight columns 16 (TILES blockIdx.x + tile): x_out = x +
+// rms(h) * post_w (stored by the workgroups with blockIdx.x = 0), Q8_0 of
+// rms(x_out) * next_w, times W^T. Returns, for thread i < 128 TILES, output
+// i % 128 of tile i / 128 (row 4 (o / 64) + o % 4, column (o / 4) % 16).
+template <int TILES>
+__device__ __forceinline__ float residual_project(ShortLds<TILES>& lds, const float* __restrict__ x,
+                                                  const float* __restrict__ h, const float* __restrict__ post_w,
+                                                  const float* __restrict__ next_w, float eps,
+                                                  const int8_t* __restrict__ wq, const float* __restrict__ wd, int ldw,
+                                                  int m, float* __restrict__ x_out) {
+  constexpr int kPer = ShortLds<TILES>::kPer;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = w / 3, part = w % 3, e = 4 * (lane + 64 * part);
+  float4 hv[2], xv[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    hv[i] = *reinterpret_cast<const float4*>(h + (size_t)(kShortTile * blockIdx.y + row + 4 * i) * kEmbd + e);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    xv[i] = *reinterpret_cast<const float4*>(x + (size_t)(kShortTile * blockIdx.y + row + 4 * i) * kEmbd + e);
+  const float4 pw = *reinterpret_cast<const float4*>(post_w + e), nw = *reinterpret_cast<const float4*>(next_w + e);
+  // The weights of this wave's blocks, on their way during the rows' work.
+  const int ti = w % TILES, ks = w / TILES;
+  const NarrowWeights weights(wq, wd, ldw, m, TILES * (int)blockIdx.x + ti, kBlocks);
+  NarrowFrag f[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) weights.load(f[i], ks * kPer + i);
+
+  // Squares of the thread's values into the transposed rows; wave 0 runs the
+  // 64 chains of the 8 rows and leaves each row's inverse in inv.
+  auto inverses = [&](const float4 (&v)[2], float* inv) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      TRow* tr = reinterpret_cast<TRow*>(lds.squares + (row + 4 * i) * kShortStride);
+      const float c4[4] = {v[i].x * v[i].x, v[i].y * v[i].y, v[i].z * v[i].z, v[i].w * v[i].w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) tr[(e + k) & 7][(e + k) >> 3] = c4[k];
+    }
+    __syncthreads();
+    if (w == 0) {
+      const TRow* rows = reinterpret_cast<const TRow*>(lds.squares + (lane >> 3) * kShortStride);
+      const float r = rms_inverse(sse2_combine_dpp(squares_chain(rows, lane & 7)), kEmbd, eps);
+      if ((lane & 7) == 0) inv[lane >> 3] = r;
+    }
+    __syncthreads();
+  };
+  inverses(hv, lds.inv[0]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // kernels.c:163-188
+    const float inv_h = lds.inv[0][row + 4 * i];
+    const float a0 = hv[i].x * inv_h, a1 = hv[i].y * inv_h, a2 = hv[i].z * inv_h, a3 = hv[i].w * inv_h;
+    const float b0 = a0 * pw.x, b1 = a1 * pw.y, b2 = a2 * pw.z, b3 = a3 * pw.w;
+    xv[i] = make_float4(xv[i].x + b0, xv[i].y + b1, xv[i].z + b2, xv[i].w + b3);
+    if (blockIdx.x == 0)
+      *reinterpret_cast<float4*>(x_out + (size_t)(kShortTile * blockIdx.y + row + 4 * i) * kEmbd + e) = xv[i];
+  }
+  inverses(xv, lds.inv[1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // kernels.c:139-151, the block over 8 lanes
+    const float inv = lds.inv[1][row + 4 * i];
+    const float p0 = xv[i].x * nw.x, p1 = xv[i].y * nw.y, p2 = xv[i].z * nw.z, p3 = xv[i].w * nw.w;
+    const float v0 = p0 * inv, v1 = p1 * inv, v2 = p2 * inv, v3 = p3 * inv;
+    const float amax = group8_max(fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3))));
+    const float d = div127(amax);
+    const float id = amax != 0.0f ? 1.0f / d : 0.0f;
+    const int kb = e / kQK, r = row + 4 * i;
+    *reinterpret_cast<uint32_t*>(lds.aq + ((kb * 2 + ((e >> 4) & 1)) * kShortTile + r) * 16 + (e & 15)) =
+        pack_i8x4(q8_value(v0, id), q8_value(v1, id), q8_value(v2, id), q8_value(v3, id));
+    if ((lane & 7) == 0) lds.dxs[kb * kShortTile + r] = fp16_bits_to_fp32(fp32_to_fp16_bits(d));
+  }
+  __syncthreads();
+  // Lane 16 g + r: row r % 8, values 8 g .. 8 g + 7 of the block.
+  const int g = lane >> 4, aoff = ((g >> 1) * kShortTile + (lane & 7)) * 16 + (g & 1) * 8;
+  const int xoff = 4 * (g & 1) + (lane & 3);
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int kb = ks * kPer + i;
+    f[i].a = *reinterpret_cast<const uint64_t*>(lds.aq + kb * 32 * kShortTile + aoff);
+    f[i].dx = lds.dxs[kb * kShortTile + xoff];
+    const float4 t = narrow_terms(f[i]);
+    if (lane < 32) lds.terms[ti][kb * 32 + lane] = t;
+  }
+  __syncthreads();
+  const int i = (int)threadIdx.x;
+  float sum = 0.0f;
+  if (i < 128 * TILES) {
+    const float* t = reinterpret_cast<const float*>(lds.terms[i >> 7]) + (i & 127);
+    float v[kBlocks];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) v[b] = t[128 * b];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) sum = sum + v[b];
+  }
+  return sum;
+}
+
+// The raw Q|K|V rows (no QK-norm / RoPE) of x_out. Grid (kQKVCols / 32, rows /
+// kShortTile). x_out must not be x: every workgroup reads x.
+__global__ void __launch_bounds__(kShortThreads)
+residual_qkv_kernel(const float* __restrict__ x, const float* __restrict__ h, const float* __restrict__ post_w,
+                    const float* __restrict__ next_w, float eps, const int8_t* __restrict__ wq,
+                    const float* __restrict__ wd, int ldw, float* __restrict__ x_out, float* __restrict__ out) {
+  __shared__ ShortLds<2> lds;
+  const float sum = residual_project<2>(lds, x, h, post_w, next_w, eps, wq, wd, ldw, kQKVCols, x_out);
+  const int i = (int)threadIdx.x, o = i & 127;
+  if (i < 256)
+    out[(size_t)(kShortTile * blockIdx.y + 4 * (o >> 6) + (o & 3)) * kQKVCols + 32 * blockIdx.x + 16 * (i >> 7) +
+        ((o >> 2) & 15)] = sum;
+}
+
+// The same rows, then gate|up (interleaved 32-row groups), GeGLU and Q8_0
+// into gq / gd [kFF / 32][rows]. Grid (kFF / 32, rows / kShortTile).
+__global__ void __launch_bounds__(kShortThreads)
+residual_geglu_kernel(const float* __restrict__ x, const float* __restrict__ h, const float* __restrict__ post_w,
+                      const float* __restrict__ next_w, float eps, const int8_t* __restrict__ wq,
+                      const float* __restrict__ wd, int ldw, float* __restrict__ x_out, int8_t* __restrict__ gq,
+                      float* __restrict__ gd, int rows) {
+  __shared__ ShortLds<4> lds;
+  __shared__ float gu[kShortTile * kGuPitch];
+  const float sum = residual_project<4>(lds, x, h, post_w, next_w, eps, wq, wd, ldw, 2 * kFF, x_out);
+  const int i = (int)threadIdx.x, o = i & 127;
+  if (i < 512) gu[(4 * (o >> 6) + (o & 3)) * kGuPitch + 16 * (i >> 7) + ((o >> 2) & 15)] = sum;
+  __syncthreads();
+  if (i < 32 * kShortTile)
+    narrow_geglu_store(gu, kShortTile * (int)blockIdx.y, (int)blockIdx.x, rows, kFF / kQK, gq, gd, rows);
+}
+
+// ------------------------------------------------------------ attention
+
+// A workgroup of 16 waves takes one head and kShortQueries query rows of a
+// wave of at most kShortRows packed rows from the raw projection rows
+// [q0 q1 q2 | k | v] to the quantized context: all waves normalise and rotate
+// the k rows (two each), the first kShortQueries waves also a query row each,
+// which they then carry through. (With 16 query rows per workgroup the LDS
+// reads of 16 score and context waves on one CU bound the kernel.) Normalised and
+// rotated q and k rows are kept chain-major in LDS, [row][chain d % 4][step
+// d / 4], so that a lane of chain c reads four steps with one 16-byte read
+// (pitches of 68 and 272 floats: a 16-lane read group covers 4 rows x 4 chains
+// on distinct banks). Scores: lane 4 k + c runs chain c of keys k and k + 16
+// (kernels.c:289-294), the chains combined as (s0 + s2) + (s1 + s3); then the
+// row's maximum, expf, the sum in key order and the context in key order,
+// lanes over dimensions, over the row's own keys only.
+constexpr int kShortRows = 32;
+constexpr int kShortQueries = 4;
+constexpr int kShortPitch = kHeadDim + 8;  // floats per raw row
+constexpr int kChainPitch = kHeadDim / 4 + 4, kChainRow = 4 * kChainPitch;
+
+struct ShortAttentionLds {
+  float raw[kShortQueries + kShortRows][kShortPitch];  // q rows, then k rows
+  alignas(16) float q[kShortQueries][kChainRow];
+  alignas(16) float k[kShortRows][kChainRow];
+  alignas(16) float v[kShortRows][kHeadDim];
+  alignas(16) float p[kShortQueries][kShortRows];
+  uint64_t exp_tab[32];
+};
+
+__global__ void __launch_bounds__(1024)
+short_attention_kernel(const float* __restrict__ qkv, const uint4* __restrict__ tok, const float* __restrict__ q_w,
+                       const float* __restrict__ k_w, const float* __restrict__ rope, const int32_t* __restrict__ pos,
+                       float eps, int window, int rows, int8_t* __restrict__ cq, float* __restrict__ cd) {
+  __shared__ ShortAttentionLds lds;
+  constexpr int half = kHeadDim / 2;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hd = (int)blockIdx.x, qw = w % kShortQueries, t = kShortQueries * (int)blockIdx.y + qw;
+  const bool two = rows > 16;  // uniform: keys 16 .. 31 exist
+  // Rows of this wave: query row t, key rows w and w + 16.
+  const bool query = w < kShortQueries;  // this wave carries query row t
+  // This wave's key rows, w and (two) w + 16.
+  const int tk0 = w, tk1 = two ? w + 16 : w;
+  const int pq = pos[t], p0 = pos[tk0], p1 = pos[tk1];
+  const uint4 meta = tok[t];
+  const float* kr0 = qkv + (size_t)tk0 * kQKVCols + kHeads * kHeadDim + 4 * lane;
+  const float* kr1 = qkv + (size_t)tk1 * kQKVCols + kHeads * kHeadDim + 4 * lane;
+  const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float4 q4 = query ? *reinterpret_cast<const float4*>(qkv + (size_t)t * kQKVCols + hd * kHeadDim + 4 * lane) : zero;
+  const float4 k40 = *reinterpret_cast<const float4*>(kr0);
+  const float4 k41 = two ? *reinterpret_cast<const float4*>(kr1) : zero;
+  // A row's norm weights and cos/sin for dimensions lane + 64 j.
+  struct Row4 {
+    float v[4];
+  };
+  auto row4 = [&](const float* p) { return Row4{{p[lane], p[lane + 64], p[lane + 128], p[lane + 192]}}; };
+  const Row4 kw = row4(k_w), qw4 = query ? row4(q_w) : kw;
+  const Row4 c0 = row4(rope + (size_t)p0 * kHeadDim), c1 = two ? row4(rope + (size_t)p1 * kHeadDim) : c0,
+             cq4 = query ? row4(rope + (size_t)pq * kHeadDim) : c0;
+  const float4 v40 = *reinterpret_cast<const float4*>(kr0 + kHeadDim);
+  const float4 v41 = two ? *reinterpret_cast<const float4*>(kr1 + kHeadDim) : zero;
+  if (threadIdx.x < 32) lds.exp_tab[threadIdx.x] = libm::kExp2Tab.t[threadIdx.x];
+  float* rawq = lds.raw[qw];
+  float* rawk0 = lds.raw[kShortQueries + tk0];
+  float* rawk1 = lds.raw[kShortQueries + tk1];
+  if (query) *reinterpret_cast<float4*>(rawq + 4 * lane) = q4;
+  *reinterpret_cast<float4*>(rawk0 + 4 * lane) = k40;
+  if (two) *reinterpret_cast<float4*>(rawk1 + 4 * lane) = k41;
+  wave_lds_fence();
+  // kernels.c:233-264: lanes 0-7 run the chains of key row w, 8-15 of w + 16,
+  // 16-23 of the query row.
+  const float* chain_row = (lane >> 3) == 1 && two ? rawk1 : ((lane >> 3) == 2 && query ? rawq : rawk0);
+  const float own = rms_inverse(sse2_combine_dpp(sse2_chain<kHeadDim>(chain_row, lane & 7)), kHeadDim, eps);
+  auto norm_rope = [&](const float* raw, float* dst, const Row4& g, const Row4& cs, int from, bool q) {
+    const float inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), from));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int dd = lane + 64 * j;
+      const float c = cs.v[j], s = cs.v[2 + j];
+      const float x0 = raw[dd] * g.v[j] * inv;
+      const float x1 = raw[dd + half] * g.v[2 + j] * inv;
+      const float a0 = x0 * c, a1 = x1 * s;
+      const float b0 = x0 * s, b1 = x1 * c;
+      float lo = a0 - a1, hi = b0 + b1;
+      if (q) {
+        lo = lo * 0.0625f;
+        hi = hi * 0.0625f;
+      }
+      dst[(dd & 3) * kChainPitch + (dd >> 2)] = lo;
+      dst[(dd & 3) * kChainPitch + ((dd + half) >> 2)] = hi;
+    }
+  };
+  norm_rope(rawk0, lds.k[tk0], kw, c0, 0, false);
+  if (two) norm_rope(rawk1, lds.k[tk1], kw, c1, 8, false);
+  if (query) norm_rope(rawq, lds.q[qw], qw4, cq4, 16, true);
+  *reinterpret_cast<float4*>(lds.v[tk0] + 4 * lane) = v40;
+  if (two) *reinterpret_cast<float4*>(lds.v[tk1] + 4 * lane) = v41;
+  __syncthreads();
+  if (!query) return;
+  // Scores of row t.
+  const int key = lane >> 2, c = lane & 3;
+  float s[2] = {0.0f, 0.0f};
+  const float4* qp = reinterpret_cast<const float4*>(lds.q[qw] + c * kChainPitch);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (i == 1 && !two) break;
+    const float4* kp = reinterpret_cast<const float4*>(lds.k[key + 16 * i] + c * kChainPitch);
+    float a = 0.0f;
+#pragma unroll
+    for (int st = 0; st < kHeadDim / 16; ++st) {
+      const float4 qv = qp[st], kv = kp[st];
+      const float p0 = qv.x * kv.x, p1 = qv.y * kv.y, p2 = qv.z * kv.z, p3 = qv.w * kv.w;
+      a = a + p0;
+      a = a + p1;
+      a = a + p2;
+      a = a + p3;
+    }
+    a = a + dpp<kQuad2301>(a);     // s0 + s2, s1 + s3
+    s[i] = a + dpp<kQuad1032>(a);  // their sum
+  }
+  uint32_t first, last;
+  key_range((uint32_t)t, meta.x, meta.y, window, first, last);
+  const bool in0 = (uint32_t)key >= first && (uint32_t)key < last;
+  const bool in1 = two && (uint32_t)key + 16 >= first && (uint32_t)key + 16 < last;
+  float m = fmaxf(in0 ? s[0] : -__builtin_inff(), in1 ? s[1] : -__builtin_inff());
+  m = fmaxf(m, dpp<0x141>(m));  // row_half_mirror: the other quad of each 8 lanes
+  m = rows4_max(fmaxf(m, dpp<0x140>(m)));  // row_mirror, then the four rows
+  const float e0 = libm::expf_tab(s[0] - m, lds.exp_tab), e1 = libm::expf_tab(s[1] - m, lds.exp_tab);
+  if (c == 0) {
+    lds.p[qw][key] = in0 ? e0 : 0.0f;
+    lds.p[qw][key + 16] = in1 ? e1 : 0.0f;
+  }
+  wave_lds_fence();
+  // The sum in key order; +0 outside the row's keys changes no sum.
+  float sum = 0.0f;
+  const float4* pp = reinterpret_cast<const float4*>(lds.p[qw]);
+#pragma unroll
+  for (int i = 0; i < kShortRows / 4; ++i) {
+    if (4 * i >= rows) break;  // uniform
+    const float4 p4 = pp[i];
+    sum = sum + p4.x;
+    sum = sum + p4.y;
+    sum = sum + p4.z;
+    sum = sum + p4.w;
+  }
+  const float inv = 1.0f / sum;
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const int kfirst = __builtin_amdgcn_readfirstlane((int)first), klast = __builtin_amdgcn_readfirstlane((int)last);
+#pragma unroll 4
+  for (int k = kfirst; k < klast; ++k) {
+    const float wk = lds.p[qw][k] * inv;
+    const float4 vv = *reinterpret_cast<const float4*>(lds.v[k] + 4 * lane);
+    const float p0 = wk * vv.x, p1 = wk * vv.y, p2 = wk * vv.z, p3 = wk * vv.w;
+    acc = make_float4(acc.x + p0, acc.y + p1, acc.z + p2, acc.w + p3);
+  }
+  // Q8_0 (quants.c:97-177): 8 lanes hold a block.
+  const float amax = group8_max(fmaxf(fmaxf(fabsf(acc.x), fabsf(acc.y)), fmaxf(fabsf(acc.z), fabsf(acc.w))));
+  const float d = div127(amax);
+  const float id = amax != 0.0f ? 1.0f / d : 0.0f;
+  const unsigned e = (unsigned)(hd * kHeadDim + 4 * lane);
+  if ((lane & 7) == 0) cd[(size_t)(e / kQK) * rows + t] = fp16_bits_to_fp32(fp32_to_fp16_bits(d));
+  *reinterpret_cast<uint32_t*>(cq + q8_tile_offset(t, e, kBlocks)) =
+      pack_i8x4(q8_value(acc.x, id), q8_value(acc.y, id), q8_value(acc.z, id), q8_value(acc.w, id));
+}
+
+}  // namespace eg2
