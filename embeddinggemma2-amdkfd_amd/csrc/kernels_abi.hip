@@ -12,15 +12,17 @@
 // are not the reference kernels' bits.
 //
 // Designs:
-//  - projections (eg2_mm*): fp32 MFMA (v_mfma_f32_16x16x4f32) on LDS-staged
-//    32-deep K slices of the activations and of the weights decoded to fp32
-//    (F32, F16, BF16 or Q8_0 blocks over the flattened matrix), zero-padded
-//    past k. The MFMA's k index is a permutation of the slice chosen so that
-//    each lane reads contiguous float4s of its row: lane group g (lanes
-//    16g .. 16g+15) feeds slice elements g*KW/4 .. (g+1)*KW/4 - 1, one per
-//    MFMA. The 16x16 tile splits the slice over its four waves and adds
-//    their partial tiles at the end; the wider tiles give each wave its own
-//    16x16 blocks.
+//  - projections (eg2_mm*): bf16 MFMA on exact bf16 parts of the operands
+//    (F32 weights: fp32 MFMA), each wave over every fourth 32-deep step of the
+//    tile; and a general form for any k and alignment: fp32 MFMA
+//    (v_mfma_f32_16x16x4f32) on LDS-staged 32-deep K slices of the activations
+//    and of the weights decoded to fp32 (F32, F16, BF16 or Q8_0 blocks over
+//    the flattened matrix), zero-padded past k. There the MFMA's k index is a
+//    permutation of the slice chosen so that each lane reads contiguous
+//    float4s of its row: lane group g (lanes 16g .. 16g+15) feeds slice
+//    elements g*KW/4 .. (g+1)*KW/4 - 1, one per MFMA. The 16x16 tile splits
+//    the slice over its four waves and adds their partial tiles at the end;
+//    the wider tiles give each wave its own 16x16 blocks.
 //  - attention: keys in chunks of 64, one per lane: every lane computes its
 //    key's whole dot product against q (broadcast from LDS), so a chunk
 //    costs one wave max and one wave sum instead of one reduction per key;
@@ -86,14 +88,13 @@ __device__ __forceinline__ float weight_at(const void* w, size_t i, unsigned typ
 constexpr int kSlice = 32;           // K values per LDS stage
 constexpr int kPitch = kSlice + 4;   // floats per staged row
 
-// out[n x m] = x[n x k] . W[m x k]^T for a TH x TW tile per 256-thread
-// workgroup (4 waves).
+// The general form: any k, any alignment, and the tiles whose sums overflow or
+// hold infinities or NaN (mm_tile). out[n x m] = x[n x k] . W[m x k]^T for a
+// TH x TW tile per 256-thread workgroup (4 waves), fp32 MFMA on LDS-staged
+// slices of the activations and the decoded weights.
 template <int TH, int TW>
-__device__ void mm_mfma(const EgMM& p) {
+__device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, floatx4* part) {
   static_assert((TH == 16 && (TW == 16 || TW == 64)) || (TH == 64 && TW == 64), "tile shapes of the contract");
-  __shared__ __align__(16) float xs[TH * kPitch];
-  __shared__ __align__(16) float ws[TW * kPitch];
-  __shared__ __align__(16) floatx4 part[(TH == 16 && TW == 16) ? 3 * 64 : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r16 = lane & 15;
   const unsigned row0 = blockIdx.y * TH, col0 = blockIdx.x * TW;
@@ -161,6 +162,367 @@ __device__ void mm_mfma(const EgMM& p) {
         const unsigned row = row0 + rbase + 16 * i + 4 * g + v, col = col0 + cbase + 16 * j + r16;
         if (row < p.n && col < p.m) p.out[(size_t)row * p.m + col] = acc[i][j][v];
       }
+}
+
+// The usual form, k a multiple of 32 and operands aligned (mm_direct_fits),
+// on bf16 MFMA (v_mfma_f32_16x16x32_bf16) with fp32 sums. The activations are
+// split exactly into three bf16 parts (8 + 8 + 8 of their 24 significant
+// bits, by truncation); Q8_0 values are whole numbers of at most 8 bits and
+// BF16 weights are bf16, so three products per weight are exact, and a Q8_0
+// block's scale is one fma on its 32-value dot; F16 weights split exactly into
+// two parts (six products); F32 weights stay on fp32 MFMA
+// (v_mfma_f32_16x16x4f32). A product of 32 values takes 52 matrix cycles per
+// 16 x 16 tile instead of 263, and fewer roundings: the error against a
+// float64 product (2-norm) at 640 x 512 x 2048 is 7.0e-8 for Q8_0, 1.2e-7
+// BF16, 1.5e-7 F16, 2.1e-7 F32, where the general form has 4.0e-7.
+//
+// What bounded the general form was its staging: scalar loads, a decode with
+// a branch and a 64-bit address per weight, two barriers per 32 values. On
+// one card, general / this form, Q8_0: eg2_mm 40 x 512 x 512 16.8 / 4.6 us,
+// eg2_mm64 40 x 768 x 1152 63.6 / 7.9, eg2_mm64x64 640 x 512 x 2048 69.7 /
+// 15.4, 2048 x 768 x 1152 159.8 / 29.6 (bf16 weights 14.7 / 4.3, 53.6 / 6.1,
+// 64.0 / 13.1, 153 / 25).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+struct Bf16Parts {
+  uintx4 part[3];
+};
+// The high halves of two floats as a bf16 pair (a in the low half).
+__device__ __forceinline__ uint32_t high_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
+}
+__device__ __forceinline__ float truncated(float a) { return __uint_as_float(__float_as_uint(a) & 0xffff0000u); }
+// Eight floats as three bf16 parts each: a == part 0 + part 1 + part 2.
+template <int PARTS>
+__device__ __forceinline__ Bf16Parts split_bf16(const float (&v)[8]) {
+  Bf16Parts s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) {
+      s.part[q][i] = high_halves(a, b);
+      if (q + 1 < PARTS) {
+        a = a - truncated(a);
+        b = b - truncated(b);
+      }
+    }
+  }
+  return s;
+}
+__device__ __forceinline__ floatx4 mfma_bf16(uintx4 a, uintx4 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                 0);
+}
+
+// One wave's operands of a step on their way through its own LDS area. A wave
+// reads global memory along the rows (8 lanes a 128-byte line of x: reading
+// the MFMA's order directly, 16 rows to a 16-lane group, a wave touches 64
+// lines per instruction and the step took 3,100-5,200 cycles of loads alone)
+// and picks the fragments up in the MFMA's order: lane 16 g + r holds row (or
+// column) r, values 8 g .. 8 g + 7 of the step. A wave's LDS accesses execute
+// in order and no other wave uses its area, so there is no barrier. Pitches
+// keep the 16 rows of a fragment read on distinct banks.
+constexpr int kStepPitch = 36;  // floats per staged fp32 row
+
+// fp32 rows: x of every type, F32 weights.
+template <int BLOCKS>  // 16-row blocks
+struct StepRows {
+  floatx4 v[2 * BLOCKS];
+  __device__ __forceinline__ void load(const float* m, unsigned k, unsigned row0, unsigned rows, unsigned base) {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < 2 * BLOCKS; ++i)
+      v[i] = *reinterpret_cast<const floatx4*>(m + (size_t)min(row0 + 8 * i + (lane >> 3), rows - 1) * k + base +
+                                              4 * (lane & 7));
+  }
+  __device__ __forceinline__ void put(float* lds) const {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < 2 * BLOCKS; ++i)
+      *reinterpret_cast<floatx4*>(lds + (8 * i + (lane >> 3)) * kStepPitch + 4 * (lane & 7)) = v[i];
+  }
+};
+__device__ __forceinline__ void step_row(const float* lds, int block, float (&f)[8]) {
+  const int lane = threadIdx.x & 63;
+  const floatx4* p = reinterpret_cast<const floatx4*>(lds + (16 * block + (lane & 15)) * kStepPitch + 8 * (lane >> 4));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const floatx4 v = p[i];
+    f[4 * i] = v[0], f[4 * i + 1] = v[1], f[4 * i + 2] = v[2], f[4 * i + 3] = v[3];
+  }
+}
+
+// Weight columns by type: load() along the rows, put() into LDS, get() the
+// lane's fragment of a 16-column block.
+template <unsigned TYPE, int BLOCKS>
+struct StepWeights {  // F16, BF16: 64 bytes a column and step
+  static constexpr int kPitch = 80;
+  uintx4 v[BLOCKS];
+  __device__ __forceinline__ void load(const void* w, unsigned k, unsigned col0, unsigned m, unsigned base) {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j)
+      v[j] = *reinterpret_cast<const uintx4*>(static_cast<const uint16_t*>(w) +
+                                             (size_t)min(col0 + 16 * j + (lane >> 2), m - 1) * k + base + 8 * (lane & 3));
+  }
+  __device__ __forceinline__ void put(float* lds) const {
+    const unsigned lane = threadIdx.x & 63;
+    unsigned char* b = reinterpret_cast<unsigned char*>(lds);
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j)
+      *reinterpret_cast<uintx4*>(b + (16 * j + (lane >> 2)) * kPitch + 16 * (lane & 3)) = v[j];
+  }
+  static __device__ __forceinline__ uintx4 get(const float* lds, int block) {
+    const int lane = threadIdx.x & 63;
+    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const unsigned char*>(lds) +
+                                           (16 * block + (lane & 15)) * kPitch + 16 * (lane >> 4));
+  }
+};
+template <int BLOCKS>
+struct StepWeights<8, BLOCKS> {  // Q8_0: a 34-byte block a column and step, at even addresses
+  static constexpr int kPitch = 40;
+  static constexpr int kScales = 16 * BLOCKS * kPitch / 4;  // floats before the scales
+  uint32_t v[BLOCKS][3];
+  uint32_t shift[BLOCKS];
+  __device__ __forceinline__ void load(const void* w, unsigned k, unsigned col0, unsigned m, unsigned base) {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j) {
+      // The lane's 8 values (and, in lane 0 of the four, the scale) lie in
+      // three aligned words from 8 q bytes into the block rounded down to 4:
+      // each word holds bytes of this block, so none crosses into a page the
+      // matrix does not reach. (Unaligned 8-byte loads cost 0.9 us a step.)
+      const unsigned char* blk = static_cast<const unsigned char*>(w) +
+                                 ((size_t)min(col0 + 16 * j + (lane >> 2), m - 1) * (k / 32) + base / 32) * 34 +
+                                 8 * (lane & 3);
+      shift[j] = (uint32_t)(reinterpret_cast<uintptr_t>(blk) & 2);
+      const uint32_t* p = reinterpret_cast<const uint32_t*>(blk - shift[j]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) v[j][i] = p[i];
+    }
+  }
+  __device__ __forceinline__ void put(float* lds) const {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j) {
+      const unsigned col = 16 * j + (lane >> 2);
+      const bool odd = shift[j] != 0;  // the values start 4 bytes in, not 2
+      const uint32_t lo = odd ? v[j][1] : __builtin_amdgcn_alignbyte(v[j][1], v[j][0], 2);
+      const uint32_t hi = odd ? v[j][2] : __builtin_amdgcn_alignbyte(v[j][2], v[j][1], 2);
+      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(lds) + col * kPitch + 8 * (lane & 3)) =
+          make_uint2(lo, hi);
+      if ((lane & 3) == 0) lds[kScales + col] = eg2::fp16_bits_to_fp32(odd ? v[j][0] >> 16 : v[j][0] & 0xffffu);
+    }
+  }
+  static __device__ __forceinline__ uintx4 get(const float* lds, int block, float& scale) {  // as bf16
+    const int lane = threadIdx.x & 63;
+    const uint2 q = *reinterpret_cast<const uint2*>(reinterpret_cast<const unsigned char*>(lds) +
+                                                    (16 * block + (lane & 15)) * kPitch + 8 * (lane >> 4));
+    scale = lds[kScales + 16 * block + (lane & 15)];
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[e] = (float)(int8_t)(q.x >> (8 * e));
+      f[4 + e] = (float)(int8_t)(q.y >> (8 * e));
+    }
+    return split_bf16<1>(f).part[0];
+  }
+};
+template <int BLOCKS>
+struct StepWeights<0, BLOCKS> {
+  StepRows<BLOCKS> rows;
+  __device__ __forceinline__ void load(const void* w, unsigned k, unsigned col0, unsigned m, unsigned base) {
+    rows.load(static_cast<const float*>(w), k, col0, m, base);
+  }
+  __device__ __forceinline__ void put(float* lds) const { rows.put(lds); }
+};
+// LDS floats per wave: the rows, then the widest weights (F32).
+template <int RB, int CB>
+constexpr int kStepLds = 16 * (RB + CB) * kStepPitch;
+
+// acc[i][j] += rows 16 i .. of the step's activations times columns 16 j .. of
+// its weights, from the wave's LDS area. The products run part by part over
+// several tiles, so that an MFMA does not wait for the one before it.
+template <unsigned TYPE, int RB, int CB>
+__device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx4 (&acc)[RB][CB]) {
+  if constexpr (TYPE == 0) {
+    float a[RB][8], b[CB][8];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) step_row(xs, i, a[i]);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) step_row(ws, j, b[j]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+  } else {
+    Bf16Parts a[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      float f[8];
+      step_row(xs, i, f);
+      a[i] = split_bf16<3>(f);
+    }
+    if constexpr (TYPE == 8) {
+      constexpr int JB = RB == 1 ? CB : 1;  // column blocks at a time: RB JB = 4 independent dots
+#pragma unroll
+      for (int j0 = 0; j0 < CB; j0 += JB) {
+        uintx4 b[JB];
+        float d[JB];
+        floatx4 dot[RB][JB];
+#pragma unroll
+        for (int j = 0; j < JB; ++j) {
+          b[j] = StepWeights<8, CB>::get(ws, j0 + j, d[j]);
+#pragma unroll
+          for (int i = 0; i < RB; ++i) dot[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int q = 2; q >= 0; --q)
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < JB; ++j) dot[i][j] = mfma_bf16(a[i].part[q], b[j], dot[i][j]);
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[i][j0 + j][v] = __builtin_fmaf(dot[i][j][v], d[j], acc[i][j0 + j][v]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        const uintx4 raw = StepWeights<TYPE, CB>::get(ws, j);
+        constexpr int kParts = TYPE == 1 ? 2 : 1;
+        uintx4 b[2] = {raw, raw};
+        if constexpr (TYPE == 1) {
+                    float f[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] = eg2::fp16_bits_to_fp32((raw[e / 2] >> (16 * (e & 1))) & 0xffffu);
+          const Bf16Parts s = split_bf16<2>(f);
+          b[0] = s.part[0];
+          b[1] = s.part[1];
+        }
+#pragma unroll
+        for (int q = 2; q >= 0; --q)
+#pragma unroll
+          for (int c = kParts - 1; c >= 0; --c)
+#pragma unroll
+            for (int i = 0; i < RB; ++i) acc[i][j] = mfma_bf16(a[i].part[q], b[c], acc[i][j]);
+      }
+    }
+  }
+}
+
+// One wave's 16 RB x 16 CB tile at (row0, col0): steps first, first + stride,
+// ... of the k / 32, DEPTH of them in flight. Rows past n and columns past m
+// repeat the last one.
+template <unsigned TYPE, int RB, int CB, int DEPTH>
+__device__ __forceinline__ void mm_direct(const EgMM& p, unsigned row0, unsigned col0, unsigned first, unsigned stride,
+                                          float* lds, floatx4 (&acc)[RB][CB]) {
+  const unsigned steps = p.k / 32;
+  float *xs = lds, *ws = lds + 16 * RB * kStepPitch;
+  StepRows<RB> x[DEPTH];
+  StepWeights<TYPE, CB> w[DEPTH];
+  auto load = [&](int slot, unsigned step) {
+    const unsigned base = 32 * min(step, steps - 1);  // past the end: the last step again, not used
+    w[slot].load(p.weight, p.k, col0, p.m, base);
+    x[slot].load(p.x, p.k, row0, p.n, base);
+  };
+#pragma unroll
+  for (int s = 0; s < DEPTH; ++s) load(s, first + s * stride);
+  for (unsigned step = first; step < steps; step += DEPTH * stride) {
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) {
+      if (step + s * stride >= steps) break;  // uniform
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // after the previous step's fragment reads
+      w[s].put(ws);
+      x[s].put(xs);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      load(s, step + (s + DEPTH) * stride);
+      mm_step<TYPE, RB, CB>(xs, ws, acc);
+    }
+  }
+}
+
+__device__ __forceinline__ bool mm_direct_fits(const EgMM& p) {
+  const uintptr_t w = reinterpret_cast<uintptr_t>(p.weight), x = reinterpret_cast<uintptr_t>(p.x);
+  return p.k % 32 == 0 && p.k > 0 && x % 16 == 0 && (p.type == 8 ? w % 2 == 0 : w % 16 == 0);
+}
+
+// A TH x TW tile per workgroup: each of the 4 waves takes the whole tile over
+// every fourth step (so an activation is loaded and split once per workgroup,
+// and a 512-deep product is 4 steps, not 16, of a wave's serial chain), and
+// the four partial tiles are added through LDS, wave w finishing column block
+// w. Where a sum comes out infinite or NaN -- non-finite operands, or a Q8_0
+// dot that overflows before its scale -- the tile is computed again in the
+// general form, which multiplies decoded weights.
+// Returns whether this thread's sums are finite; stores nothing unless every
+// thread's are.
+template <unsigned TYPE, int TH, int TW>
+__device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStepLds<TH / 16, TW / 16>],
+                                              floatx4 (*part)[TW / 16][64]) {
+  constexpr int RB = TH / 16, CB = TW / 16, kDepth = TH == 64 ? 1 : 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
+  const unsigned row0 = blockIdx.y * TH, col0 = blockIdx.x * TW;
+  floatx4 acc[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, wave, 4, step[wave], acc);
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+    __syncthreads();  // the waves' step areas, then the previous row block's parts, are no longer read
+#pragma unroll
+    for (int j = 0; j < CB; ++j) part[wave][j][lane] = acc[i][j];
+    __syncthreads();
+    if (wave < CB) {
+      acc[i][0] = ((part[0][wave][lane] + part[1][wave][lane]) + part[2][wave][lane]) + part[3][wave][lane];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) finite = finite && fabsf(acc[i][0][v]) <= 3.40282347e38f;
+    }
+  }
+  if (__syncthreads_or(!finite)) return false;
+  if (wave >= CB) return true;
+  const unsigned col = col0 + 16 * wave + r;
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const unsigned row = row0 + 16 * i + 4 * g + v;
+      if (row < p.n && col < p.m) p.out[(size_t)row * p.m + col] = acc[i][0][v];
+    }
+  return true;
+}
+
+template <int TH, int TW>
+__device__ __forceinline__ void mm_tile(const EgMM& p) {
+  __shared__ union {
+    alignas(16) float step[4][kStepLds<TH / 16, TW / 16>];
+    floatx4 part[4][TW / 16][64];
+    struct {
+      floatx4 part[(TH == 16 && TW == 16) ? 3 * 64 : 1];
+      alignas(16) float xs[TH * kPitch], ws[TW * kPitch];
+    } general;
+  } lds;
+  if (blockIdx.y * TH >= p.n || blockIdx.x * TW >= p.m) return;
+  bool done = false;  // uniform
+  if (mm_direct_fits(p)) {
+    switch (p.type) {
+      case 0: done = mm_tile_typed<0, TH, TW>(p, lds.step, lds.part); break;
+      case 1: done = mm_tile_typed<1, TH, TW>(p, lds.step, lds.part); break;
+      case 30: done = mm_tile_typed<30, TH, TW>(p, lds.step, lds.part); break;
+      default: done = mm_tile_typed<8, TH, TW>(p, lds.step, lds.part); break;
+    }
+  }
+  if (!done) mm_general<TH, TW>(p, lds.general.xs, lds.general.ws, lds.general.part);
 }
 
 // -------------------------------------------------------------- row sums
@@ -349,10 +711,10 @@ extern "C" __global__ void eg2_gather768(EgGather p) {
 }
 
 // kernels/eg2.c:41-119 semantics, four tile shapes.
-extern "C" __global__ void __launch_bounds__(256) eg2_mm(EgMM p) { mm_mfma<16, 16>(p); }
-extern "C" __global__ void __launch_bounds__(256) eg2_mm64(EgMM p) { mm_mfma<16, 64>(p); }
-extern "C" __global__ void __launch_bounds__(256) eg2_mm64x64(EgMM p) { mm_mfma<64, 64>(p); }
-extern "C" __global__ void __launch_bounds__(256) eg2_mmstep8(EgMM p) { mm_mfma<64, 64>(p); }
+extern "C" __global__ void __launch_bounds__(256) eg2_mm(EgMM p) { mm_tile<16, 16>(p); }
+extern "C" __global__ void __launch_bounds__(256) eg2_mm64(EgMM p) { mm_tile<16, 64>(p); }
+extern "C" __global__ void __launch_bounds__(256) eg2_mm64x64(EgMM p) { mm_tile<64, 64>(p); }
+extern "C" __global__ void __launch_bounds__(256) eg2_mmstep8(EgMM p) { mm_tile<64, 64>(p); }
 
 // out = ((x * scale) * inv) * w, inv = 1/sqrt(mean((x * scale)^2) + 1e-6);
 // w may be NULL (= 1); out == x is valid (kernels/eg2.c:121-133 semantics).

@@ -1,0 +1,73 @@
+"""The by-name projections' two forms (kernels_abi.hip): the bf16-part form of
+aligned operands with k a multiple of 32, against a float64 product and
+against the general form (reached by moving an operand off its alignment), at
+the sizes where it can go wrong: partial tiles both ways, odd block counts
+(Q8_0 blocks then start on both halves of a word), one step and a step count
+that leaves waves idle; and infinities, NaN and a Q8_0 dot that overflows
+before its scale, which the general form must decide, bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_operators import MM_VARIANTS, dev, encode_weights, host
+
+pytestmark = pytest.mark.gpu
+TYPES = [0, 1, 8, 30]
+
+
+def run(eg2, gpu, variant, x, raw, wtype, m, x_shift=0, w_shift=0):
+    """x_shift floats and w_shift bytes put before the operands."""
+    import torch
+
+    name, width, height, _ = variant
+    n, k = x.shape
+    xd = dev(np.concatenate([np.zeros(x_shift, np.float32), x.reshape(-1)]), gpu)
+    wd = dev(np.concatenate([np.zeros(w_shift, np.uint8), raw.reshape(-1).view(np.uint8)]), gpu)
+    yd = torch.full((n, m), float("nan"), dtype=torch.float32, device=gpu)
+    rec = eg2.EgMM(yd.data_ptr(), xd.data_ptr() + 4 * x_shift, wd.data_ptr() + w_shift, n, k, m, wtype)
+    eg2.ops.op(name, rec, ((m + width - 1) // width, (n + height - 1) // height), 256)
+    return host(yd)
+
+
+@pytest.mark.parametrize("variant", MM_VARIANTS[:3], ids=[v[0] for v in MM_VARIANTS[:3]])
+@pytest.mark.parametrize("wtype", TYPES)
+@pytest.mark.parametrize("shape", [(1, 32, 1), (17, 96, 35), (65, 160, 130), (130, 768, 67)])
+def test_aligned_form_against_float64_and_general(eg2, gpu, variant, wtype, shape):
+    n, k, m = shape
+    rng = np.random.default_rng(n + k + wtype)
+    x = (rng.standard_normal((n, k)) * 10.0 ** rng.uniform(-3, 3, (n, 1))).astype(np.float32)
+    raw, dec = encode_weights((rng.standard_normal((m, k)) * 0.05).astype(np.float32), wtype)
+    x64, w64 = x.astype(np.float64), dec.astype(np.float64)
+    want, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64).T
+    got = run(eg2, gpu, variant, x, raw, wtype, m)
+    general = run(eg2, gpu, variant, x, raw, wtype, m, x_shift=1)
+    # A 32-bit sum of k products: at most k roundings of 2^-24 each.
+    assert np.all(np.abs(got - want) <= k * 2.0 ** -24 * mag)
+    # Precision is not lost against the general form: the rms of the errors in
+    # units of sum |x w| (over enough outputs to be steady). F32 weights have
+    # the same fp32 MFMA chains in both, split into equally long ones over the
+    # 16 x 16 tile's waves only where k is a multiple of 128.
+    if n * m >= 500 and (wtype != 0 or k % 128 == 0):
+        rms = lambda y: np.sqrt((((y - want) / mag) ** 2).mean())
+        assert rms(got) <= 1.1 * rms(general)
+    if wtype == 8:  # blocks at the other parity, and at odd addresses (the general form)
+        assert np.array_equal(run(eg2, gpu, variant, x, raw, wtype, m, w_shift=2), got)
+        assert np.array_equal(run(eg2, gpu, variant, x, raw, wtype, m, w_shift=1), general)
+
+
+@pytest.mark.parametrize("variant", MM_VARIANTS[:3], ids=[v[0] for v in MM_VARIANTS[:3]])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_non_finite_sums_take_the_general_form(eg2, gpu, variant, wtype):
+    n, k, m = 70, 128, 70
+    rng = np.random.default_rng(wtype)
+    w = (rng.standard_normal((m, k)) * 0.05).astype(np.float32)
+    w[3, :32] = 0.0
+    raw, _ = encode_weights(w, wtype)
+    for bad in (np.inf, -np.inf, np.nan, np.uint32(0x7F800001).view(np.float32), np.float32(3e38)):
+        x = rng.standard_normal((n, k)).astype(np.float32)
+        x[5, 7] = bad
+        got = run(eg2, gpu, variant, x, raw, wtype, m)
+        general = run(eg2, gpu, variant, x, raw, wtype, m, x_shift=1)
+        assert np.array_equal(np.isnan(got), np.isnan(general))
+        assert np.array_equal(got[5], general[5], equal_nan=True) or bad == np.float32(3e38)
+        ok = np.isfinite(general)
+        assert np.array_equal(ok, np.isfinite(got)) and np.allclose(got[ok], general[ok], rtol=1e-4, atol=1e-4)
