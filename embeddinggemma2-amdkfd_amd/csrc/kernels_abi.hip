@@ -620,13 +620,16 @@ __device__ __forceinline__ void rotate(float a, float b, float c, float s, float
 // keys [bounds[2t], bounds[2t+1]) clipped to |t - s| <= window (window >
 // 0). q rows of D floats per (t, h); K/V rows of KVS floats with head h's
 // KV block at (h / GROUP) * D.
+// Computed by one wave with LDS of its own (qs, ps).
+__device__ __forceinline__ void wave_lds_order() {  // a wave's LDS accesses execute in order: keep the compiler to it
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 template <int D, int HEADS, int KVS, int GROUP>
-__device__ void attention_chunked(const EgAttention& p) {
+__device__ __forceinline__ void attention_chunked(const EgAttention& p, unsigned row, floatx4* qs, float* ps) {
   static_assert(D % 256 == 0, "lanes own float4s of the context");
   constexpr int CV = D / 256;  // float4 of the context per lane
-  __shared__ __align__(16) floatx4 qs[D / 4];
-  __shared__ float ps[64];
-  const unsigned row = blockIdx.x, lane = threadIdx.x;
+  const unsigned lane = threadIdx.x & 63;
   const unsigned t = row / HEADS, h = row % HEADS, kv = (h / GROUP) * D;
   if (t >= p.n) return;
   unsigned lo = p.bounds[2 * t], hi = p.bounds[2 * t + 1];
@@ -635,7 +638,7 @@ __device__ void attention_chunked(const EgAttention& p) {
     hi = min(hi, t + p.window + 1);
   }
   for (unsigned c = lane; c < D / 4; c += 64) qs[c] = reinterpret_cast<const floatx4*>(p.q + (size_t)row * D)[c];
-  __syncthreads();
+  wave_lds_order();
   float run_max = -__builtin_inff(), den = 0.0f;
   floatx4 acc[CV];
 #pragma unroll
@@ -659,7 +662,7 @@ __device__ void attention_chunked(const EgAttention& p) {
     const float pk = key < hi ? eg2::libm::expf(score - next) : 0.0f;
     den = den * alpha + dpp_wave_sum(pk);
     ps[lane] = pk;
-    __syncthreads();
+    wave_lds_order();
 #pragma unroll
     for (int u = 0; u < CV; ++u) acc[u] = acc[u] * alpha;
     const unsigned count = min(64u, hi - c0);
@@ -673,13 +676,278 @@ __device__ void attention_chunked(const EgAttention& p) {
         for (int e = 0; e < 4; ++e) acc[u][e] = __builtin_fmaf(w, v4[e], acc[u][e]);
       }
     }
-    __syncthreads();  // ps is rewritten by the next chunk
+    wave_lds_order();  // ps is rewritten by the next chunk
     run_max = next;
   }
   const float inv = hi > lo ? 1.0f / den : 0.0f;
 #pragma unroll
   for (int u = 0; u < CV; ++u)
     *reinterpret_cast<floatx4*>(p.out + (size_t)row * D + 4 * lane + 256 * u) = acc[u] * inv;
+}
+
+// The same attention over tiles of 16 tokens x one head, which eg2_op_launch
+// takes for the contract's whole grid from kTileTokens tokens on (the
+// by-symbol kernel's one wave per (token, head) reads every key and value row
+// once per token and head: 17 GB from the L2 for one 2048-token sequence). A
+// workgroup of kTileWaves waves shares the 16 queries in LDS; wave w takes
+// every kTileWaves-th 16-key block of the keys that any of its tokens has,
+// with its own running maximum, sum and context (the softmax recurrence of the
+// form above), and the waves' results are rescaled to the common maximum and
+// added at the end. Both products run on fp32 MFMA (v_mfma_f32_16x16x4f32):
+//  - scores: lane 16 g + r feeds key r; one float4 of its row, dimensions
+//    16 E + 4 g .., is four MFMAs (q from LDS in the same order). The key rows
+//    come through the wave's LDS 64 dimensions at a time, read along the rows
+//    (in the MFMA's order a load touches 64 lines, which alone took twice the
+//    MFMAs' time), the next 64 on their way meanwhile;
+//  - context: the 16 x 16 weights go through LDS to the operand order (lane
+//    16 g + r: query r, keys 4 g .. 4 g + 3), and a lane's float4 of a value
+//    row, dimensions 64 T + 4 r .., feeds four output tiles.
+// A key outside a token's range weighs 0 there. The 2-norm error to a float64
+// softmax is that of the form above or less (2.2e-7 against 2.8e-7 at 1021
+// tokens in 9 texts, 3.8e-7 against 8.4e-7 on one of 2048). Bound by the
+// MFMAs (128 of 33 cycles per 16 x 16 scores) and, over few keys, by the
+// chain of one block: eg2_attention256, that form / this one in us: 1021
+// tokens in 9 texts 112 / 27, 2048 in 16 320 / 70, one of 2048 2,240 / 223;
+// eg2_attention512, one of 2048, 4,451 / 459.
+constexpr int kTileWaves = 8;
+// Below this the packing decides (its lengths are on the device): 256 tokens
+// in 4 texts 13.0 / 10.6, in 32 texts 6.2 / 10.1; 512 in 32 texts of 16, the
+// shortest that still gains, 10.7 / 10.4 (eg2_attention512 18.4 / 17.6).
+constexpr unsigned kTileTokens = 512;
+
+template <int D>
+struct AttentionTileLds {
+  alignas(16) float q[16][D + 4];
+  alignas(16) float p[kTileWaves][16][20];
+  float m[kTileWaves][16], l[kTileWaves][16];
+  // 64 dimensions of a wave's 16 keys; at the end, of its 16 rows' context.
+  alignas(16) float part[kTileWaves][16][68];
+  uint64_t exp_tab[32];
+};
+
+// Reductions over the 16 lanes of a DPP row, on every lane of it.
+template <int CTRL>
+__device__ __forceinline__ float dpp16(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, dpp16<0xB1>(v));
+  v = fmaxf(v, dpp16<0x4E>(v));
+  v = fmaxf(v, dpp16<0x141>(v));
+  return fmaxf(v, dpp16<0x140>(v));
+}
+__device__ __forceinline__ float row16_sum(float v) {
+  v = v + dpp16<0xB1>(v);
+  v = v + dpp16<0x4E>(v);
+  v = v + dpp16<0x141>(v);
+  return v + dpp16<0x140>(v);
+}
+
+template <int D, int HEADS, int KVS, int GROUP>
+__global__ void __launch_bounds__(64 * kTileWaves)
+attention_tile_kernel(EgAttention p) {
+  constexpr int T = D / 64;  // 64-dimension parts of the context
+  __shared__ AttentionTileLds<D> lds;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const unsigned t0 = 16 * blockIdx.x, h = blockIdx.y, kv = (h / GROUP) * D;
+  for (int c = tid; c < 16 * D / 4; c += 64 * kTileWaves) {
+    const int row = c / (D / 4), e = c % (D / 4);
+    *reinterpret_cast<floatx4*>(&lds.q[row][4 * e]) =
+        *reinterpret_cast<const floatx4*>(p.q + ((size_t)min(t0 + row, p.n - 1) * HEADS + h) * D + 4 * e);
+  }
+  if (tid < 32) lds.exp_tab[tid] = eg2::libm::kExp2Tab.t[tid];
+  auto exp_ = [&](float x) { return eg2::libm::expf_tab(x, lds.exp_tab); };
+  // Key ranges: of token t0 + r in every lane (for the union), of the lane's
+  // output rows 4 g + v.
+  auto range = [&](unsigned t, unsigned& lo, unsigned& hi) {
+    lo = hi = 0;
+    if (t >= p.n) return;
+    lo = p.bounds[2 * t];
+    hi = p.bounds[2 * t + 1];
+    if (p.window) {
+      if (t > p.window) lo = max(lo, t - p.window);
+      hi = min(hi, t + p.window + 1);
+    }
+    if (hi <= lo) lo = hi = 0;
+  };
+  unsigned lo[4], hi[4], first = 0xffffffffu, last = 0;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) range(t0 + 4 * g + v, lo[v], hi[v]);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const unsigned a = __builtin_amdgcn_readlane(lo[i & 3], 16 * (i >> 2)), b = __builtin_amdgcn_readlane(hi[i & 3], 16 * (i >> 2));
+    if (b > a) {
+      first = min(first, a);
+      last = max(last, b);
+    }
+  }
+  first = min(first, last);
+  float m[4], l[4];
+  floatx4 acc[4 * T];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) m[v] = -__builtin_inff(), l[v] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4 * T; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  __syncthreads();
+  // Rows 4 i + lane / 16 of a key block, dimensions 64 part + 4 (lane % 16) ..
+  // (rows past the last repeat it; their scores are masked).
+  floatx4 kr[4];
+  auto load_k = [&](unsigned k0, int part) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      kr[i] = *reinterpret_cast<const floatx4*>(p.k + (size_t)min(k0 + 4 * i + g, last - 1) * KVS + kv + 64 * part + 4 * r);
+  };
+  bool polluted = false;
+  if (first + 16 * w < last) load_k(first + 16 * w, 0);
+  for (unsigned k0 = first + 16 * w; k0 < last; k0 += 16 * kTileWaves) {
+    // Scores of keys k0 .. + 15, in four chains.
+    floatx4 s[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int part = 0; part < T; ++part) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<floatx4*>(&lds.part[w][4 * i + g][4 * r]) = kr[i];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (part + 1 < T)
+        load_k(k0, part + 1);
+      else if (k0 + 16 * kTileWaves < last)
+        load_k(k0 + 16 * kTileWaves, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const floatx4 kf = *reinterpret_cast<const floatx4*>(&lds.part[w][r][16 * e + 4 * g]);
+        const floatx4 qf = *reinterpret_cast<const floatx4*>(&lds.q[r][64 * part + 16 * e + 4 * g]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c], kf[c], s[c], 0, 0, 0);
+      }
+    }
+    // The block's first value rows, on their way during the softmax: keys
+    // k0 + 4 g + j, kAhead j in flight (one at 512 dimensions, whose context
+    // takes half of the registers).
+    constexpr int kAhead = D == 256 ? 2 : 1;
+    floatx4 vr[kAhead][T];
+    auto load_v = [&](int slot, int j) {
+      const float* vrow = p.v + (size_t)min(k0 + 4 * g + j, last - 1) * KVS + kv + 4 * r;
+#pragma unroll
+      for (int part = 0; part < T; ++part) vr[slot][part] = *reinterpret_cast<const floatx4*>(vrow + 64 * part);
+    };
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) load_v(j, j);
+    float score[4], next[4];
+    bool grown = false;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {  // row 4 g + v, key k0 + r
+      const bool in = k0 + r >= lo[v] && k0 + r < hi[v];
+      score[v] = in ? (s[0][v] + s[1][v]) + (s[2][v] + s[3][v]) : -__builtin_inff();
+      next[v] = fmaxf(m[v], row16_max(score[v]));
+      grown = grown || next[v] != m[v];
+    }
+    if (__any(grown)) {
+      float alpha[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        alpha[v] = next[v] == -__builtin_inff() ? 0.0f : exp_(m[v] - next[v]);  // no key of this row yet: all zero
+        l[v] = l[v] * alpha[v];
+        m[v] = next[v];
+      }
+#pragma unroll
+      for (int i = 0; i < 4 * T; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[i][v] = acc[i][v] * alpha[v];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const bool in = k0 + r >= lo[v] && k0 + r < hi[v];
+      const float pk = in ? exp_(score[v] - m[v]) : 0.0f;
+      l[v] = l[v] + row16_sum(pk);
+      lds.p[w][4 * g + v][r] = pk;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const floatx4 pf = *reinterpret_cast<const floatx4*>(&lds.p[w][r][4 * g]);  // query r, keys 4 g ..
+    // A key outside a row's range weighs +0, but +0 times an infinite or NaN
+    // value is NaN: where some row does not have all 16 keys, such values send
+    // the whole tile to the per-row form below.
+    bool all_in = true;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) all_in = all_in && lo[v] <= k0 && k0 + 16 <= hi[v];
+    const bool partial = !__all(all_in);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (partial) {  // uniform
+        float probe = 0.0f;
+#pragma unroll
+        for (int part = 0; part < T; ++part)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) probe = __builtin_fmaf(vr[j % kAhead][part][i], 0.0f, probe);
+        polluted = polluted || !(probe == 0.0f);
+      }
+#pragma unroll
+      for (int part = 0; part < T; ++part)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[4 * part + i] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(pf[j], vr[j % kAhead][part][i], acc[4 * part + i], 0, 0, 0);
+      if (j + kAhead < 4) load_v(j % kAhead, j + kAhead);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // p is rewritten by the next block
+  }
+  // The waves' contexts brought to the rows' common maximum and added; thread
+  // 16 i + row computes wave i's factor for the row.
+  if (__syncthreads_or(polluted)) {
+    for (unsigned i = w; i < 16 && t0 + i < p.n; i += kTileWaves)
+      attention_chunked<D, HEADS, KVS, GROUP>(p, (t0 + i) * HEADS + h, reinterpret_cast<floatx4*>(lds.q[w]),
+                                              lds.part[w][0]);
+    return;
+  }
+  if (r == 0) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) lds.m[w][4 * g + v] = m[v], lds.l[w][4 * g + v] = l[v];
+  }
+  __syncthreads();
+  if (tid < 16 * kTileWaves) {
+    const int row = tid & 15;
+    const float own = lds.m[tid >> 4][row];
+    float top = own;
+#pragma unroll
+    for (int i = 0; i < kTileWaves; ++i) top = fmaxf(top, lds.m[i][row]);
+    lds.p[tid >> 4][row][0] = own == -__builtin_inff() ? 0.0f : exp_(own - top);
+  }
+  __syncthreads();
+  float scale[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int row = 4 * g + v;
+    float den = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kTileWaves; ++i) den = den + lds.l[i][row] * lds.p[i][row][0];
+    scale[v] = hi[v] > lo[v] ? lds.p[w][row][0] / den : 0.0f;
+  }
+#pragma unroll
+  for (int part = 0; part < T; ++part) {
+    if (part) __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      floatx4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = acc[4 * part + i][v] * scale[v];
+      *reinterpret_cast<floatx4*>(&lds.part[w][4 * g + v][4 * r]) = o;
+    }
+    __syncthreads();
+    const int row = tid >> 5, e = 2 * (tid & 31);  // 512 threads x 2 outputs
+    float a = 0.0f, b = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kTileWaves; ++i) {
+      a = a + lds.part[i][row][e];
+      b = b + lds.part[i][row][e + 1];
+    }
+    if (t0 + row < p.n) {
+      float* dst = p.out + ((size_t)(t0 + row) * HEADS + h) * D + 64 * part + e;
+      dst[0] = a;
+      dst[1] = b;
+    }
+  }
 }
 
 }  // namespace
@@ -755,14 +1023,20 @@ extern "C" __global__ void eg2_rope(EgRope p) {
 // kernels/eg2.c:145-170 semantics: 4 query heads per token; d 256 reads KV
 // head h/2 of two, d 512 the single KV head (K/V rows of 512 floats).
 extern "C" __global__ void __launch_bounds__(64) eg2_attention256(EgAttention p) {
-  attention_chunked<256, 4, 512, 2>(p);
+  __shared__ __align__(16) floatx4 qs[64];
+  __shared__ float ps[64];
+  attention_chunked<256, 4, 512, 2>(p, blockIdx.x, qs, ps);
 }
 extern "C" __global__ void __launch_bounds__(64) eg2_attention512(EgAttention p) {
-  attention_chunked<512, 4, 512, 4>(p);
+  __shared__ __align__(16) floatx4 qs[128];
+  __shared__ float ps[64];
+  attention_chunked<512, 4, 512, 4>(p, blockIdx.x, qs, ps);
 }
 // 3 query heads sharing one KV head of 256 (K/V rows of 256 floats).
 extern "C" __global__ void __launch_bounds__(64) eg2_attention256x3(EgAttention p) {
-  attention_chunked<256, 3, 256, 3>(p);
+  __shared__ __align__(16) floatx4 qs[64];
+  __shared__ float ps[64];
+  attention_chunked<256, 3, 256, 3>(p, blockIdx.x, qs, ps);
 }
 
 // Mode 0: (x + other) * scale; 1: gelu(x) * other; 2: gelu(x) * the
@@ -868,6 +1142,8 @@ struct OpEntry {
   size_t record_size;
   Block block;
   bool (*valid)(const void* record);
+  const void* tile = nullptr;  // attention: the tiled kernel for the whole grid of heads x n
+  unsigned heads = 0;
 };
 
 template <class R>
@@ -915,11 +1191,11 @@ const OpEntry kOps[] = {
     {"eg2_norm", reinterpret_cast<const void*>(&eg2_norm), sizeof(EgNorm), Block::k64, valid_norm},
     {"eg2_rope", reinterpret_cast<const void*>(&eg2_rope), sizeof(EgRope), Block::kAny, valid_rope},
     {"eg2_attention256", reinterpret_cast<const void*>(&eg2_attention256), sizeof(EgAttention), Block::k64,
-     valid_attention},
+     valid_attention, reinterpret_cast<const void*>(&attention_tile_kernel<256, 4, 512, 2>), 4},
     {"eg2_attention512", reinterpret_cast<const void*>(&eg2_attention512), sizeof(EgAttention), Block::k64,
-     valid_attention},
+     valid_attention, reinterpret_cast<const void*>(&attention_tile_kernel<512, 4, 512, 4>), 4},
     {"eg2_attention256x3", reinterpret_cast<const void*>(&eg2_attention256x3), sizeof(EgAttention), Block::k64,
-     valid_attention},
+     valid_attention, reinterpret_cast<const void*>(&attention_tile_kernel<256, 3, 256, 3>), 3},
     {"eg2_element", reinterpret_cast<const void*>(&eg2_element), sizeof(EgElement), Block::kAny, valid_element},
     {"eg2_pool", reinterpret_cast<const void*>(&eg2_pool), sizeof(EgPool), Block::kAny, valid_pool},
     {"eg2_norm_residual", reinterpret_cast<const void*>(&eg2_norm_residual), sizeof(EgNormResidual), Block::k64,
@@ -940,6 +1216,15 @@ extern "C" int eg2_op_launch(const char* name, const void* record, size_t record
     if ((op.block == Block::k64 && block != 64) || (op.block == Block::k256 && block != 256))
       return (int)hipErrorInvalidValue;
     if (!op.valid(record)) return (int)hipErrorInvalidValue;
+    if (op.tile && grid_y == 1) {
+      const EgAttention& p = as<EgAttention>(record);
+      if (p.n >= kTileTokens && (uint64_t)op.heads * p.n == grid_x) {
+        EgAttention rec = p;
+        void* args[] = {&rec};
+        return (int)hipLaunchKernel(op.tile, dim3((p.n + 15) / 16, op.heads), dim3(64 * kTileWaves), args, 0,
+                                    reinterpret_cast<hipStream_t>(stream));
+      }
+    }
     // The kernarg segment is the record itself: copy it so the caller's
     // buffer may be reused as soon as this returns.
     alignas(16) unsigned char kernarg[64];

@@ -1,0 +1,84 @@
+"""The by-name attention's tiled kernel (kernels_abi.hip), taken for the whole
+grid of 512 tokens or more, against a float64 softmax at the reference
+operator test's tolerance (tests/kernels.cpp:114-137): the first size that
+takes it and the last that does not, a partial last tile, sequences of one
+token and of more key blocks than waves, tiles that straddle sequences,
+tokens with no key, ranges unlike their neighbours', and windows."""
+import numpy as np
+import pytest
+
+from test_gpu_operators import attention_reference, dev, host
+
+pytestmark = pytest.mark.gpu
+OPS = {"eg2_attention256": (4, 256, 512, 2), "eg2_attention512": (4, 512, 512, 4), "eg2_attention256x3": (3, 256, 256, 3)}
+
+
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("lens,window,odd", [([511], 0, False), ([512], 0, False), ([1, 300, 17, 211, 1], 0, True),
+                                             ([1, 300, 17, 211, 1], 50, True), ([16] * 33, 3, False)],
+                         ids=["511", "512", "ragged", "ragged-w50", "33x16-w3"])
+def test_tiled_attention_against_float64(eg2, gpu, op, lens, window, odd):
+    import torch
+
+    heads, d, kvs, group = OPS[op]
+    n = sum(lens)
+    rng = np.random.default_rng(n + window + d)
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    bounds = np.array([(starts[s], starts[s + 1]) for s in range(len(lens)) for _ in range(lens[s])], np.uint32)
+    if odd:
+        bounds[40] = (7, 7)       # no key
+        bounds[41] = (9, 3)       # none either
+        bounds[300] = (2, 450)    # a range of its own
+        bounds[n - 1] = (0, n)
+    q = (rng.standard_normal(n * heads * d) / np.sqrt(d)).astype(np.float32)
+    k = rng.standard_normal(n * kvs).astype(np.float32)
+    v = rng.standard_normal(n * kvs).astype(np.float32)
+    y = torch.full((n * heads * d,), float("nan"), device=gpu)
+    qd, kd, vd, bd = dev(q, gpu), dev(k, gpu), dev(v, gpu), dev(bounds.reshape(-1).view(np.int32), gpu)
+    rec = eg2.EgAttention(y.data_ptr(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), bd.data_ptr(), n, window)
+    eg2.ops.op(op, rec, heads * n, 64)
+    got = host(y).reshape(n, heads, d)
+    empty = []
+    full = bounds.copy()
+    for t in range(n):
+        lo, hi = int(bounds[t, 0]), int(bounds[t, 1])
+        if window:
+            lo, hi = max(lo, t - window), min(hi, t + window + 1)
+        if hi <= lo:
+            empty.append(t)
+            full[t] = (t, t + 1)  # the reference needs a key; compared with zero below
+    want = attention_reference(q, k, v, full.reshape(-1), n, heads, d, kvs, lambda h: h // group, window)
+    want = want.reshape(n, heads, d)
+    want[empty] = 0.0
+    assert np.abs(got - want).max() <= 2e-5
+    assert (got[empty] == 0).all()
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_non_finite_values_stay_in_their_sequence(eg2, gpu, op):
+    """An infinite and a NaN value row: the sequence that holds them is not
+    finite, and the others are what they are without them. (A tile that meets
+    such values in a partial block is computed in the per-row form, so its rows
+    may differ by both forms' tolerance, 2 x 2e-5.)"""
+    import torch
+
+    heads, d, kvs, _ = OPS[op]
+    lens = [250, 21, 9, 300]
+    n = sum(lens)
+    rng = np.random.default_rng(d)
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    bounds = np.array([(starts[s], starts[s + 1]) for s in range(len(lens)) for _ in range(lens[s])], np.uint32)
+    q, k, v = ((rng.standard_normal(n * w) * 0.1).astype(np.float32) for w in (heads * d, kvs, kvs))
+    bad = v.reshape(n, kvs).copy()
+    bad[252, 5] = np.inf
+    bad[270, 300 % kvs] = np.nan
+    out = []
+    for values in (v, bad):
+        y = torch.full((n * heads * d,), float("nan"), device=gpu)
+        t = [dev(a, gpu) for a in (q, k, values.reshape(-1), bounds.reshape(-1).view(np.int32))]
+        rec = eg2.EgAttention(y.data_ptr(), *(a.data_ptr() for a in t), n, 0)
+        eg2.ops.op(op, rec, heads * n, 64)
+        out.append(host(y).reshape(n, heads * d))
+    rows = np.r_[0:250, 271:n]
+    assert np.abs(out[0][rows] - out[1][rows]).max() <= 4e-5
+    assert not np.isfinite(out[1][250:271]).all(axis=1).any()
