@@ -605,8 +605,9 @@ hipError_t launch_residual_qkv(const float* x, const float* h, const float* post
                                const int8_t* wq, const float* wd, int ldw, float* x_out, float* out, int rows,
                                hipStream_t st) {
   if (rows <= 0 || !short_wave(rows) || x == x_out || ldw < kQKVCols) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(residual_qkv_kernel, dim3(kQKVCols / 32, rows / kShortTile), dim3(kShortThreads), 0, st, x, h, post_w, next_w, eps,
-                     wq, wd, ldw, x_out, out);
+  const int tile = short_tile(rows);
+  hipLaunchKernelGGL(tile == 4 ? residual_qkv_kernel<4> : residual_qkv_kernel<8>, dim3(kQKVCols / 32, rows / tile),
+                     dim3(kShortThreads), 0, st, x, h, post_w, next_w, eps, wq, wd, ldw, x_out, out);
   return hipGetLastError();
 }
 
@@ -614,8 +615,9 @@ hipError_t launch_residual_geglu(const float* x, const float* h, const float* po
                                  const int8_t* wq, const float* wd, int ldw, float* x_out, int8_t* gq, float* gd,
                                  int rows, hipStream_t st) {
   if (rows <= 0 || !short_wave(rows) || x == x_out || ldw < 2 * kFF) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(residual_geglu_kernel, dim3(kFF / kQK, rows / kShortTile), dim3(kShortThreads), 0, st, x, h, post_w,
-                     next_w, eps, wq, wd, ldw, x_out, gq, gd, rows);
+  const int tile = short_tile(rows);
+  hipLaunchKernelGGL(tile == 4 ? residual_geglu_kernel<4> : residual_geglu_kernel<8>, dim3(kFF / kQK, rows / tile),
+                     dim3(kShortThreads), 0, st, x, h, post_w, next_w, eps, wq, wd, ldw, x_out, gq, gd, rows);
   return hipGetLastError();
 }
 

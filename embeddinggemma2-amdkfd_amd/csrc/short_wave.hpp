@@ -13,7 +13,7 @@
 // takes attention from the raw projection to the quantized context with all
 // keys and values in LDS. The same operations in the same order as the
 // kernels they replace: the same bits. One query of 11
-// tokens through 24 layers: 1,119 -> 737 us.
+// tokens through 24 layers: 1,119 -> 696 us.
 #pragma once
 
 #include "eg2_device.hpp"
@@ -30,54 +30,57 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// A residual + projection workgroup: 12 waves, kShortTile rows. Thread (wave
-// w, lane) holds columns 256 (w % 3) + 4 lane .. + 3 of rows w / 3 and
-// w / 3 + 4, so a norm weight vector is read once per workgroup, not once per
-// row. What a CU has to read bounds the start of these kernels (64 B per
-// cycle: with 16 rows and a row per wave, 96 KB of rows and 96 KB of norm
-// weights took 5,700 cycles of 18,700), hence also 8 rows rather than 16 per
-// workgroup; the MFMA tile's other 8 rows repeat them and are not stored.
-constexpr int kShortTile = 8;
+// A residual + projection workgroup: 12 waves, ROWS (4 or 8) rows. Thread
+// (wave w, lane) holds columns 256 (w % 3) + 4 lane .. + 3 of row w / 3 (and
+// w / 3 + 4), so a norm weight vector is read once per workgroup, not once per
+// row. What a CU has to read and then computes on elementwise bounds these
+// kernels (with 16 rows and a row per wave, 96 KB of rows and 96 KB of norm
+// weights took 5,700 cycles of 18,700 at 64 B per cycle), hence few rows per
+// workgroup: 4 in a 16-row wave, 8 in a 32-row one, 160 and 144 workgroups
+// (one 11-token query with 8: 735 us, with 4: 696; 30 tokens with 8: 767, with
+// 4 for Q|K|V: 788); the MFMA tile's other rows repeat them and are not stored.
+inline int short_tile(int rows) { return rows <= 16 ? 4 : 8; }
 constexpr int kShortWaves = 12, kShortThreads = 64 * kShortWaves;
-constexpr int kShortStride = 8 * kTPitch + 4;  // staged squares per row: 8 rows read at once on distinct banks
+constexpr int kShortStride = 8 * kTPitch + 4;  // staged squares per row: the rows read at once on distinct banks
 
 // The LDS of such a workgroup: the rows' staged squares, then the terms of
 // TILES 16-column tiles, their 24 blocks split over 12 / TILES waves; the
-// quantized rows [block][2][8 rows][16] and their scales [block][8 rows].
-template <int TILES>
+// quantized rows [block][2][ROWS][16] and their scales [block][ROWS].
+template <int TILES, int ROWS>
 struct ShortLds {
   static constexpr int kSplit = kShortWaves / TILES, kPer = kBlocks / kSplit;
   static_assert(kSplit * kPer == kBlocks, "24 blocks split evenly");
   union alignas(16) {
-    float squares[kShortTile * kShortStride];
-    float4 terms[TILES][kBlocks * 32];  // lanes 0 .. 31: rows 0 .. 7
+    float squares[ROWS * kShortStride];
+    float4 terms[TILES][kBlocks * 4 * ROWS];  // lanes below 4 ROWS: the rows
   };
-  alignas(16) int8_t aq[kBlocks * 32 * kShortTile];
-  float dxs[kBlocks * kShortTile];
-  float inv[2][kShortTile];
+  alignas(16) int8_t aq[kBlocks * 32 * ROWS];
+  float dxs[kBlocks * ROWS];
+  float inv[2][ROWS];
 };
 
 // residual_norm_quant_kernel's work on the workgroup's rows, then the
 // projection onto weight columns 16 (TILES blockIdx.x + tile): x_out = x +
 // rms(h) * post_w (stored by the workgroups with blockIdx.x = 0), Q8_0 of
-// rms(x_out) * next_w, times W^T. Returns, for thread i < 128 TILES, output
-// i % 128 of tile i / 128 (row 4 (o / 64) + o % 4, column (o / 4) % 16).
-template <int TILES>
-__device__ __forceinline__ float residual_project(ShortLds<TILES>& lds, const float* __restrict__ x,
+// rms(x_out) * next_w, times W^T. Returns, for thread i < 16 ROWS TILES, output
+// o = i % (16 ROWS) of tile i / (16 ROWS) (row 4 (o / 64) + o % 4, column (o /
+// 4) % 16).
+template <int TILES, int ROWS>
+__device__ __forceinline__ float residual_project(ShortLds<TILES, ROWS>& lds, const float* __restrict__ x,
                                                   const float* __restrict__ h, const float* __restrict__ post_w,
                                                   const float* __restrict__ next_w, float eps,
                                                   const int8_t* __restrict__ wq, const float* __restrict__ wd, int ldw,
                                                   int m, float* __restrict__ x_out) {
-  constexpr int kPer = ShortLds<TILES>::kPer;
+  constexpr int kPer = ShortLds<TILES, ROWS>::kPer, kEach = ROWS / 4;  // rows per thread
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = w / 3, part = w % 3, e = 4 * (lane + 64 * part);
-  float4 hv[2], xv[2];
+  float4 hv[kEach], xv[kEach];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-    hv[i] = *reinterpret_cast<const float4*>(h + (size_t)(kShortTile * blockIdx.y + row + 4 * i) * kEmbd + e);
+  for (int i = 0; i < kEach; ++i)
+    hv[i] = *reinterpret_cast<const float4*>(h + (size_t)(ROWS * blockIdx.y + row + 4 * i) * kEmbd + e);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-    xv[i] = *reinterpret_cast<const float4*>(x + (size_t)(kShortTile * blockIdx.y + row + 4 * i) * kEmbd + e);
+  for (int i = 0; i < kEach; ++i)
+    xv[i] = *reinterpret_cast<const float4*>(x + (size_t)(ROWS * blockIdx.y + row + 4 * i) * kEmbd + e);
   const float4 pw = *reinterpret_cast<const float4*>(post_w + e), nw = *reinterpret_cast<const float4*>(next_w + e);
   // The weights of this wave's blocks, on their way during the rows' work.
   const int ti = w % TILES, ks = w / TILES;
@@ -88,35 +91,35 @@ __device__ __forceinline__ float residual_project(ShortLds<TILES>& lds, const fl
 
   // Squares of the thread's values into the transposed rows; wave 0 runs the
   // 64 chains of the 8 rows and leaves each row's inverse in inv.
-  auto inverses = [&](const float4 (&v)[2], float* inv) {
+  auto inverses = [&](const float4 (&v)[kEach], float* inv) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kEach; ++i) {
       TRow* tr = reinterpret_cast<TRow*>(lds.squares + (row + 4 * i) * kShortStride);
       const float c4[4] = {v[i].x * v[i].x, v[i].y * v[i].y, v[i].z * v[i].z, v[i].w * v[i].w};
 #pragma unroll
       for (int k = 0; k < 4; ++k) tr[(e + k) & 7][(e + k) >> 3] = c4[k];
     }
     __syncthreads();
-    if (w == 0) {
-      const TRow* rows = reinterpret_cast<const TRow*>(lds.squares + (lane >> 3) * kShortStride);
+    if (w == 0) {  // with 4 rows, every chain twice
+      const TRow* rows = reinterpret_cast<const TRow*>(lds.squares + (lane >> 3) % ROWS * kShortStride);
       const float r = rms_inverse(sse2_combine_dpp(squares_chain(rows, lane & 7)), kEmbd, eps);
-      if ((lane & 7) == 0) inv[lane >> 3] = r;
+      if ((lane & 7) == 0) inv[(lane >> 3) % ROWS] = r;
     }
     __syncthreads();
   };
   inverses(hv, lds.inv[0]);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {  // kernels.c:163-188
+  for (int i = 0; i < kEach; ++i) {  // kernels.c:163-188
     const float inv_h = lds.inv[0][row + 4 * i];
     const float a0 = hv[i].x * inv_h, a1 = hv[i].y * inv_h, a2 = hv[i].z * inv_h, a3 = hv[i].w * inv_h;
     const float b0 = a0 * pw.x, b1 = a1 * pw.y, b2 = a2 * pw.z, b3 = a3 * pw.w;
     xv[i] = make_float4(xv[i].x + b0, xv[i].y + b1, xv[i].z + b2, xv[i].w + b3);
     if (blockIdx.x == 0)
-      *reinterpret_cast<float4*>(x_out + (size_t)(kShortTile * blockIdx.y + row + 4 * i) * kEmbd + e) = xv[i];
+      *reinterpret_cast<float4*>(x_out + (size_t)(ROWS * blockIdx.y + row + 4 * i) * kEmbd + e) = xv[i];
   }
   inverses(xv, lds.inv[1]);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {  // kernels.c:139-151, the block over 8 lanes
+  for (int i = 0; i < kEach; ++i) {  // kernels.c:139-151, the block over 8 lanes
     const float inv = lds.inv[1][row + 4 * i];
     const float p0 = xv[i].x * nw.x, p1 = xv[i].y * nw.y, p2 = xv[i].z * nw.z, p3 = xv[i].w * nw.w;
     const float v0 = p0 * inv, v1 = p1 * inv, v2 = p2 * inv, v3 = p3 * inv;
@@ -124,30 +127,30 @@ __device__ __forceinline__ float residual_project(ShortLds<TILES>& lds, const fl
     const float d = div127(amax);
     const float id = amax != 0.0f ? 1.0f / d : 0.0f;
     const int kb = e / kQK, r = row + 4 * i;
-    *reinterpret_cast<uint32_t*>(lds.aq + ((kb * 2 + ((e >> 4) & 1)) * kShortTile + r) * 16 + (e & 15)) =
+    *reinterpret_cast<uint32_t*>(lds.aq + ((kb * 2 + ((e >> 4) & 1)) * ROWS + r) * 16 + (e & 15)) =
         pack_i8x4(q8_value(v0, id), q8_value(v1, id), q8_value(v2, id), q8_value(v3, id));
-    if ((lane & 7) == 0) lds.dxs[kb * kShortTile + r] = fp16_bits_to_fp32(fp32_to_fp16_bits(d));
+    if ((lane & 7) == 0) lds.dxs[kb * ROWS + r] = fp16_bits_to_fp32(fp32_to_fp16_bits(d));
   }
   __syncthreads();
-  // Lane 16 g + r: row r % 8, values 8 g .. 8 g + 7 of the block.
-  const int g = lane >> 4, aoff = ((g >> 1) * kShortTile + (lane & 7)) * 16 + (g & 1) * 8;
-  const int xoff = 4 * (g & 1) + (lane & 3);
+  // Lane 16 g + r: row r % ROWS, values 8 g .. 8 g + 7 of the block.
+  const int g = lane >> 4, aoff = ((g >> 1) * ROWS + (lane & (ROWS - 1))) * 16 + (g & 1) * 8;
+  const int xoff = (4 * g + (lane & 3)) & (ROWS - 1);
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int kb = ks * kPer + i;
-    f[i].a = *reinterpret_cast<const uint64_t*>(lds.aq + kb * 32 * kShortTile + aoff);
-    f[i].dx = lds.dxs[kb * kShortTile + xoff];
+    f[i].a = *reinterpret_cast<const uint64_t*>(lds.aq + kb * 32 * ROWS + aoff);
+    f[i].dx = lds.dxs[kb * ROWS + xoff];
     const float4 t = narrow_terms(f[i]);
-    if (lane < 32) lds.terms[ti][kb * 32 + lane] = t;
+    if (lane < 4 * ROWS) lds.terms[ti][kb * 4 * ROWS + lane] = t;
   }
   __syncthreads();
   const int i = (int)threadIdx.x;
   float sum = 0.0f;
-  if (i < 128 * TILES) {
-    const float* t = reinterpret_cast<const float*>(lds.terms[i >> 7]) + (i & 127);
+  if (i < 16 * ROWS * TILES) {
+    const float* t = reinterpret_cast<const float*>(lds.terms[i / (16 * ROWS)]) + i % (16 * ROWS);
     float v[kBlocks];
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b) v[b] = t[128 * b];
+    for (int b = 0; b < kBlocks; ++b) v[b] = t[16 * ROWS * b];
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) sum = sum + v[b];
   }
@@ -155,34 +158,36 @@ __device__ __forceinline__ float residual_project(ShortLds<TILES>& lds, const fl
 }
 
 // The raw Q|K|V rows (no QK-norm / RoPE) of x_out. Grid (kQKVCols / 32, rows /
-// kShortTile). x_out must not be x: every workgroup reads x.
+// ROWS). x_out must not be x: every workgroup reads x.
+template <int ROWS>
 __global__ void __launch_bounds__(kShortThreads)
 residual_qkv_kernel(const float* __restrict__ x, const float* __restrict__ h, const float* __restrict__ post_w,
                     const float* __restrict__ next_w, float eps, const int8_t* __restrict__ wq,
                     const float* __restrict__ wd, int ldw, float* __restrict__ x_out, float* __restrict__ out) {
-  __shared__ ShortLds<2> lds;
-  const float sum = residual_project<2>(lds, x, h, post_w, next_w, eps, wq, wd, ldw, kQKVCols, x_out);
-  const int i = (int)threadIdx.x, o = i & 127;
-  if (i < 256)
-    out[(size_t)(kShortTile * blockIdx.y + 4 * (o >> 6) + (o & 3)) * kQKVCols + 32 * blockIdx.x + 16 * (i >> 7) +
+  __shared__ ShortLds<2, ROWS> lds;
+  const float sum = residual_project<2, ROWS>(lds, x, h, post_w, next_w, eps, wq, wd, ldw, kQKVCols, x_out);
+  const int i = (int)threadIdx.x, o = i % (16 * ROWS);
+  if (i < 32 * ROWS)
+    out[(size_t)(ROWS * blockIdx.y + 4 * (o >> 6) + (o & 3)) * kQKVCols + 32 * blockIdx.x + 16 * (i / (16 * ROWS)) +
         ((o >> 2) & 15)] = sum;
 }
 
 // The same rows, then gate|up (interleaved 32-row groups), GeGLU and Q8_0
-// into gq / gd [kFF / 32][rows]. Grid (kFF / 32, rows / kShortTile).
+// into gq / gd [kFF / 32][rows]. Grid (kFF / 32, rows / ROWS).
+template <int ROWS>
 __global__ void __launch_bounds__(kShortThreads)
 residual_geglu_kernel(const float* __restrict__ x, const float* __restrict__ h, const float* __restrict__ post_w,
                       const float* __restrict__ next_w, float eps, const int8_t* __restrict__ wq,
                       const float* __restrict__ wd, int ldw, float* __restrict__ x_out, int8_t* __restrict__ gq,
                       float* __restrict__ gd, int rows) {
-  __shared__ ShortLds<4> lds;
-  __shared__ float gu[kShortTile * kGuPitch];
-  const float sum = residual_project<4>(lds, x, h, post_w, next_w, eps, wq, wd, ldw, 2 * kFF, x_out);
-  const int i = (int)threadIdx.x, o = i & 127;
-  if (i < 512) gu[(4 * (o >> 6) + (o & 3)) * kGuPitch + 16 * (i >> 7) + ((o >> 2) & 15)] = sum;
+  __shared__ ShortLds<4, ROWS> lds;
+  __shared__ float gu[ROWS * kGuPitch];
+  const float sum = residual_project<4, ROWS>(lds, x, h, post_w, next_w, eps, wq, wd, ldw, 2 * kFF, x_out);
+  const int i = (int)threadIdx.x, o = i % (16 * ROWS);
+  if (i < 64 * ROWS) gu[(4 * (o >> 6) + (o & 3)) * kGuPitch + 16 * (i / (16 * ROWS)) + ((o >> 2) & 15)] = sum;
   __syncthreads();
-  if (i < 32 * kShortTile)
-    narrow_geglu_store(gu, kShortTile * (int)blockIdx.y, (int)blockIdx.x, rows, kFF / kQK, gq, gd, rows);
+  if (i < 32 * ROWS)
+    narrow_geglu_store(gu, ROWS * (int)blockIdx.y, (int)blockIdx.x, rows, kFF / kQK, gq, gd, rows);
 }
 
 // ------------------------------------------------------------ attention
