@@ -216,6 +216,22 @@ struct Layer {
   int window;
 };
 
+// Where the parts of a wave's metadata lie, in 32-bit words, for `rows` padded
+// rows: the items, whose number depends on the packing, come last.
+struct MetaAt {
+  size_t count, ids, pos, off, tok, items;
+};
+inline MetaAt meta_at(size_t rows) {
+  MetaAt m;
+  m.count = 0;
+  m.ids = 64;
+  m.pos = m.ids + rows;
+  m.off = m.pos + rows;
+  m.tok = (m.off + rows + 1 + 63) / 64 * 64;
+  m.items = m.tok + 4 * rows;
+  return m;
+}
+
 // One wave in flight: a stream, the workspace of a 2048-token wave, pinned
 // staging, and the hipGraphs recorded on them. Several lanes share one
 // context's weights, so consecutive waves overlap on the device: one wave's
@@ -230,13 +246,13 @@ struct Lane {
   int8_t *xq, *cq, *mid_q;
   float* qkv;     // [rows][q0 q1 q2 | k | v] after QK-norm / RoPE
   float* scores;  // attention scratch: 1/sum per (token, head), then a score row per (token, head)
-  int32_t *ids_d, *pos_d;
-  // Attention plan: score and context work items, their two counts, one
-  // record per token.
-  uint32_t *items_d, *count_d, *tok_d, *off_d;
-  // Pinned staging.
-  int32_t *ids_h, *pos_h;
-  uint32_t *items_h, *count_h, *tok_h, *off_h;
+  // A wave's ids, positions, sequence offsets and attention plan (the two
+  // counts, one record per token, the score and context work items), in one
+  // buffer on the device and in pinned staging, so that a wave's upload is one
+  // copy: six copies of a few KB, each a kernel of its own on the device, stood
+  // before the first kernel of every wave. The parts' places depend on the
+  // padded row count alone (meta_at), as a graph's pointers must.
+  uint32_t *meta_d, *meta_h;
   float* out_h;
   std::map<unsigned, hipGraphExec_t> graphs;  // key: graph_key(padded rows, longest sequence)
   unsigned staged_tokens = 0, staged_rows = 0, staged_longest = 0;
@@ -542,22 +558,13 @@ void Backend::alloc_lane(Lane& L) {
   L.cd = dalloc<float>((size_t)kCap * (kEmbd / 32));
   L.qkv = dalloc<float>((size_t)kCap * kQKV);
   L.scores = dalloc<float>(attn_cap_.score_floats);
-  L.ids_d = dalloc<int32_t>(kCap);
-  L.pos_d = dalloc<int32_t>(kCap);
-  L.items_d = dalloc<uint32_t>(8 * attn_cap_.items);
-  L.count_d = dalloc<uint32_t>(2);
-  L.tok_d = dalloc<uint32_t>(4 * (size_t)kCap);
-  L.off_d = dalloc<uint32_t>(kCap + 1);
+  const size_t meta_words = meta_at(kCap).items + 8 * attn_cap_.items;
+  L.meta_d = dalloc<uint32_t>(meta_words);
   L.pooled = dalloc<float>((size_t)kCap * kEmbd);
   L.mid = dalloc<float>((size_t)kCap * kDenseFF);
   L.mid_q = dalloc<int8_t>(eg2_q8_tile_bytes(kCap, kDenseFF));
   L.mid_d = dalloc<float>((size_t)kCap * (kDenseFF / 32));
-  L.ids_h = halloc<int32_t>(kCap);
-  L.pos_h = halloc<int32_t>(kCap);
-  L.items_h = halloc<uint32_t>(8 * attn_cap_.items);
-  L.count_h = halloc<uint32_t>(2);
-  L.tok_h = halloc<uint32_t>(4 * (size_t)kCap);
-  L.off_h = halloc<uint32_t>(kCap + 1);
+  L.meta_h = halloc<uint32_t>(meta_words);
   L.out_h = halloc<float>((size_t)kCap * kEmbd);
 }
 
@@ -597,7 +604,11 @@ void Backend::gemm(Lane& ln, const char* name, const int8_t* xq, const float* xd
 void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
   hipStream_t s = ln.stream;
   const int n = (int)rows;
-  launch(ln, "embed", eg2::launch_embed_norm_quant(token_embd_, ln.ids_d, n, std::sqrt((float)kEmbd),
+  const MetaAt at = meta_at(rows);
+  const int32_t* ids = reinterpret_cast<const int32_t*>(ln.meta_d + at.ids);
+  const int32_t* pos = reinterpret_cast<const int32_t*>(ln.meta_d + at.pos);
+  const uint32_t *items = ln.meta_d + at.items, *count = ln.meta_d + at.count, *tok = ln.meta_d + at.tok;
+  launch(ln, "embed", eg2::launch_embed_norm_quant(token_embd_, ids, n, std::sqrt((float)kEmbd),
                                                    layers_[0].attn_norm, eps_, ln.x, ln.xq, ln.xd, s));
   if (eg2::short_wave(n)) {
     record_short_layers(ln, rows);
@@ -608,11 +619,11 @@ void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
     // Q|K|V projection with QK-norm / RoPE in its epilogue: the attention
     // operand rows, no unnormalised projection in HBM.
     launch(ln, "gemm_qkv_rope", eg2::launch_gemm_q8_qkv_rope(ln.xq, ln.xd, n, L.qkv.q, L.qkv.d, L.qkv.ld, n, kEmbd,
-                                                             L.q_norm, L.k_norm, L.rope, ln.pos_d, eps_, ln.qkv, s));
-    launch(ln, "attention_scores", eg2::launch_attention_scores(ln.qkv, ln.items_d, ln.count_d, eg2::kAttentionGrid,
+                                                             L.q_norm, L.k_norm, L.rope, pos, eps_, ln.qkv, s));
+    launch(ln, "attention_scores", eg2::launch_attention_scores(ln.qkv, items, count, eg2::kAttentionGrid,
                                                                 L.window, n, ln.scores, s));
-    launch(ln, "attention_softmax", eg2::launch_attention_softmax(ln.tok_d, L.window, n, (int)longest, ln.scores, s));
-    launch(ln, "attention_context", eg2::launch_attention_context(ln.qkv, ln.items_d, ln.count_d, eg2::kAttentionGrid,
+    launch(ln, "attention_softmax", eg2::launch_attention_softmax(tok, L.window, n, (int)longest, ln.scores, s));
+    launch(ln, "attention_context", eg2::launch_attention_context(ln.qkv, items, count, eg2::kAttentionGrid,
                                                                   L.window, n, ln.scores, ln.cq, ln.cd, s));
     gemm(ln, "gemm_o", ln.cq, ln.cd, L.o, ln.h, n, kEmbd, s);
     // The FFN input goes to the attention context's buffers (free after the
@@ -635,6 +646,9 @@ void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
 void Backend::record_short_layers(Lane& ln, unsigned rows) {
   hipStream_t s = ln.stream;
   const int n = (int)rows;
+  const MetaAt at = meta_at(rows);
+  const int32_t* pos = reinterpret_cast<const int32_t*>(ln.meta_d + at.pos);
+  const uint32_t* tok = ln.meta_d + at.tok;
   float *x = ln.x, *other = ln.x2;
   for (size_t il = 0; il < layers_.size(); ++il) {
     const Layer& L = layers_[il];
@@ -646,7 +660,7 @@ void Backend::record_short_layers(Lane& ln, unsigned rows) {
                                       other, ln.qkv, n, s));
       std::swap(x, other);
     }
-    launch(ln, "attention", eg2::launch_short_attention(ln.qkv, ln.tok_d, L.q_norm, L.k_norm, L.rope, ln.pos_d, eps_,
+    launch(ln, "attention", eg2::launch_short_attention(ln.qkv, tok, L.q_norm, L.k_norm, L.rope, pos, eps_,
                                                         L.window, n, ln.cq, ln.cd, s));
     gemm(ln, "gemm_o", ln.cq, ln.cd, L.o, ln.h, n, kEmbd, s);
     launch(ln, "residual_gemm_gate_up_geglu",
@@ -667,11 +681,12 @@ void Backend::record_head(Lane& ln, int B) {
   hipStream_t s = ln.stream;
   // A short wave leaves its rows in the second buffer (record_short_layers).
   const float* x = eg2::short_wave((int)ln.staged_rows) ? ln.x2 : ln.x;
+  const uint32_t* off = ln.meta_d + meta_at(ln.staged_rows).off;
   if (dense_) {
     // EXTRACTION.md:178-181: dense_2 then dense_3 on the mean pool
     // (kernels.c:417-425 without its L2), each input Q8_0-quantized,
     // then the L2 of kernels.c:393-396.
-    launch(ln, "pool", eg2::launch_pool_mean(x, ln.off_d, ln.pooled, B, s));
+    launch(ln, "pool", eg2::launch_pool_mean(x, off, ln.pooled, B, s));
     launch(ln, "dense_quant", eg2::launch_quantize_rows(ln.pooled, kEmbd, ln.cq, ln.cd, B, s));
     gemm(ln, "dense_2", ln.cq, ln.cd, dense2_, ln.mid, B, kDenseFF, s);
     launch(ln, "dense_quant", eg2::launch_quantize_rows(ln.mid, kDenseFF, ln.mid_q, ln.mid_d, B, s));
@@ -681,10 +696,10 @@ void Backend::record_head(Lane& ln, int B) {
     // One workgroup per sequence reads it through one CU; past 256
     // tokens the mean spreads over 12 workgroups per sequence and the
     // L2 follows (the same result, bit for bit).
-    launch(ln, "pool", eg2::launch_pool_mean(x, ln.off_d, ln.pooled, B, s));
+    launch(ln, "pool", eg2::launch_pool_mean(x, off, ln.pooled, B, s));
     launch(ln, "pool_l2", eg2::launch_l2_prefix(ln.pooled, kEmbd, kEmbd, B, s));
   } else {
-    launch(ln, "pool", eg2::launch_pool_l2(x, ln.off_d, ln.pooled, B, s));
+    launch(ln, "pool", eg2::launch_pool_l2(x, off, ln.pooled, B, s));
   }
 }
 
@@ -751,38 +766,33 @@ void Backend::stage(Lane& ln, const int32_t* ids, const size_t* offsets, size_t 
 
   // Metadata; rows [n, rows) form one dummy sequence that is never pooled.
   const unsigned rows = padded_rows(n);
+  const MetaAt at = meta_at(rows);
+  int32_t* ids_h = reinterpret_cast<int32_t*>(ln.meta_h + at.ids);
+  int32_t* pos_h = reinterpret_cast<int32_t*>(ln.meta_h + at.pos);
   for (size_t s = 0; s < batch; ++s)
     for (size_t t = offsets[s]; t < offsets[s + 1]; ++t) {
-      ln.ids_h[t] = ids[t];
-      ln.pos_h[t] = (int32_t)(t - offsets[s]);
+      ids_h[t] = ids[t];
+      pos_h[t] = (int32_t)(t - offsets[s]);
     }
   for (unsigned t = n; t < rows; ++t) {
-    ln.ids_h[t] = 0;
-    ln.pos_h[t] = (int32_t)(t - n);
+    ids_h[t] = 0;
+    pos_h[t] = (int32_t)(t - n);
   }
-  for (size_t s = 0; s <= batch; ++s) ln.off_h[s] = (uint32_t)offsets[s];
+  for (size_t s = 0; s <= batch; ++s) ln.meta_h[at.off + s] = (uint32_t)offsets[s];
   // The attention plan; the padding rows form one more sequence. Its counts
   // are checked against the allocation before anything is written.
   std::vector<size_t> all(offsets, offsets + batch + 1);
   if (rows > n) all.push_back(rows);
   eg2::AttentionCounts used{0, 0, 0};
-  if (!eg2::build_attention_plan(all.data(), all.size() - 1, attn_cap_, ln.items_h, ln.tok_h, &used))
+  if (!eg2::build_attention_plan(all.data(), all.size() - 1, attn_cap_, ln.meta_h + at.items, ln.meta_h + at.tok, &used))
     throw std::runtime_error("attention work list exceeds its capacity");
-  ln.count_h[0] = (uint32_t)used.score_items;
-  ln.count_h[1] = (uint32_t)(used.items - used.score_items);
+  ln.meta_h[at.count] = (uint32_t)used.score_items;
+  ln.meta_h[at.count + 1] = (uint32_t)(used.items - used.score_items);
 
   device_step([&] {
     hipStream_t s = ln.stream;
-    check(hipMemcpyAsync(ln.ids_d, ln.ids_h, rows * sizeof(int32_t), hipMemcpyHostToDevice, s), "copy ids");
-    check(hipMemcpyAsync(ln.pos_d, ln.pos_h, rows * sizeof(int32_t), hipMemcpyHostToDevice, s), "copy positions");
-    check(hipMemcpyAsync(ln.items_d, ln.items_h, 8 * used.items * sizeof(uint32_t), hipMemcpyHostToDevice, s),
-          "copy attention items");
-    check(hipMemcpyAsync(ln.count_d, ln.count_h, 2 * sizeof(uint32_t), hipMemcpyHostToDevice, s),
-          "copy attention counts");
-    check(hipMemcpyAsync(ln.tok_d, ln.tok_h, 4 * (size_t)rows * sizeof(uint32_t), hipMemcpyHostToDevice, s),
-          "copy token records");
-    check(hipMemcpyAsync(ln.off_d, ln.off_h, (batch + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, s),
-          "copy offsets");
+    check(hipMemcpyAsync(ln.meta_d, ln.meta_h, (at.items + 8 * used.items) * sizeof(uint32_t), hipMemcpyHostToDevice, s),
+          "copy wave metadata");
     const unsigned key = graph_key(rows, longest);
     if (use_graph_ && !profile_ && ln.graphs.find(key) == ln.graphs.end()) {
       hipGraph_t graph = nullptr;
