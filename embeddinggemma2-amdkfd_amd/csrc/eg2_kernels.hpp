@@ -104,7 +104,7 @@ hipError_t launch_attention_static(const float* qkv, const uint32_t* offsets, in
                                    int8_t* cq, float* cd, hipStream_t st);
 
 // The fused kernels of a short wave's layer (short_wave.hpp), for waves of
-// 16 or 32 rows (short_wave): the residual update and norms with the next
+// 16, 32 or 48 rows (short_wave): the residual update and norms with the next
 // projection, and attention from the raw Q|K|V rows. tok: the plan's token
 // records. x_out must not be x. Bit-identical to the separate kernels.
 bool short_wave(int rows);

@@ -12,8 +12,8 @@
 // 2048-token workspace.
 //
 // Batch (src/gemma2_kfd.cpp:268-353): validate, build per-token metadata
-// (sequence bounds, positions), pad the wave to a multiple of 32 rows (16 for up
-// to 16 tokens) with a dummy sequence, run the layer stack -- captured once per padded wave size
+// (sequence bounds, positions), pad the wave to a multiple of 32 rows (of 16 for
+// up to 48 tokens) with a dummy sequence, run the layer stack -- captured once per padded wave size
 // as a hipGraph -- then pooling, the optional dense head and L2, and copy the
 // [batch][768] embeddings back. Every call is serialised; a device failure
 // poisons the context (src/gemma2_kfd.cpp:190-191, 214-215, 270).
@@ -60,8 +60,9 @@ inline unsigned attention_form(unsigned longest) {
   return bound[softmax_form(longest)];
 }
 inline unsigned graph_key(unsigned rows, unsigned longest) { return 4 * rows + softmax_form(longest); }
-// Rows of a wave of n tokens: a multiple of 32, or 16 for up to 16 tokens.
-inline unsigned padded_rows(unsigned n) { return n <= 16 ? 16 : (n + 31) / 32 * 32; }
+// Rows of a wave of n tokens: a multiple of 16 for up to 48 tokens (the short
+// wave's kernels), else of 32.
+inline unsigned padded_rows(unsigned n) { return n <= 48 ? (n + 15) / 16 * 16 : (n + 31) / 32 * 32; }
 constexpr int kEmbd = 768, kFF = 1152, kHeadDim = 256, kQKV = 768 + 2 * 256, kDenseFF = 3072;
 constexpr int kVocab = 262144;
 constexpr double kTimeoutSeconds = 30.0;  // src/gemma2_kfd.cpp:21
@@ -242,7 +243,7 @@ struct Lane {
   hipStream_t stream = nullptr;
   std::mutex mutex;
   float *x, *h, *xd, *cd, *pooled, *mid, *mid_d;
-  float* x2;  // the residual stream's second buffer in a short wave (32 rows)
+  float* x2;  // the residual stream's second buffer in a short wave (48 rows)
   int8_t *xq, *cq, *mid_q;
   float* qkv;     // [rows][q0 q1 q2 | k | v] after QK-norm / RoPE
   float* scores;  // attention scratch: 1/sum per (token, head), then a score row per (token, head)
@@ -551,7 +552,7 @@ void Backend::alloc_lane(Lane& L) {
   check(hipExtStreamCreateWithCUMask(&L.stream, (uint32_t)mask.size(), mask.data()), "hipExtStreamCreateWithCUMask");
   L.x = dalloc<float>((size_t)kCap * kEmbd);
   L.h = dalloc<float>((size_t)kCap * kEmbd);
-  L.x2 = dalloc<float>(32 * (size_t)kEmbd);
+  L.x2 = dalloc<float>(48 * (size_t)kEmbd);
   L.xq = dalloc<int8_t>(eg2_q8_tile_bytes(kCap, kFF));
   L.xd = dalloc<float>((size_t)kCap * (kFF / 32));
   L.cq = dalloc<int8_t>(eg2_q8_tile_bytes(kCap, kEmbd));
@@ -639,7 +640,7 @@ void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
   launch(ln, "output_norm", eg2::launch_rms_norm_rows(ln.x, output_norm_, eps_, n, s));
 }
 
-// The layers of a short wave (eg2::short_wave: 16 or 32 rows) after the
+// The layers of a short wave (eg2::short_wave: 16 to 48 rows) after the
 // embedding, five kernels per layer: each residual update runs at the head
 // of the projection that consumes it, from one buffer of the residual stream
 // to the other, and attention is one kernel from the raw Q|K|V rows.

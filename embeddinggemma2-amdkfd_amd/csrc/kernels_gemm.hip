@@ -625,7 +625,11 @@ hipError_t launch_short_attention(const float* qkv, const uint32_t* tok, const f
                                   const float* rope, const int32_t* pos, float eps, int window, int rows, int8_t* cq,
                                   float* cd, hipStream_t st) {
   if (rows <= 0 || !short_wave(rows) || window < 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(short_attention_kernel, dim3(kHeads, rows / kShortQueries), dim3(1024), 0, st, qkv,
+  static_assert(kShortRows == 48, "one form per 16 rows");
+  auto* kernel = rows == 16   ? short_attention_kernel<1>
+                 : rows == 32 ? short_attention_kernel<2>
+                              : short_attention_kernel<3>;
+  hipLaunchKernelGGL(kernel, dim3(kHeads, rows / kShortQueries), dim3(1024), 0, st, qkv,
                      reinterpret_cast<const uint4*>(tok), q_w, k_w, rope, pos, eps, window, rows, cq, cd);
   return hipGetLastError();
 }

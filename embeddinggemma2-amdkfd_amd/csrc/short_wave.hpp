@@ -12,8 +12,12 @@
 // weights are on their way, and one workgroup per (head, few query rows)
 // takes attention from the raw projection to the quantized context with all
 // keys and values in LDS. The same operations in the same order as the
-// kernels they replace: the same bits. One query of 11
-// tokens through 24 layers: 1,119 -> 696 us.
+// kernels they replace: the same bits. Through 24
+// layers, host work included: 11 tokens 1,119 -> 650 us, 45 tokens 1,142 -> 787
+// (30 tokens: 745). At 64 rows the form ends: the residual kernels'
+// 320 and 288 workgroups are more than the 256 CUs, and raw rows, rotated keys and
+// values no longer fit one CU's LDS at once (with the values written over the raw
+// rows behind one more barrier: 1,120-1,140 us, the separate kernels 1,140-1,150).
 #pragma once
 
 #include "eg2_device.hpp"
@@ -36,7 +40,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // row. What a CU has to read and then computes on elementwise bounds these
 // kernels (with 16 rows and a row per wave, 96 KB of rows and 96 KB of norm
 // weights took 5,700 cycles of 18,700 at 64 B per cycle), hence few rows per
-// workgroup: 4 in a 16-row wave, 8 in a 32-row one, 160 and 144 workgroups
+// workgroup: 4 in a 16-row wave, 8 in a longer one, 144 to 240 workgroups
 // (one 11-token query with 8: 735 us, with 4: 696; 30 tokens with 8: 767, with
 // 4 for Q|K|V: 788); the MFMA tile's other rows repeat them and are not stored.
 inline int short_tile(int rows) { return rows <= 16 ? 4 : 8; }
@@ -195,72 +199,82 @@ residual_geglu_kernel(const float* __restrict__ x, const float* __restrict__ h, 
 // A workgroup of 16 waves takes one head and kShortQueries query rows of a
 // wave of at most kShortRows packed rows from the raw projection rows
 // [q0 q1 q2 | k | v] to the quantized context: all waves normalise and rotate
-// the k rows (two each), the first kShortQueries waves also a query row each,
+// the k rows (KG each), the first kShortQueries waves also a query row each,
 // which they then carry through. (With 16 query rows per workgroup the LDS
 // reads of 16 score and context waves on one CU bound the kernel.) Normalised and
 // rotated q and k rows are kept chain-major in LDS, [row][chain d % 4][step
 // d / 4], so that a lane of chain c reads four steps with one 16-byte read
 // (pitches of 68 and 272 floats: a 16-lane read group covers 4 rows x 4 chains
-// on distinct banks). Scores: lane 4 k + c runs chain c of keys k and k + 16
+// on distinct banks). Scores: lane 4 k + c runs chain c of keys k + 16 i
 // (kernels.c:289-294), the chains combined as (s0 + s2) + (s1 + s3); then the
 // row's maximum, expf, the sum in key order and the context in key order,
-// lanes over dimensions, over the row's own keys only.
-constexpr int kShortRows = 32;
+// lanes over dimensions, over the row's own keys only. One form per KG groups of
+// 16 rows: every row count known when compiled, no branch between the loads, and a
+// 16-row wave has 16 rows' LDS (one form with the second 16 rows behind
+// a branch: an 11-token query 677 us, now 650; 30 tokens 752 and 745).
+constexpr int kShortRows = 48;
 constexpr int kShortQueries = 4;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kShortPitch = kHeadDim + 8;  // floats per raw row
 constexpr int kChainPitch = kHeadDim / 4 + 4, kChainRow = 4 * kChainPitch;
 
+template <int KG>  // groups of 16 key rows
 struct ShortAttentionLds {
-  float raw[kShortQueries + kShortRows][kShortPitch];  // q rows, then k rows
+  alignas(16) float raw[kShortQueries + 16 * KG][kShortPitch];  // q rows, then k rows
   alignas(16) float q[kShortQueries][kChainRow];
-  alignas(16) float k[kShortRows][kChainRow];
-  alignas(16) float v[kShortRows][kHeadDim];
-  alignas(16) float p[kShortQueries][kShortRows];
+  alignas(16) float k[16 * KG][kChainRow];
+  alignas(16) float v[16 * KG][kHeadDim];
+  alignas(16) float p[kShortQueries][16 * KG];
   uint64_t exp_tab[32];
 };
 
+template <int KG>
 __global__ void __launch_bounds__(1024)
 short_attention_kernel(const float* __restrict__ qkv, const uint4* __restrict__ tok, const float* __restrict__ q_w,
                        const float* __restrict__ k_w, const float* __restrict__ rope, const int32_t* __restrict__ pos,
                        float eps, int window, int rows, int8_t* __restrict__ cq, float* __restrict__ cd) {
-  __shared__ ShortAttentionLds lds;
+  __shared__ ShortAttentionLds<KG> lds;
   constexpr int half = kHeadDim / 2;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hd = (int)blockIdx.x, qw = w % kShortQueries, t = kShortQueries * (int)blockIdx.y + qw;
-  const bool two = rows > 16;  // uniform: keys 16 .. 31 exist
-  // Rows of this wave: query row t, key rows w and w + 16.
   const bool query = w < kShortQueries;  // this wave carries query row t
-  // This wave's key rows, w and (two) w + 16.
-  const int tk0 = w, tk1 = two ? w + 16 : w;
-  const int pq = pos[t], p0 = pos[tk0], p1 = pos[tk1];
+  // This wave's key rows: w + 16 i.
+  int pk[KG];
+#pragma unroll
+  for (int i = 0; i < KG; ++i) pk[i] = pos[w + 16 * i];
+  const int pq = pos[t];
   const uint4 meta = tok[t];
-  const float* kr0 = qkv + (size_t)tk0 * kQKVCols + kHeads * kHeadDim + 4 * lane;
-  const float* kr1 = qkv + (size_t)tk1 * kQKVCols + kHeads * kHeadDim + 4 * lane;
+  const float* kr = qkv + (size_t)w * kQKVCols + kHeads * kHeadDim + 4 * lane;
   const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const float4 q4 = query ? *reinterpret_cast<const float4*>(qkv + (size_t)t * kQKVCols + hd * kHeadDim + 4 * lane) : zero;
-  const float4 k40 = *reinterpret_cast<const float4*>(kr0);
-  const float4 k41 = two ? *reinterpret_cast<const float4*>(kr1) : zero;
+  floatx4 k4[KG], v4[KG];  // no HIP vector structs: an array of those is kept in LDS
+#pragma unroll
+  for (int i = 0; i < KG; ++i) k4[i] = *reinterpret_cast<const floatx4*>(kr + (size_t)16 * i * kQKVCols);
   // A row's norm weights and cos/sin for dimensions lane + 64 j.
   struct Row4 {
     float v[4];
   };
   auto row4 = [&](const float* p) { return Row4{{p[lane], p[lane + 64], p[lane + 128], p[lane + 192]}}; };
   const Row4 kw = row4(k_w), qw4 = query ? row4(q_w) : kw;
-  const Row4 c0 = row4(rope + (size_t)p0 * kHeadDim), c1 = two ? row4(rope + (size_t)p1 * kHeadDim) : c0,
-             cq4 = query ? row4(rope + (size_t)pq * kHeadDim) : c0;
-  const float4 v40 = *reinterpret_cast<const float4*>(kr0 + kHeadDim);
-  const float4 v41 = two ? *reinterpret_cast<const float4*>(kr1 + kHeadDim) : zero;
+  Row4 kc[KG];
+#pragma unroll
+  for (int i = 0; i < KG; ++i) kc[i] = row4(rope + (size_t)pk[i] * kHeadDim);
+  const Row4 cq4 = query ? row4(rope + (size_t)pq * kHeadDim) : kc[0];
+#pragma unroll
+  for (int i = 0; i < KG; ++i) v4[i] = *reinterpret_cast<const floatx4*>(kr + (size_t)16 * i * kQKVCols + kHeadDim);
   if (threadIdx.x < 32) lds.exp_tab[threadIdx.x] = libm::kExp2Tab.t[threadIdx.x];
   float* rawq = lds.raw[qw];
-  float* rawk0 = lds.raw[kShortQueries + tk0];
-  float* rawk1 = lds.raw[kShortQueries + tk1];
+  auto rawk = [&](int i) { return lds.raw[kShortQueries + w + 16 * i]; };
   if (query) *reinterpret_cast<float4*>(rawq + 4 * lane) = q4;
-  *reinterpret_cast<float4*>(rawk0 + 4 * lane) = k40;
-  if (two) *reinterpret_cast<float4*>(rawk1 + 4 * lane) = k41;
+#pragma unroll
+  for (int i = 0; i < KG; ++i) *reinterpret_cast<floatx4*>(rawk(i) + 4 * lane) = k4[i];
   wave_lds_fence();
-  // kernels.c:233-264: lanes 0-7 run the chains of key row w, 8-15 of w + 16,
-  // 16-23 of the query row.
-  const float* chain_row = (lane >> 3) == 1 && two ? rawk1 : ((lane >> 3) == 2 && query ? rawq : rawk0);
+  // kernels.c:233-264: lanes 8 i .. 8 i + 7 run the chains of key row w + 16 i,
+  // the next eight those of the query row.
+  const float* chain_row = rawk(0);
+#pragma unroll
+  for (int i = 1; i < KG; ++i) chain_row = (lane >> 3) == i ? rawk(i) : chain_row;
+  if (query && (lane >> 3) == KG) chain_row = rawq;
   const float own = rms_inverse(sse2_combine_dpp(sse2_chain<kHeadDim>(chain_row, lane & 7)), kHeadDim, eps);
   auto norm_rope = [&](const float* raw, float* dst, const Row4& g, const Row4& cs, int from, bool q) {
     const float inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), from));
@@ -281,20 +295,19 @@ short_attention_kernel(const float* __restrict__ qkv, const uint4* __restrict__ 
       dst[(dd & 3) * kChainPitch + ((dd + half) >> 2)] = hi;
     }
   };
-  norm_rope(rawk0, lds.k[tk0], kw, c0, 0, false);
-  if (two) norm_rope(rawk1, lds.k[tk1], kw, c1, 8, false);
-  if (query) norm_rope(rawq, lds.q[qw], qw4, cq4, 16, true);
-  *reinterpret_cast<float4*>(lds.v[tk0] + 4 * lane) = v40;
-  if (two) *reinterpret_cast<float4*>(lds.v[tk1] + 4 * lane) = v41;
+#pragma unroll
+  for (int i = 0; i < KG; ++i) norm_rope(rawk(i), lds.k[w + 16 * i], kw, kc[i], 8 * i, false);
+  if (query) norm_rope(rawq, lds.q[qw], qw4, cq4, 8 * KG, true);
+#pragma unroll
+  for (int i = 0; i < KG; ++i) *reinterpret_cast<floatx4*>(lds.v[w + 16 * i] + 4 * lane) = v4[i];
   __syncthreads();
   if (!query) return;
   // Scores of row t.
   const int key = lane >> 2, c = lane & 3;
-  float s[2] = {0.0f, 0.0f};
+  float s[KG];
   const float4* qp = reinterpret_cast<const float4*>(lds.q[qw] + c * kChainPitch);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    if (i == 1 && !two) break;
+  for (int i = 0; i < KG; ++i) {
     const float4* kp = reinterpret_cast<const float4*>(lds.k[key + 16 * i] + c * kChainPitch);
     float a = 0.0f;
 #pragma unroll
@@ -311,23 +324,23 @@ short_attention_kernel(const float* __restrict__ qkv, const uint4* __restrict__ 
   }
   uint32_t first, last;
   key_range((uint32_t)t, meta.x, meta.y, window, first, last);
-  const bool in0 = (uint32_t)key >= first && (uint32_t)key < last;
-  const bool in1 = two && (uint32_t)key + 16 >= first && (uint32_t)key + 16 < last;
-  float m = fmaxf(in0 ? s[0] : -__builtin_inff(), in1 ? s[1] : -__builtin_inff());
+  auto in = [&](int i) { return (uint32_t)(key + 16 * i) >= first && (uint32_t)(key + 16 * i) < last; };
+  float m = -__builtin_inff();
+#pragma unroll
+  for (int i = 0; i < KG; ++i) m = fmaxf(m, in(i) ? s[i] : -__builtin_inff());
   m = fmaxf(m, dpp<0x141>(m));  // row_half_mirror: the other quad of each 8 lanes
   m = rows4_max(fmaxf(m, dpp<0x140>(m)));  // row_mirror, then the four rows
-  const float e0 = libm::expf_tab(s[0] - m, lds.exp_tab), e1 = libm::expf_tab(s[1] - m, lds.exp_tab);
-  if (c == 0) {
-    lds.p[qw][key] = in0 ? e0 : 0.0f;
-    lds.p[qw][key + 16] = in1 ? e1 : 0.0f;
+#pragma unroll
+  for (int i = 0; i < KG; ++i) {
+    const float e = libm::expf_tab(s[i] - m, lds.exp_tab);
+    if (c == 0) lds.p[qw][key + 16 * i] = in(i) ? e : 0.0f;
   }
   wave_lds_fence();
   // The sum in key order; +0 outside the row's keys changes no sum.
   float sum = 0.0f;
   const float4* pp = reinterpret_cast<const float4*>(lds.p[qw]);
 #pragma unroll
-  for (int i = 0; i < kShortRows / 4; ++i) {
-    if (4 * i >= rows) break;  // uniform
+  for (int i = 0; i < 4 * KG; ++i) {
     const float4 p4 = pp[i];
     sum = sum + p4.x;
     sum = sum + p4.y;

@@ -1,7 +1,7 @@
-"""Waves of up to 32 tokens take fused kernels of their own (short_wave.hpp:
+"""Waves of up to 48 tokens take fused kernels of their own (short_wave.hpp:
 the residual with the next projection, attention in one kernel, rows padded
-to 16 or 32); their embeddings against the oracle bit for bit at the edges:
-one token, a full 16- and 32-row wave and one past each, packings with and
+to a multiple of 16); their embeddings against the oracle bit for bit at the edges:
+one token, a full 16-, 32- and 48-row wave and one past each, packings with and
 without a padding sequence, sequences of one token, and a window that cuts
 into the sequences on two layers of three."""
 import numpy as np
@@ -12,7 +12,8 @@ import oracle_lib as OL
 
 pytestmark = pytest.mark.gpu
 
-LENS = [[1], [11], [16], [17], [31], [32], [33], [1] * 16, [1] * 17, [3, 9, 4], [20, 12], [5, 8, 2, 9, 1], [16, 1]]
+LENS = [[1], [11], [16], [17], [31], [32], [33], [1] * 16, [1] * 17, [3, 9, 4], [20, 12], [5, 8, 2, 9, 1], [16, 1],
+        [47], [48], [49], [33, 15], [30, 1, 10], [1] * 48, [7] * 6]
 
 
 @pytest.fixture(scope="module", params=[0, 8])
