@@ -37,6 +37,11 @@ hipError_t launch_gemm_q8(const int8_t* xq, const float* xd, int ldx, const int8
 hipError_t launch_gemm_q8_qkv_rope(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd,
                                    int ldw, int n, int k, const float* q_w, const float* k_w, const float* rope,
                                    const int32_t* pos, float eps, float* out, hipStream_t st);
+// The same result for a stream whose launches are recorded: two kernels where
+// those are faster than one (kernels_gemm.hip).
+hipError_t launch_qkv_rope_recorded(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd,
+                                    int ldw, int n, int k, const float* q_w, const float* k_w, const float* rope,
+                                    const int32_t* pos, float eps, float* out, hipStream_t st);
 hipError_t launch_gemm_q8_geglu(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd, int ldw,
                                 int8_t* gq, float* gd, int ldg, int n, int ff, int k, hipStream_t st);
 

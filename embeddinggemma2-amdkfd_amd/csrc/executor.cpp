@@ -619,8 +619,9 @@ void Backend::record_layers(Lane& ln, unsigned rows, unsigned longest) {
     const Layer& L = layers_[il];
     // Q|K|V projection with QK-norm / RoPE in its epilogue: the attention
     // operand rows, no unnormalised projection in HBM.
-    launch(ln, "gemm_qkv_rope", eg2::launch_gemm_q8_qkv_rope(ln.xq, ln.xd, n, L.qkv.q, L.qkv.d, L.qkv.ld, n, kEmbd,
-                                                             L.q_norm, L.k_norm, L.rope, pos, eps_, ln.qkv, s));
+    launch(ln, "gemm_qkv_rope",
+           eg2::launch_qkv_rope_recorded(ln.xq, ln.xd, n, L.qkv.q, L.qkv.d, L.qkv.ld, n, kEmbd, L.q_norm, L.k_norm,
+                                         L.rope, pos, eps_, ln.qkv, s));
     launch(ln, "attention_scores", eg2::launch_attention_scores(ln.qkv, items, count, eg2::kAttentionGrid,
                                                                 L.window, n, ln.scores, s));
     launch(ln, "attention_softmax", eg2::launch_attention_softmax(tok, L.window, n, (int)longest, ln.scores, s));

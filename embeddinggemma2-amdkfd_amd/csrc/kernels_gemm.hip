@@ -412,10 +412,13 @@ constexpr int kNarrowTiles = 1792;
 // gate|up + GeGLU: n 32 8.4 / 5.9, 96 8.7 / 6.1, 192 8.5 / 8.1, 256 8.7 / 10.6
 // (36 workgroups of 53 KB per 16 rows).
 constexpr int kNarrowGegluRows = 192;
-// Q|K|V: the fused kernel gives a head's 256 columns to one workgroup, so 32
-// rows run on 5 CUs; below this the narrow projection (80 workgroups per 16
-// rows) followed by the standalone QK-norm / RoPE in place is faster: n 1
-// 8.3 / 5.1, 64 9.1 / 6.2, 256 9.3 / 8.2, 352 9.3 / 9.7. Same bits.
+// Q|K|V in a recorded graph: the fused kernel gives a head's 256 columns to one
+// workgroup, so 32 rows run on 5 CUs; below this the narrow projection (80
+// workgroups per 16 rows) followed by the standalone QK-norm / RoPE in place is
+// faster on the device: n 1 8.3 / 5.1, 64 9.1 / 6.2, 256 9.3 / 8.2, 352 9.3 / 9.7.
+// Same bits. Launched one call at a time from the host it is not: the second
+// launch costs more than the kernels save (9.2 us fused, 11.3 in two), so the
+// operator keeps the one kernel at every size.
 constexpr int kNarrowQkvRows = 256;
 
 hipError_t launch_gemm_q8(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd, int ldw,
@@ -580,11 +583,6 @@ hipError_t launch_gemm_q8_qkv_rope(const int8_t* xq, const float* xd, int ldx, c
                                    const int32_t* pos, float eps, float* out, hipStream_t st) {
   if (n <= 0 || k <= 0 || k % kQK != 0 || ldx < n || ldw < kQKVCols) return hipErrorInvalidValue;
   if (!scales_fit(k, ldx) || !scales_fit(k, ldw)) return hipErrorInvalidValue;
-  if (n <= kNarrowQkvRows) {
-    const hipError_t e = launch_gemm_q8(xq, xd, ldx, wq, wd, ldw, out, n, kQKVCols, k, kQKVCols, st);
-    if (e != hipSuccess) return e;
-    return launch_qk_norm_rope(out, q_w, k_w, rope, pos, eps, out, n, st);
-  }
   const XcdRegions reg = xcd_split((n + 31) / 32, kQkvHeads);
   const dim3 grid(kXcds * reg.rows * reg.cols);
   const int nb = k / kQK;
@@ -596,6 +594,16 @@ hipError_t launch_gemm_q8_qkv_rope(const int8_t* xq, const float* xd, int ldx, c
     hipLaunchKernelGGL(gemm_q8_qkv_rope_kernel<true>, grid, dim3(512), lds, st, xq, xd, ldx, wq, wd, ldw, n, nb, q_w,
                        k_w, rope, pos, eps, out);
   return hipGetLastError();
+}
+
+hipError_t launch_qkv_rope_recorded(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd,
+                                    int ldw, int n, int k, const float* q_w, const float* k_w, const float* rope,
+                                    const int32_t* pos, float eps, float* out, hipStream_t st) {
+  if (n > kNarrowQkvRows || ldw < kQKVCols)
+    return launch_gemm_q8_qkv_rope(xq, xd, ldx, wq, wd, ldw, n, k, q_w, k_w, rope, pos, eps, out, st);
+  const hipError_t e = launch_gemm_q8(xq, xd, ldx, wq, wd, ldw, out, n, kQKVCols, k, kQKVCols, st);
+  if (e != hipSuccess) return e;
+  return launch_qk_norm_rope(out, q_w, k_w, rope, pos, eps, out, n, st);
 }
 
 // The short wave's fused kernels (short_wave.hpp).
