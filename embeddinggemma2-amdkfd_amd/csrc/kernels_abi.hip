@@ -657,9 +657,12 @@ __device__ __forceinline__ void attention_chunked(const EgAttention& p, unsigned
       }
       score = (s4[0] + s4[1]) + (s4[2] + s4[3]);
     }
-    const float next = fmaxf(run_max, dpp_wave_max(score));  // finite: the chunk has a key
-    const float alpha = eg2::libm::expf(run_max - next);     // 0 for the first chunk
-    const float pk = key < hi ? eg2::libm::expf(score - next) : 0.0f;
+    // A score of -inf (no key, an infinite element, a dot product past the
+    // range) weighs 0, also while no other has been met and the maximum itself
+    // is -inf; a row with no other score ends as 0/0.
+    const float next = fmaxf(run_max, dpp_wave_max(score));
+    const float alpha = run_max == -__builtin_inff() ? 0.0f : eg2::libm::expf(run_max - next);
+    const float pk = score == -__builtin_inff() ? 0.0f : eg2::libm::expf(score - next);
     den = den * alpha + dpp_wave_sum(pk);
     ps[lane] = pk;
     wave_lds_order();
@@ -859,8 +862,7 @@ attention_tile_kernel(EgAttention p) {
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const bool in = k0 + r >= lo[v] && k0 + r < hi[v];
-      const float pk = in ? exp_(score[v] - m[v]) : 0.0f;
+      const float pk = score[v] == -__builtin_inff() ? 0.0f : exp_(score[v] - m[v]);
       l[v] = l[v] + row16_sum(pk);
       lds.p[w][4 * g + v][r] = pk;
     }

@@ -82,3 +82,59 @@ def test_non_finite_values_stay_in_their_sequence(eg2, gpu, op):
     rows = np.r_[0:250, 271:n]
     assert np.abs(out[0][rows] - out[1][rows]).max() <= 4e-5
     assert not np.isfinite(out[1][250:271]).all(axis=1).any()
+
+
+def softmax_reference(q, k, v, bounds, n, heads, d, kvs, group, window):
+    """float64 attention where a score of -inf weighs nothing, and a NaN or
+    +inf score, or no score above -inf, makes the row NaN."""
+    out = np.zeros((n, heads, d))
+    q, k, v = q.reshape(n, heads, d).astype(np.float64), k.reshape(n, kvs), v.reshape(n, kvs).astype(np.float64)
+    for t in range(n):
+        lo, hi = int(bounds[t, 0]), int(bounds[t, 1])
+        if window:
+            lo, hi = max(lo, t - window), min(hi, t + window + 1)
+        for h in range(heads):
+            cols = slice(h // group * d, (h // group + 1) * d)
+            with np.errstate(all="ignore"):
+                s = (k[lo:hi, cols].astype(np.float64) * q[t, h]).sum(1)
+                s[s < -3.5e38] = -np.inf  # past the range of 32 bits
+                w = np.exp(s - s.max())
+                out[t, h] = (w / w.sum()) @ v[lo:hi, cols]
+    return out
+
+
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("n", [511, 512, 640])
+@pytest.mark.parametrize("window", [0, 20])
+def test_scores_of_minus_infinity_weigh_nothing(eg2, gpu, op, n, window):
+    """Keys whose score is -inf, by an infinite element or by a dot product
+    past the range of 32 bits: alone in a 16-key block of their text (its 17th
+    and 33rd key), as a text's only key, and 70 in a row at a text's start, so
+    that whole blocks and chunks of a row score -inf before a finite one; and
+    keys that score +inf or NaN, which make their text's rows NaN."""
+    import torch
+
+    heads, d, kvs, group = OPS[op]
+    lens = [17, 33, 60, 1, n - 111]
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    bounds = np.array([(starts[s], starts[s + 1]) for s in range(len(lens)) for _ in range(lens[s])], np.uint32)
+    rng = np.random.default_rng(n + d + window)
+    q = (rng.standard_normal((n, heads, d)) / np.sqrt(d)).astype(np.float32)
+    q[:, :, 3] = 2.0
+    k, v = (rng.standard_normal((n, kvs)).astype(np.float32) for _ in range(2))
+    k[16, 3::d] = -np.inf
+    k[49, 3::d] = -3e38
+    k[80, 3::d] = np.inf
+    k[110, 3::d] = -np.inf
+    k[111:181, 3::d] = -np.inf
+    if window:
+        k[300, 3::d] = np.nan
+    y = torch.full((n * heads * d,), 7.0, device=gpu)
+    t = [dev(a, gpu) for a in (q, k, v, bounds.reshape(-1).view(np.int32))]
+    rec = eg2.EgAttention(y.data_ptr(), *(a.data_ptr() for a in t), n, window)
+    eg2.ops.op(op, rec, heads * n, 64)
+    got = host(y).reshape(n, heads, d)
+    want = softmax_reference(q, k, v, bounds, n, heads, d, kvs, group, window)
+    assert np.isnan(want[110]).all() and np.isfinite(want[:50]).all() and np.isfinite(want[400:]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.nanmax(np.abs(got - want)) <= 2e-5
