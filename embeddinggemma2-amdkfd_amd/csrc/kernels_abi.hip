@@ -342,11 +342,19 @@ struct StepWeights<0, BLOCKS> {
 template <int RB, int CB>
 constexpr int kStepLds = 16 * (RB + CB) * kStepPitch;
 
+// Accumulators per row block: one per column block; with F32 weights and one
+// 16 x 16 tile four, a quarter of the products each, added at the end. The
+// general form splits every step over the tile's four waves, so one chain per
+// wave would be up to four times as long as its chains (one step: 1.5 times
+// their rms error); four are as short at one step and shorter at more.
+template <unsigned TYPE, int RB, int CB>
+constexpr int kAcc = TYPE == 0 && RB * CB == 1 ? 4 : CB;
+
 // acc[i][j] += rows 16 i .. of the step's activations times columns 16 j .. of
 // its weights, from the wave's LDS area. The products run part by part over
 // several tiles, so that an MFMA does not wait for the one before it.
 template <unsigned TYPE, int RB, int CB>
-__device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx4 (&acc)[RB][CB]) {
+__device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx4 (&acc)[RB][kAcc<TYPE, RB, CB>]) {
   if constexpr (TYPE == 0) {
     float a[RB][8], b[CB][8];
 #pragma unroll
@@ -358,8 +366,10 @@ __device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx
 #pragma unroll
       for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int j = 0; j < CB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < CB; ++j) {
+          floatx4& sum = acc[i][kAcc<TYPE, RB, CB> == CB ? j : e % 4];
+          sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], sum, 0, 0, 0);
+        }
   } else {
     Bf16Parts a[RB];
 #pragma unroll
@@ -401,7 +411,7 @@ __device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx
         constexpr int kParts = TYPE == 1 ? 2 : 1;
         uintx4 b[2] = {raw, raw};
         if constexpr (TYPE == 1) {
-                    float f[8];
+          float f[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) f[e] = eg2::fp16_bits_to_fp32((raw[e / 2] >> (16 * (e & 1))) & 0xffffu);
           const Bf16Parts s = split_bf16<2>(f);
@@ -424,7 +434,7 @@ __device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx
 // repeat the last one.
 template <unsigned TYPE, int RB, int CB, int DEPTH>
 __device__ __forceinline__ void mm_direct(const EgMM& p, unsigned row0, unsigned col0, unsigned first, unsigned stride,
-                                          float* lds, floatx4 (&acc)[RB][CB]) {
+                                          float* lds, floatx4 (&acc)[RB][kAcc<TYPE, RB, CB>]) {
   const unsigned steps = p.k / 32;
   float *xs = lds, *ws = lds + 16 * RB * kStepPitch;
   StepRows<RB> x[DEPTH];
@@ -470,12 +480,14 @@ __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStep
   constexpr int RB = TH / 16, CB = TW / 16, kDepth = TH == 64 ? 1 : 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
   const unsigned row0 = blockIdx.y * TH, col0 = blockIdx.x * TW;
-  floatx4 acc[RB][CB];
+  constexpr int kA = kAcc<TYPE, RB, CB>;
+  floatx4 acc[RB][kA];
 #pragma unroll
   for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int j = 0; j < CB; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < kA; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, wave, 4, step[wave], acc);
+  if constexpr (kA > CB) acc[0][0] = (acc[0][0] + acc[0][1]) + (acc[0][2] + acc[0][3]);
   bool finite = true;
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
