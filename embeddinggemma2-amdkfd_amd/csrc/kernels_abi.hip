@@ -88,12 +88,14 @@ __device__ __forceinline__ float weight_at(const void* w, size_t i, unsigned typ
 constexpr int kSlice = 32;           // K values per LDS stage
 constexpr int kPitch = kSlice + 4;   // floats per staged row
 
-// The general form: any k, any alignment, and the tiles whose sums overflow or
-// hold infinities or NaN (mm_tile). out[n x m] = x[n x k] . W[m x k]^T for a
+// The general form: any k, any alignment, and the sums that overflow or hold
+// infinities or NaN (mm_tile). out[n x m] = x[n x k] . W[m x k]^T for a
 // TH x TW tile per 256-thread workgroup (4 waves), fp32 MFMA on LDS-staged
-// slices of the activations and the decoded weights.
+// slices of the activations and the decoded weights. With `redo` (a bit per
+// output, [row][column / 16]) only those outputs are stored.
 template <int TH, int TW>
-__device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, floatx4* part) {
+__device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, floatx4* part,
+                                           const uint16_t (*redo)[TW / 16]) {
   static_assert((TH == 16 && (TW == 16 || TW == 64)) || (TH == 64 && TW == 64), "tile shapes of the contract");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r16 = lane & 15;
@@ -159,8 +161,10 @@ __device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, 
     for (int j = 0; j < CB; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const unsigned row = row0 + rbase + 16 * i + 4 * g + v, col = col0 + cbase + 16 * j + r16;
-        if (row < p.n && col < p.m) p.out[(size_t)row * p.m + col] = acc[i][j][v];
+        const int tr = rbase + 16 * i + 4 * g + v, tc = cbase / 16 + j;
+        const unsigned row = row0 + tr, col = col0 + 16 * tc + r16;
+        if (row < p.n && col < p.m && (!redo || (redo[tr][tc] >> r16) & 1))
+          p.out[(size_t)row * p.m + col] = acc[i][j][v];
       }
 }
 
@@ -465,18 +469,20 @@ __device__ __forceinline__ bool mm_direct_fits(const EgMM& p) {
   return p.k % 32 == 0 && p.k > 0 && x % 16 == 0 && (p.type == 8 ? w % 2 == 0 : w % 16 == 0);
 }
 
+__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.40282347e38f; }
+
 // A TH x TW tile per workgroup: each of the 4 waves takes the whole tile over
 // every fourth step (so an activation is loaded and split once per workgroup,
 // and a 512-deep product is 4 steps, not 16, of a wave's serial chain), and
 // the four partial tiles are added through LDS, wave w finishing column block
-// w. Where a sum comes out infinite or NaN -- non-finite operands, or a Q8_0
-// dot that overflows before its scale -- the tile is computed again in the
-// general form, which multiplies decoded weights.
-// Returns whether this thread's sums are finite; stores nothing unless every
-// thread's are.
+// w. A sum that comes out infinite or NaN -- non-finite operands, or a Q8_0
+// dot that overflows before its scale -- is not stored but noted in `redo`,
+// for the general form, which multiplies decoded weights: an output's bits
+// follow from its own row and column alone. Returns whether every output of the
+// tile is stored.
 template <unsigned TYPE, int TH, int TW>
 __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStepLds<TH / 16, TW / 16>],
-                                              floatx4 (*part)[TW / 16][64]) {
+                                              floatx4 (*part)[TW / 16][64], uint16_t (*redo)[TW / 16]) {
   constexpr int RB = TH / 16, CB = TW / 16, kDepth = TH == 64 ? 1 : 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
   const unsigned row0 = blockIdx.y * TH, col0 = blockIdx.x * TW;
@@ -488,7 +494,7 @@ __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStep
     for (int j = 0; j < kA; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, wave, 4, step[wave], acc);
   if constexpr (kA > CB) acc[0][0] = (acc[0][0] + acc[0][1]) + (acc[0][2] + acc[0][3]);
-  bool finite = true;
+  bool good = true;
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     __syncthreads();  // the waves' step areas, then the previous row block's parts, are no longer read
@@ -498,20 +504,34 @@ __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStep
     if (wave < CB) {
       acc[i][0] = ((part[0][wave][lane] + part[1][wave][lane]) + part[2][wave][lane]) + part[3][wave][lane];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) finite = finite && fabsf(acc[i][0][v]) <= 3.40282347e38f;
+      for (int v = 0; v < 4; ++v) good = good && is_finite(acc[i][0][v]);
     }
   }
-  if (__syncthreads_or(!finite)) return false;
-  if (wave >= CB) return true;
-  const unsigned col = col0 + 16 * wave + r;
+  const bool done = !__syncthreads_or(!good);
+  // Stores the outputs that `bad` does not hold for.
+  auto store = [&](auto bad) {
+    if (wave >= CB) return;
+    const unsigned col = col0 + 16 * wave + r;
 #pragma unroll
-  for (int i = 0; i < RB; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const unsigned row = row0 + 16 * i + 4 * g + v;
-      if (row < p.n && col < p.m) p.out[(size_t)row * p.m + col] = acc[i][0][v];
-    }
-  return true;
+      for (int v = 0; v < 4; ++v) {
+        const unsigned row = row0 + 16 * i + 4 * g + v;
+        if (!bad(i, v) && row < p.n && col < p.m) p.out[(size_t)row * p.m + col] = acc[i][0][v];
+      }
+  };
+  if (done) {
+    store([](int, int) { return false; });
+  } else {
+    store([&](int i, int v) {
+      const bool bad = !is_finite(acc[i][0][v]);
+      const uint64_t b = __ballot(bad);  // lanes 16 g ..: row 4 g + v
+      if (r == 0) redo[16 * i + 4 * g + v][wave] = (uint16_t)(b >> (16 * g));
+      return bad;
+    });
+    __syncthreads();
+  }
+  return done;
 }
 
 template <int TH, int TW>
@@ -524,17 +544,19 @@ __device__ __forceinline__ void mm_tile(const EgMM& p) {
       alignas(16) float xs[TH * kPitch], ws[TW * kPitch];
     } general;
   } lds;
+  __shared__ uint16_t redo[TH][TW / 16];
   if (blockIdx.y * TH >= p.n || blockIdx.x * TW >= p.m) return;
+  const bool direct = mm_direct_fits(p);
   bool done = false;  // uniform
-  if (mm_direct_fits(p)) {
+  if (direct) {
     switch (p.type) {
-      case 0: done = mm_tile_typed<0, TH, TW>(p, lds.step, lds.part); break;
-      case 1: done = mm_tile_typed<1, TH, TW>(p, lds.step, lds.part); break;
-      case 30: done = mm_tile_typed<30, TH, TW>(p, lds.step, lds.part); break;
-      default: done = mm_tile_typed<8, TH, TW>(p, lds.step, lds.part); break;
+      case 0: done = mm_tile_typed<0, TH, TW>(p, lds.step, lds.part, redo); break;
+      case 1: done = mm_tile_typed<1, TH, TW>(p, lds.step, lds.part, redo); break;
+      case 30: done = mm_tile_typed<30, TH, TW>(p, lds.step, lds.part, redo); break;
+      default: done = mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, redo); break;
     }
   }
-  if (!done) mm_general<TH, TW>(p, lds.general.xs, lds.general.ws, lds.general.part);
+  if (!done) mm_general<TH, TW>(p, lds.general.xs, lds.general.ws, lds.general.part, direct ? redo : nullptr);
 }
 
 // -------------------------------------------------------------- row sums

@@ -85,3 +85,47 @@ def test_few_steps_keep_the_general_form_s_precision(eg2, gpu, wtype, k):
     rms = lambda y: np.sqrt(((y - want) ** 2).mean())
     got, general = (run(eg2, gpu, MM_VARIANTS[0], x, raw, wtype, m, x_shift=s) for s in (0, 1))
     assert rms(got) <= 1.01 * rms(general)
+
+
+@pytest.mark.parametrize("variant", MM_VARIANTS[:3], ids=[v[0] for v in MM_VARIANTS[:3]])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_rows_do_not_depend_on_their_neighbours(eg2, gpu, variant, wtype):
+    """NaN, infinite, overflowing and tiny rows: the others keep their bits."""
+    n, k, m = 70, 128, 70
+    rng = np.random.default_rng(wtype)
+    raw, _ = encode_weights((rng.standard_normal((m, k)) * 0.05).astype(np.float32), wtype)
+    x = rng.standard_normal((n, k)).astype(np.float32)
+    clean = run(eg2, gpu, variant, x, raw, wtype, m)
+    bad = x.copy()
+    bad[3, 5], bad[20, 31], bad[41, 100] = np.nan, -np.inf, 3e38
+    bad[64] *= np.float32(2.0 ** -118)
+    got = run(eg2, gpu, variant, bad, raw, wtype, m)
+    rest = np.setdiff1d(np.arange(n), [3, 20, 41, 64])
+    assert np.array_equal(got[rest].view(np.uint32), clean[rest].view(np.uint32))
+
+
+@pytest.mark.parametrize("variant", MM_VARIANTS[:3], ids=[v[0] for v in MM_VARIANTS[:3]])
+@pytest.mark.parametrize("wtype", TYPES)
+def test_non_finite_weights_take_the_general_form(eg2, gpu, variant, wtype):
+    """An infinity or a NaN among the weights (of Q8_0: a block's scale): its
+    column is the general form's, bit for bit, and no other column changes."""
+    n, k, m = 70, 128, 70
+    rng = np.random.default_rng(wtype)
+    w = (rng.standard_normal((m, k)) * 0.05).astype(np.float32)
+    x = rng.standard_normal((n, k)).astype(np.float32)
+    x[9] = 0.0
+    raw, _ = encode_weights(w, wtype)
+    clean = run(eg2, gpu, variant, x, raw, wtype, m)
+    codes = {0: (0x7F800000, 0xFF800000, 0x7FC00000), 30: (0x7F80, 0xFF80, 0x7FC0)}.get(wtype, (0x7C00, 0xFC00, 0x7E00))
+    for code in codes:
+        bad = raw.reshape(-1).view(np.uint8).copy()
+        if wtype == 8:
+            bad.reshape(m, k // 32, 34)[17, 2, :2].view(np.uint16)[0] = code
+        else:
+            bad.view(np.uint32 if wtype == 0 else np.uint16).reshape(m, k)[17, 70] = code
+        got = run(eg2, gpu, variant, x, bad, wtype, m)
+        general = run(eg2, gpu, variant, x, bad, wtype, m, x_shift=1)
+        assert not np.isfinite(general[:, 17]).any()
+        assert np.array_equal(got[:, 17], general[:, 17], equal_nan=True)
+        other = np.arange(m) != 17
+        assert np.array_equal(got[:, other], clean[:, other])
