@@ -171,7 +171,7 @@ __device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, 
 // The usual form, k a multiple of 32 and operands aligned (mm_direct_fits),
 // on bf16 MFMA (v_mfma_f32_16x16x32_bf16) with fp32 sums. The activations are
 // split exactly into three bf16 parts (8 + 8 + 8 of their 24 significant
-// bits, by truncation); Q8_0 values are whole numbers of at most 8 bits and
+// bits, by truncation; a row too small for that takes the general form); Q8_0 values are whole numbers of at most 8 bits and
 // BF16 weights are bf16, so three products per weight are exact, and a Q8_0
 // block's scale is one fma on its 32-value dot; F16 weights split exactly into
 // two parts (six products); F32 weights stay on fp32 MFMA
@@ -215,6 +215,12 @@ __device__ __forceinline__ Bf16Parts split_bf16(const float (&v)[8]) {
   }
   return s;
 }
+// bf16 holds whole steps of 2^-133, so a value below 2^-110 loses bits of its
+// last part, at most 2^-133 in all: nothing beside a value of 2^-100 or more,
+// but all of the precision in a row that has none. (One maximum per two values
+// in the loop; noting the lost bits themselves costs as many instructions, but
+// F16 weights lost 10% by the registers' lifetimes.)
+constexpr float kSplitsFrom = 0x1p-100f;
 __device__ __forceinline__ floatx4 mfma_bf16(uintx4 a, uintx4 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
                                                  0);
@@ -356,9 +362,12 @@ constexpr int kAcc = TYPE == 0 && RB * CB == 1 ? 4 : CB;
 
 // acc[i][j] += rows 16 i .. of the step's activations times columns 16 j .. of
 // its weights, from the wave's LDS area. The products run part by part over
-// several tiles, so that an MFMA does not wait for the one before it.
+// several tiles, so that an MFMA does not wait for the one before it. Where
+// activations are split, largest[i] takes up the magnitudes of this lane's
+// values of row 16 i + lane % 16 (kSplitsFrom).
 template <unsigned TYPE, int RB, int CB>
-__device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx4 (&acc)[RB][kAcc<TYPE, RB, CB>]) {
+__device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx4 (&acc)[RB][kAcc<TYPE, RB, CB>],
+                                        float (&largest)[RB]) {
   if constexpr (TYPE == 0) {
     float a[RB][8], b[CB][8];
 #pragma unroll
@@ -381,6 +390,8 @@ __device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx
       float f[8];
       step_row(xs, i, f);
       a[i] = split_bf16<3>(f);
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) largest[i] = fmaxf(fmaxf(fabsf(f[e]), fabsf(f[e + 1])), largest[i]);
     }
     if constexpr (TYPE == 8) {
       constexpr int JB = RB == 1 ? CB : 1;  // column blocks at a time: RB JB = 4 independent dots
@@ -438,7 +449,8 @@ __device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx
 // repeat the last one.
 template <unsigned TYPE, int RB, int CB, int DEPTH>
 __device__ __forceinline__ void mm_direct(const EgMM& p, unsigned row0, unsigned col0, unsigned first, unsigned stride,
-                                          float* lds, floatx4 (&acc)[RB][kAcc<TYPE, RB, CB>]) {
+                                          float* lds, floatx4 (&acc)[RB][kAcc<TYPE, RB, CB>],
+                                          float (&largest)[RB]) {
   const unsigned steps = p.k / 32;
   float *xs = lds, *ws = lds + 16 * RB * kStepPitch;
   StepRows<RB> x[DEPTH];
@@ -459,7 +471,7 @@ __device__ __forceinline__ void mm_direct(const EgMM& p, unsigned row0, unsigned
       x[s].put(xs);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       load(s, step + (s + DEPTH) * stride);
-      mm_step<TYPE, RB, CB>(xs, ws, acc);
+      mm_step<TYPE, RB, CB>(xs, ws, acc, largest);
     }
   }
 }
@@ -476,13 +488,15 @@ __device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823
 // and a 512-deep product is 4 steps, not 16, of a wave's serial chain), and
 // the four partial tiles are added through LDS, wave w finishing column block
 // w. A sum that comes out infinite or NaN -- non-finite operands, or a Q8_0
-// dot that overflows before its scale -- is not stored but noted in `redo`,
-// for the general form, which multiplies decoded weights: an output's bits
-// follow from its own row and column alone. Returns whether every output of the
-// tile is stored.
+// dot that overflows before its scale -- and the sums of a row too small to
+// split (a lane's share of it: all zero or below kSplitsFrom, not all zero) are
+// not stored but noted in `redo`, for the general form, which multiplies
+// decoded weights by whole activations: an output's bits follow from its own row
+// and column alone. Returns whether every output of the tile is stored.
 template <unsigned TYPE, int TH, int TW>
 __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStepLds<TH / 16, TW / 16>],
-                                              floatx4 (*part)[TW / 16][64], uint16_t (*redo)[TW / 16]) {
+                                              floatx4 (*part)[TW / 16][64], uint16_t (*small)[TH / 16],
+                                              uint16_t (*redo)[TW / 16]) {
   constexpr int RB = TH / 16, CB = TW / 16, kDepth = TH == 64 ? 1 : 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
   const unsigned row0 = blockIdx.y * TH, col0 = blockIdx.x * TW;
@@ -492,9 +506,13 @@ __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStep
   for (int i = 0; i < RB; ++i)
 #pragma unroll
     for (int j = 0; j < kA; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, wave, 4, step[wave], acc);
+  float largest[RB] = {};
+  mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, wave, 4, step[wave], acc, largest);
   if constexpr (kA > CB) acc[0][0] = (acc[0][0] + acc[0][1]) + (acc[0][2] + acc[0][3]);
+  auto too_small = [&](int i) { return TYPE != 0 && largest[i] > 0.0f && largest[i] < kSplitsFrom; };
   bool good = true;
+#pragma unroll
+  for (int i = 0; i < RB; ++i) good = good && !too_small(i);
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     __syncthreads();  // the waves' step areas, then the previous row block's parts, are no longer read
@@ -523,8 +541,15 @@ __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStep
   if (done) {
     store([](int, int) { return false; });
   } else {
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const uint64_t b = __ballot(too_small(i));  // lanes r, 16 + r, ..: row 16 i + r
+      if (lane == 0) small[wave][i] = (uint16_t)(b | b >> 16 | b >> 32 | b >> 48);
+    }
+    __syncthreads();
     store([&](int i, int v) {
-      const bool bad = !is_finite(acc[i][0][v]);
+      const uint32_t rows = small[0][i] | small[1][i] | small[2][i] | small[3][i];
+      const bool bad = (rows >> (4 * g + v)) & 1 || !is_finite(acc[i][0][v]);
       const uint64_t b = __ballot(bad);  // lanes 16 g ..: row 4 g + v
       if (r == 0) redo[16 * i + 4 * g + v][wave] = (uint16_t)(b >> (16 * g));
       return bad;
@@ -544,16 +569,16 @@ __device__ __forceinline__ void mm_tile(const EgMM& p) {
       alignas(16) float xs[TH * kPitch], ws[TW * kPitch];
     } general;
   } lds;
-  __shared__ uint16_t redo[TH][TW / 16];
+  __shared__ uint16_t small[4][TH / 16], redo[TH][TW / 16];
   if (blockIdx.y * TH >= p.n || blockIdx.x * TW >= p.m) return;
   const bool direct = mm_direct_fits(p);
   bool done = false;  // uniform
   if (direct) {
     switch (p.type) {
-      case 0: done = mm_tile_typed<0, TH, TW>(p, lds.step, lds.part, redo); break;
-      case 1: done = mm_tile_typed<1, TH, TW>(p, lds.step, lds.part, redo); break;
-      case 30: done = mm_tile_typed<30, TH, TW>(p, lds.step, lds.part, redo); break;
-      default: done = mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, redo); break;
+      case 0: done = mm_tile_typed<0, TH, TW>(p, lds.step, lds.part, small, redo); break;
+      case 1: done = mm_tile_typed<1, TH, TW>(p, lds.step, lds.part, small, redo); break;
+      case 30: done = mm_tile_typed<30, TH, TW>(p, lds.step, lds.part, small, redo); break;
+      default: done = mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, small, redo); break;
     }
   }
   if (!done) mm_general<TH, TW>(p, lds.general.xs, lds.general.ws, lds.general.part, direct ? redo : nullptr);

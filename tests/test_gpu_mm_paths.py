@@ -89,6 +89,26 @@ def test_few_steps_keep_the_general_form_s_precision(eg2, gpu, wtype, k):
 
 @pytest.mark.parametrize("variant", MM_VARIANTS[:3], ids=[v[0] for v in MM_VARIANTS[:3]])
 @pytest.mark.parametrize("wtype", TYPES)
+def test_small_activations_keep_their_bits(eg2, gpu, variant, wtype):
+    """Rows of 2^-100 to 2^-126: the lowest part of such a value is below what
+    bf16 holds. Weights of 2^12, so that the sums are normal numbers."""
+    n, k, m = 70, 256, 70
+    rng = np.random.default_rng(wtype)
+    x = rng.standard_normal((n, k)) * 2.0 ** -np.linspace(100, 126, n)[:, None]
+    x[::7] = rng.standard_normal((len(x[::7]), k))  # ordinary rows between them
+    x = x.astype(np.float32)
+    w = rng.standard_normal((m, k)) * 2.0 ** 12
+    raw, dec = encode_weights(w.astype(np.float32), wtype)
+    x64, w64 = x.astype(np.float64), dec.astype(np.float64)
+    want, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64).T
+    got, general = (run(eg2, gpu, variant, x, raw, wtype, m, x_shift=s) for s in (0, 1))
+    rms = lambda y: np.sqrt((((y - want) / mag) ** 2).mean())
+    assert np.all(np.abs(got - want) <= k * 2.0 ** -24 * mag)
+    assert rms(got) <= 1.1 * rms(general)
+
+
+@pytest.mark.parametrize("variant", MM_VARIANTS[:3], ids=[v[0] for v in MM_VARIANTS[:3]])
+@pytest.mark.parametrize("wtype", TYPES)
 def test_rows_do_not_depend_on_their_neighbours(eg2, gpu, variant, wtype):
     """NaN, infinite, overflowing and tiny rows: the others keep their bits."""
     n, k, m = 70, 128, 70
