@@ -456,7 +456,8 @@ __device__ __forceinline__ void mm_direct(const EgMM& p, unsigned row0, unsigned
   StepRows<RB> x[DEPTH];
   StepWeights<TYPE, CB> w[DEPTH];
   auto load = [&](int slot, unsigned step) {
-    const unsigned base = 32 * min(step, steps - 1);  // past the end: the last step again, not used
+    if (DEPTH > 1 && step >= steps) return;  // uniform
+    const unsigned base = 32 * min(step, steps - 1);  // one in flight: past the end the last step again, not used
     w[slot].load(p.weight, p.k, col0, p.m, base);
     x[slot].load(p.x, p.k, row0, p.n, base);
   };
@@ -507,7 +508,7 @@ __device__ __forceinline__ bool mm_tile_typed(const EgMM& p, float (*step)[kStep
 #pragma unroll
     for (int j = 0; j < kA; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   float largest[RB] = {};
-  mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, wave, 4, step[wave], acc, largest);
+  mm_direct<TYPE, RB, CB, kDepth>(p, row0, col0, __builtin_amdgcn_readfirstlane(wave), 4, step[wave], acc, largest);
   if constexpr (kA > CB) acc[0][0] = (acc[0][0] + acc[0][1]) + (acc[0][2] + acc[0][3]);
   auto too_small = [&](int i) { return TYPE != 0 && largest[i] > 0.0f && largest[i] < kSplitsFrom; };
   bool good = true;
