@@ -171,10 +171,11 @@ __device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, 
 // The usual form, k a multiple of 32 and operands aligned (mm_direct_fits),
 // on bf16 MFMA (v_mfma_f32_16x16x32_bf16) with fp32 sums. The activations are
 // split exactly into three bf16 parts (8 + 8 + 8 of their 24 significant
-// bits, by truncation; a row too small for that takes the general form); Q8_0 values are whole numbers of at most 8 bits and
-// BF16 weights are bf16, so three products per weight are exact, and a Q8_0
-// block's scale is one fma on its 32-value dot; F16 weights split exactly into
-// two parts (six products); F32 weights stay on fp32 MFMA
+// bits, by truncation; a row too small for that takes the general form); Q8_0
+// values are whole numbers of at most 8 bits and BF16 weights are bf16, so
+// three products per weight are exact, and a Q8_0 block's scale is one fma on
+// its 32-value dot; F16 weights split exactly into two parts (six products);
+// F32 weights stay on fp32 MFMA
 // (v_mfma_f32_16x16x4f32). A product of 32 values takes 52 matrix cycles per
 // 16 x 16 tile instead of 263, and fewer roundings: the error against a
 // float64 product (2-norm) at 640 x 512 x 2048 is 7.0e-8 for Q8_0, 1.2e-7
@@ -301,9 +302,10 @@ struct StepWeights<8, BLOCKS> {  // Q8_0: a 34-byte block a column and step, at 
 #pragma unroll
     for (int j = 0; j < BLOCKS; ++j) {
       // The lane's 8 values (and, in lane 0 of the four, the scale) lie in
-      // three aligned words from 8 q bytes into the block rounded down to 4:
-      // each word holds bytes of this block, so none crosses into a page the
-      // matrix does not reach. (Unaligned 8-byte loads cost 0.9 us a step.)
+      // three aligned words from 8 q bytes into the block rounded down to 4,
+      // the first of which may begin two bytes before the block or the last
+      // end two after it: where those are not the matrix's, kQ8Edge reads.
+      // (Unaligned 8-byte loads cost 0.9 us a step.)
       const unsigned char* blk = static_cast<const unsigned char*>(w) +
                                  ((size_t)min(col0 + 16 * j + (lane >> 2), m - 1) * (k / 32) + base / 32) * 34 +
                                  8 * (lane & 3);
@@ -317,14 +319,17 @@ struct StepWeights<8, BLOCKS> {  // Q8_0: a 34-byte block a column and step, at 
     const unsigned lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < BLOCKS; ++j) {
-      const unsigned col = 16 * j + (lane >> 2);
       const bool odd = shift[j] != 0;  // the values start 4 bytes in, not 2
       const uint32_t lo = odd ? v[j][1] : __builtin_amdgcn_alignbyte(v[j][1], v[j][0], 2);
       const uint32_t hi = odd ? v[j][2] : __builtin_amdgcn_alignbyte(v[j][2], v[j][1], 2);
-      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(lds) + col * kPitch + 8 * (lane & 3)) =
-          make_uint2(lo, hi);
-      if ((lane & 3) == 0) lds[kScales + col] = eg2::fp16_bits_to_fp32(odd ? v[j][0] >> 16 : v[j][0] & 0xffffu);
+      put_block(lds, 16 * j + (lane >> 2), lo, hi, odd ? v[j][0] >> 16 : v[j][0] & 0xffffu);
     }
+  }
+  // This lane's 8 values of its column's block; of lane 0 of the four, the scale.
+  static __device__ __forceinline__ void put_block(float* lds, unsigned col, uint32_t lo, uint32_t hi, uint32_t scale) {
+    const unsigned q = threadIdx.x & 3;
+    *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(lds) + col * kPitch + 8 * q) = make_uint2(lo, hi);
+    if (q == 0) lds[kScales + col] = eg2::fp16_bits_to_fp32(scale);
   }
   static __device__ __forceinline__ uintx4 get(const float* lds, int block, float& scale) {  // as bf16
     const int lane = threadIdx.x & 63;
@@ -338,6 +343,48 @@ struct StepWeights<8, BLOCKS> {  // Q8_0: a 34-byte block a column and step, at 
       f[4 + e] = (float)(int8_t)(q.y >> (8 * e));
     }
     return split_bf16<1>(f).part[0];
+  }
+};
+// Q8_0 in a tile that holds the matrix's first block at 2 mod 4, or its last one
+// at 0 mod 4: nothing outside a block is read. Lane q of a block's four reads two
+// aligned words and one 16-bit value: at 0 mod 4 the words hold two bytes more
+// before the lane's 8 values (lane 0: the scale) and the 16 bits their last two;
+// at 2 mod 4 the words are the values and the 16 bits the scale. (For every tile
+// this takes 3-20% longer: a load more per block.)
+constexpr unsigned kQ8Edge = 9;
+constexpr unsigned q8_words_at(unsigned q, bool odd) { return 8 * q + (odd ? 2 : 0); }
+constexpr unsigned q8_half_at(unsigned q, bool odd) { return odd ? 0 : 8 * q + 8; }
+static_assert(q8_words_at(3, true) + 8 == 34 && q8_words_at(3, false) + 8 == 32 && q8_half_at(3, false) + 2 == 34,
+              "the last lane's reads end with the block");
+template <int BLOCKS>
+struct StepWeights<kQ8Edge, BLOCKS> {
+  uint32_t v[BLOCKS][2];
+  uint32_t half[BLOCKS];
+  bool odd[BLOCKS];
+  __device__ __forceinline__ void load(const void* w, unsigned k, unsigned col0, unsigned m, unsigned base) {
+    const unsigned lane = threadIdx.x & 63, q = lane & 3;
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j) {
+      const unsigned char* blk = static_cast<const unsigned char*>(w) +
+                                 ((size_t)min(col0 + 16 * j + (lane >> 2), m - 1) * (k / 32) + base / 32) * 34;
+      odd[j] = (reinterpret_cast<uintptr_t>(blk) & 2) != 0;
+      const uint32_t* p = reinterpret_cast<const uint32_t*>(blk + q8_words_at(q, odd[j]));
+      v[j][0] = p[0];
+      v[j][1] = p[1];
+      half[j] = *reinterpret_cast<const uint16_t*>(blk + q8_half_at(q, odd[j]));
+    }
+  }
+  __device__ __forceinline__ void put(float* lds) const {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j) {
+      const uint32_t lo = odd[j] ? v[j][0] : __builtin_amdgcn_alignbyte(v[j][1], v[j][0], 2);
+      const uint32_t hi = odd[j] ? v[j][1] : __builtin_amdgcn_alignbyte(half[j], v[j][1], 2);
+      StepWeights<8, BLOCKS>::put_block(lds, 16 * j + (lane >> 2), lo, hi, odd[j] ? half[j] : v[j][0] & 0xffffu);
+    }
+  }
+  static __device__ __forceinline__ uintx4 get(const float* lds, int block, float& scale) {
+    return StepWeights<8, BLOCKS>::get(lds, block, scale);
   }
 };
 template <int BLOCKS>
@@ -393,7 +440,7 @@ __device__ __forceinline__ void mm_step(const float* xs, const float* ws, floatx
 #pragma unroll
       for (int e = 0; e < 8; e += 2) largest[i] = fmaxf(fmaxf(fabsf(f[e]), fabsf(f[e + 1])), largest[i]);
     }
-    if constexpr (TYPE == 8) {
+    if constexpr (TYPE == 8 || TYPE == kQ8Edge) {
       constexpr int JB = RB == 1 ? CB : 1;  // column blocks at a time: RB JB = 4 independent dots
 #pragma unroll
       for (int j0 = 0; j0 < CB; j0 += JB) {
@@ -579,7 +626,14 @@ __device__ __forceinline__ void mm_tile(const EgMM& p) {
       case 0: done = mm_tile_typed<0, TH, TW>(p, lds.step, lds.part, small, redo); break;
       case 1: done = mm_tile_typed<1, TH, TW>(p, lds.step, lds.part, small, redo); break;
       case 30: done = mm_tile_typed<30, TH, TW>(p, lds.step, lds.part, small, redo); break;
-      default: done = mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, small, redo); break;
+      default: {
+        const uintptr_t first = reinterpret_cast<uintptr_t>(p.weight);
+        const uintptr_t end = first + (uintptr_t)p.m * (p.k / 32) * 34;
+        const bool edge = (blockIdx.x == 0 && first % 4 != 0) || ((blockIdx.x + 1) * TW >= p.m && end % 4 != 0);
+        done = edge ? mm_tile_typed<kQ8Edge, TH, TW>(p, lds.step, lds.part, small, redo)
+                    : mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, small, redo);
+        break;
+      }
     }
   }
   if (!done) mm_general<TH, TW>(p, lds.general.xs, lds.general.ws, lds.general.part, direct ? redo : nullptr);
