@@ -784,6 +784,7 @@ __device__ __forceinline__ void attention_chunked(const EgAttention& p, unsigned
     for (int u = 0; u < CV; ++u) acc[u] = acc[u] * alpha;
     const unsigned count = min(64u, hi - c0);
     const float* vbase = p.v + (size_t)c0 * KVS + kv + 4 * lane;
+#pragma unroll 8
     for (unsigned j = 0; j < count; ++j) {
       const float w = ps[j];
 #pragma unroll
@@ -821,15 +822,24 @@ __device__ __forceinline__ void attention_chunked(const EgAttention& p, unsigned
 //    row, dimensions 64 T + 4 r .., feeds four output tiles.
 // A key outside a token's range weighs 0 there. The 2-norm error to a float64
 // softmax is that of the form above or less (2.2e-7 against 2.8e-7 at 1021
-// tokens in 9 texts, 3.8e-7 against 8.4e-7 on one of 2048). Bound by the
+// tokens in 9 texts, 3.8e-7 against 8.4e-7 on one of 2048); a row's rounding
+// depends on the tile and wave its keys fall to, so on the packing. Bound by the
 // MFMAs (128 of 33 cycles per 16 x 16 scores) and, over few keys, by the
-// chain of one block: eg2_attention256, that form / this one in us: 1021
-// tokens in 9 texts 112 / 27, 2048 in 16 320 / 70, one of 2048 2,240 / 223;
-// eg2_attention512, one of 2048, 4,451 / 459.
+// chain of one block. eg2_attention256 inside a graph, that form / this one in
+// us: 1021 tokens in texts of 113 67 / 21, 2048 in texts of 128 145 / 27, one of
+// 2048 2,240 / 212; eg2_attention512 130 / 39, 285 / 50, 4,460 / 425.
+//
+// The host knows the token count and the window but not the ranges, so a tile
+// chooses by the keys that its tokens reach: few keys close together
+// (attention_few_keys), few keys far apart (row by row), else by keys. At 512
+// tokens, that form / this one: texts of one token 6.9 / 6.3, of 8 8.4 / 6.3, of
+// 16 10.3 / 6.3, of 24 12.1 / 10.2, of 64 21.5 / 11.4; window 4 8.7 / 8.1, 16
+// 14.2 / 10.4; at 2048 texts of one token 20.4 / 13.7. (By keys alone 10.0-11.4
+// at 512 whatever the texts, 22 at 2048.) Slower than one wave per row is only
+// what no packing has, neighbours whose few keys lie far apart: 8 keys anywhere,
+// 512 tokens 8.4 / 16.5, 2048 25.8 / 32.6; the rows of a tile share its CU.
 constexpr int kTileWaves = 8;
-// Below this the packing decides (its lengths are on the device): 256 tokens
-// in 4 texts 13.0 / 10.6, in 32 texts 6.2 / 10.1; 512 in 32 texts of 16, the
-// shortest that still gains, 10.7 / 10.4 (eg2_attention512 18.4 / 17.6).
+// From here the tiles fill half of the CUs; fewer tokens were not looked into.
 constexpr unsigned kTileTokens = 512;
 
 template <int D>
@@ -858,6 +868,130 @@ __device__ __forceinline__ float row16_sum(float v) {
   v = v + dpp16<0x4E>(v);
   v = v + dpp16<0x141>(v);
   return v + dpp16<0x140>(v);
+}
+
+// A tile whose tokens reach at most kFewKeys keys [first, last) between them:
+// texts of a few tokens, or a narrow window. Split by keys such a tile would
+// have work for one wave or a few; here every wave takes all the keys over an
+// eighth of the dimensions, its keys and values on their way at once, the
+// waves' partial scores are added through LDS, and each wave carries the whole
+// softmax and the context of its own dimensions. (With a fourth block of keys
+// the split by keys is faster: texts of 64, 512 tokens, 12.9 us against 11.4,
+// of three blocks 10.2 against 10.6.) lo, hi: the key ranges of the
+// lane's rows 4 g + v. Returns whether the tile needs the per-row form (as the
+// kernel's `polluted`); it has stored nothing then.
+constexpr int kFewBlocks = 3;
+constexpr unsigned kFewKeys = 16 * kFewBlocks;
+
+template <int D, int HEADS, int KVS>
+__device__ __forceinline__ bool attention_few_keys(const EgAttention& p, AttentionTileLds<D>& lds, unsigned t0,
+                                                   unsigned h, unsigned kv, const unsigned (&lo)[4],
+                                                   const unsigned (&hi)[4], unsigned first, unsigned last) {
+  constexpr int kDims = D / kTileWaves, kPer = kDims / 16;  // a wave's dimensions; float4s of a key, outputs per lane
+  typedef float floatxp __attribute__((ext_vector_type(kPer)));
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const unsigned nb = (last - first + 15) / 16;
+  floatx4 kf[kFewBlocks][kPer];  // key r of each block, dimensions 16 e + 4 g ..
+  floatxp vf[kFewBlocks][4];     // keys 4 g + j, dimensions kPer r ..
+#pragma unroll
+  for (int b = 0; b < kFewBlocks; ++b)
+    if (b < nb) {
+      const float* row = p.k + (size_t)min(first + 16 * b + r, last - 1) * KVS + kv + kDims * w + 4 * g;
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) kf[b][e] = *reinterpret_cast<const floatx4*>(row + 16 * e);
+    }
+#pragma unroll
+  for (int b = 0; b < kFewBlocks; ++b)
+    if (b < nb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        vf[b][j] = *reinterpret_cast<const floatxp*>(p.v + (size_t)min(first + 16 * b + 4 * g + j, last - 1) * KVS +
+                                                     kv + kDims * w + kPer * r);
+    }
+  __syncthreads();  // the queries and the exp table are in LDS
+  floatx4 qf[kPer];
+#pragma unroll
+  for (int e = 0; e < kPer; ++e) qf[e] = *reinterpret_cast<const floatx4*>(&lds.q[r][kDims * w + 16 * e + 4 * g]);
+  floatx4 s[kFewBlocks];
+  floatx4* partial = reinterpret_cast<floatx4*>(lds.part[w][0]);
+  bool polluted = false;
+#pragma unroll
+  for (int b = 0; b < kFewBlocks; ++b)
+    if (b < nb) {
+      s[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int e = 0; e < kPer; ++e)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[e][c], kf[b][e][c], s[b], 0, 0, 0);
+      partial[64 * b + lane] = s[b];
+    }
+#pragma unroll
+  for (int b = 0; b < kFewBlocks; ++b)
+    if (b < nb) {
+      bool all_in = true;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) all_in = all_in && lo[v] <= first + 16 * b && first + 16 * b + 16 <= hi[v];
+      if (!__all(all_in)) {
+        float probe = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < kPer; ++i) probe = __builtin_fmaf(vf[b][j][i], 0.0f, probe);
+        polluted = polluted || !(probe == 0.0f);
+      }
+    }
+  if (__syncthreads_or(polluted)) return true;
+  float m[4], l[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) m[v] = -__builtin_inff(), l[v] = 0.0f;
+#pragma unroll
+  for (int b = 0; b < kFewBlocks; ++b)
+    if (b < nb) {
+      s[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int i = 0; i < kTileWaves; ++i)
+        s[b] = s[b] + reinterpret_cast<const floatx4*>(lds.part[i][0])[64 * b + lane];
+      const unsigned key = first + 16 * b + r;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s[b][v] = key >= lo[v] && key < hi[v] ? s[b][v] : -__builtin_inff();
+        m[v] = fmaxf(m[v], s[b][v]);
+      }
+    }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) m[v] = row16_max(m[v]);
+  floatx4 acc[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int b = 0; b < kFewBlocks; ++b)
+    if (b < nb) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float pk = s[b][v] == -__builtin_inff() ? 0.0f : eg2::libm::expf_tab(s[b][v] - m[v], lds.exp_tab);
+        l[v] = l[v] + pk;
+        lds.p[w][4 * g + v][r] = pk;
+      }
+      wave_lds_order();
+      const floatx4 pf = *reinterpret_cast<const floatx4*>(&lds.p[w][r][4 * g]);  // query r, keys 4 g ..
+      wave_lds_order();  // p is rewritten by the next block
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[j], vf[b][j][i], acc[i], 0, 0, 0);
+    }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const float inv = hi[v] > lo[v] ? 1.0f / row16_sum(l[v]) : 0.0f;
+    const unsigned t = t0 + 4 * g + v;
+    floatxp o;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) o[i] = acc[i][v] * inv;
+    if (t < p.n) *reinterpret_cast<floatxp*>(p.out + ((size_t)t * HEADS + h) * D + kDims * w + kPer * r) = o;
+  }
+  return false;
 }
 
 template <int D, int HEADS, int KVS, int GROUP>
@@ -900,170 +1034,189 @@ attention_tile_kernel(EgAttention p) {
     }
   }
   first = min(first, last);
-  float m[4], l[4];
-  floatx4 acc[4 * T];
+  // The keys split over the waves; whether the tile needs the per-row form.
+  auto by_keys = [&]() -> bool {
+    float m[4], l[4];
+    floatx4 acc[4 * T];
 #pragma unroll
-  for (int v = 0; v < 4; ++v) m[v] = -__builtin_inff(), l[v] = 0.0f;
+    for (int v = 0; v < 4; ++v) m[v] = -__builtin_inff(), l[v] = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4 * T; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  __syncthreads();
-  // Rows 4 i + lane / 16 of a key block, dimensions 64 part + 4 (lane % 16) ..
-  // (rows past the last repeat it; their scores are masked).
-  floatx4 kr[4];
-  auto load_k = [&](unsigned k0, int part) {
+    for (int i = 0; i < 4 * T; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    __syncthreads();
+    // Rows 4 i + lane / 16 of a key block, dimensions 64 part + 4 (lane % 16) ..
+    // (rows past the last repeat it; their scores are masked).
+    floatx4 kr[4];
+    auto load_k = [&](unsigned k0, int part) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      kr[i] = *reinterpret_cast<const floatx4*>(p.k + (size_t)min(k0 + 4 * i + g, last - 1) * KVS + kv + 64 * part + 4 * r);
-  };
-  bool polluted = false;
-  if (first + 16 * w < last) load_k(first + 16 * w, 0);
-  for (unsigned k0 = first + 16 * w; k0 < last; k0 += 16 * kTileWaves) {
-    // Scores of keys k0 .. + 15, in four chains.
-    floatx4 s[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) s[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int part = 0; part < T; ++part) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<floatx4*>(&lds.part[w][4 * i + g][4 * r]) = kr[i];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      if (part + 1 < T)
-        load_k(k0, part + 1);
-      else if (k0 + 16 * kTileWaves < last)
-        load_k(k0 + 16 * kTileWaves, 0);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const floatx4 kf = *reinterpret_cast<const floatx4*>(&lds.part[w][r][16 * e + 4 * g]);
-        const floatx4 qf = *reinterpret_cast<const floatx4*>(&lds.q[r][64 * part + 16 * e + 4 * g]);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c], kf[c], s[c], 0, 0, 0);
-      }
-    }
-    // The block's first value rows, on their way during the softmax: keys
-    // k0 + 4 g + j, kAhead j in flight (one at 512 dimensions, whose context
-    // takes half of the registers).
-    constexpr int kAhead = D == 256 ? 2 : 1;
-    floatx4 vr[kAhead][T];
-    auto load_v = [&](int slot, int j) {
-      const float* vrow = p.v + (size_t)min(k0 + 4 * g + j, last - 1) * KVS + kv + 4 * r;
-#pragma unroll
-      for (int part = 0; part < T; ++part) vr[slot][part] = *reinterpret_cast<const floatx4*>(vrow + 64 * part);
+      for (int i = 0; i < 4; ++i)
+        kr[i] = *reinterpret_cast<const floatx4*>(p.k + (size_t)min(k0 + 4 * i + g, last - 1) * KVS + kv + 64 * part +
+                                                 4 * r);
     };
+    bool polluted = false;
+    if (first + 16 * w < last) load_k(first + 16 * w, 0);
+    for (unsigned k0 = first + 16 * w; k0 < last; k0 += 16 * kTileWaves) {
+      // Scores of keys k0 .. + 15, in four chains.
+      floatx4 s[4];
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) load_v(j, j);
-    float score[4], next[4];
-    bool grown = false;
+      for (int c = 0; c < 4; ++c) s[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {  // row 4 g + v, key k0 + r
-      const bool in = k0 + r >= lo[v] && k0 + r < hi[v];
-      score[v] = in ? (s[0][v] + s[1][v]) + (s[2][v] + s[3][v]) : -__builtin_inff();
-      next[v] = fmaxf(m[v], row16_max(score[v]));
-      grown = grown || next[v] != m[v];
-    }
-    if (__any(grown)) {
-      float alpha[4];
+      for (int part = 0; part < T; ++part) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<floatx4*>(&lds.part[w][4 * i + g][4 * r]) = kr[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (part + 1 < T)
+          load_k(k0, part + 1);
+        else if (k0 + 16 * kTileWaves < last)
+          load_k(k0 + 16 * kTileWaves, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const floatx4 kf = *reinterpret_cast<const floatx4*>(&lds.part[w][r][16 * e + 4 * g]);
+          const floatx4 qf = *reinterpret_cast<const floatx4*>(&lds.q[r][64 * part + 16 * e + 4 * g]);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[c], kf[c], s[c], 0, 0, 0);
+        }
+      }
+      // The block's first value rows, on their way during the softmax: keys
+      // k0 + 4 g + j, kAhead j in flight (one at 512 dimensions, whose context
+      // takes half of the registers).
+      constexpr int kAhead = D == 256 ? 2 : 1;
+      floatx4 vr[kAhead][T];
+      auto load_v = [&](int slot, int j) {
+        const float* vrow = p.v + (size_t)min(k0 + 4 * g + j, last - 1) * KVS + kv + 4 * r;
+#pragma unroll
+        for (int part = 0; part < T; ++part) vr[slot][part] = *reinterpret_cast<const floatx4*>(vrow + 64 * part);
+      };
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) load_v(j, j);
+      float score[4], next[4];
+      bool grown = false;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {  // row 4 g + v, key k0 + r
+        const bool in = k0 + r >= lo[v] && k0 + r < hi[v];
+        score[v] = in ? (s[0][v] + s[1][v]) + (s[2][v] + s[3][v]) : -__builtin_inff();
+        next[v] = fmaxf(m[v], row16_max(score[v]));
+        grown = grown || next[v] != m[v];
+      }
+      if (__any(grown)) {
+        float alpha[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          alpha[v] = next[v] == -__builtin_inff() ? 0.0f : exp_(m[v] - next[v]);  // no key of this row yet: all zero
+          l[v] = l[v] * alpha[v];
+          m[v] = next[v];
+        }
+#pragma unroll
+        for (int i = 0; i < 4 * T; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[i][v] = acc[i][v] * alpha[v];
+      }
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        alpha[v] = next[v] == -__builtin_inff() ? 0.0f : exp_(m[v] - next[v]);  // no key of this row yet: all zero
-        l[v] = l[v] * alpha[v];
-        m[v] = next[v];
+        const float pk = score[v] == -__builtin_inff() ? 0.0f : exp_(score[v] - m[v]);
+        l[v] = l[v] + row16_sum(pk);
+        lds.p[w][4 * g + v][r] = pk;
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const floatx4 pf = *reinterpret_cast<const floatx4*>(&lds.p[w][r][4 * g]);  // query r, keys 4 g ..
+      // A key outside a row's range weighs +0, but +0 times an infinite or NaN
+      // value is NaN: where some row does not have all 16 keys, such values send
+      // the whole tile to the per-row form below.
+      bool all_in = true;
 #pragma unroll
-      for (int i = 0; i < 4 * T; ++i)
+      for (int v = 0; v < 4; ++v) all_in = all_in && lo[v] <= k0 && k0 + 16 <= hi[v];
+      const bool partial = !__all(all_in);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[i][v] = acc[i][v] * alpha[v];
-    }
+      for (int j = 0; j < 4; ++j) {
+        if (partial) {  // uniform
+          float probe = 0.0f;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float pk = score[v] == -__builtin_inff() ? 0.0f : exp_(score[v] - m[v]);
-      l[v] = l[v] + row16_sum(pk);
-      lds.p[w][4 * g + v][r] = pk;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const floatx4 pf = *reinterpret_cast<const floatx4*>(&lds.p[w][r][4 * g]);  // query r, keys 4 g ..
-    // A key outside a row's range weighs +0, but +0 times an infinite or NaN
-    // value is NaN: where some row does not have all 16 keys, such values send
-    // the whole tile to the per-row form below.
-    bool all_in = true;
+          for (int part = 0; part < T; ++part)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) all_in = all_in && lo[v] <= k0 && k0 + 16 <= hi[v];
-    const bool partial = !__all(all_in);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (partial) {  // uniform
-        float probe = 0.0f;
+            for (int i = 0; i < 4; ++i) probe = __builtin_fmaf(vr[j % kAhead][part][i], 0.0f, probe);
+          polluted = polluted || !(probe == 0.0f);
+        }
 #pragma unroll
         for (int part = 0; part < T; ++part)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) probe = __builtin_fmaf(vr[j % kAhead][part][i], 0.0f, probe);
-        polluted = polluted || !(probe == 0.0f);
+          for (int i = 0; i < 4; ++i)
+            acc[4 * part + i] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(pf[j], vr[j % kAhead][part][i], acc[4 * part + i], 0, 0, 0);
+        if (j + kAhead < 4) load_v(j % kAhead, j + kAhead);
       }
-#pragma unroll
-      for (int part = 0; part < T; ++part)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[4 * part + i] =
-              __builtin_amdgcn_mfma_f32_16x16x4f32(pf[j], vr[j % kAhead][part][i], acc[4 * part + i], 0, 0, 0);
-      if (j + kAhead < 4) load_v(j % kAhead, j + kAhead);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // p is rewritten by the next block
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // p is rewritten by the next block
-  }
-  // The waves' contexts brought to the rows' common maximum and added; thread
-  // 16 i + row computes wave i's factor for the row.
-  if (__syncthreads_or(polluted)) {
-    for (unsigned i = w; i < 16 && t0 + i < p.n; i += kTileWaves)
-      attention_chunked<D, HEADS, KVS, GROUP>(p, (t0 + i) * HEADS + h, reinterpret_cast<floatx4*>(lds.q[w]),
-                                              lds.part[w][0]);
-    return;
-  }
-  if (r == 0) {
+    // The waves' contexts brought to the rows' common maximum and added; thread
+    // 16 i + row computes wave i's factor for the row.
+    if (__syncthreads_or(polluted)) return true;
+    if (r == 0) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) lds.m[w][4 * g + v] = m[v], lds.l[w][4 * g + v] = l[v];
-  }
-  __syncthreads();
-  if (tid < 16 * kTileWaves) {
-    const int row = tid & 15;
-    const float own = lds.m[tid >> 4][row];
-    float top = own;
-#pragma unroll
-    for (int i = 0; i < kTileWaves; ++i) top = fmaxf(top, lds.m[i][row]);
-    lds.p[tid >> 4][row][0] = own == -__builtin_inff() ? 0.0f : exp_(own - top);
-  }
-  __syncthreads();
-  float scale[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int row = 4 * g + v;
-    float den = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kTileWaves; ++i) den = den + lds.l[i][row] * lds.p[i][row][0];
-    scale[v] = hi[v] > lo[v] ? lds.p[w][row][0] / den : 0.0f;
-  }
-#pragma unroll
-  for (int part = 0; part < T; ++part) {
-    if (part) __syncthreads();
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      floatx4 o;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = acc[4 * part + i][v] * scale[v];
-      *reinterpret_cast<floatx4*>(&lds.part[w][4 * g + v][4 * r]) = o;
+      for (int v = 0; v < 4; ++v) lds.m[w][4 * g + v] = m[v], lds.l[w][4 * g + v] = l[v];
     }
     __syncthreads();
-    const int row = tid >> 5, e = 2 * (tid & 31);  // 512 threads x 2 outputs
-    float a = 0.0f, b = 0.0f;
+    if (tid < 16 * kTileWaves) {
+      const int row = tid & 15;
+      const float own = lds.m[tid >> 4][row];
+      float top = own;
 #pragma unroll
-    for (int i = 0; i < kTileWaves; ++i) {
-      a = a + lds.part[i][row][e];
-      b = b + lds.part[i][row][e + 1];
+      for (int i = 0; i < kTileWaves; ++i) top = fmaxf(top, lds.m[i][row]);
+      lds.p[tid >> 4][row][0] = own == -__builtin_inff() ? 0.0f : exp_(own - top);
     }
-    if (t0 + row < p.n) {
-      float* dst = p.out + ((size_t)(t0 + row) * HEADS + h) * D + 64 * part + e;
-      dst[0] = a;
-      dst[1] = b;
+    __syncthreads();
+    float scale[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = 4 * g + v;
+      float den = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kTileWaves; ++i) den = den + lds.l[i][row] * lds.p[i][row][0];
+      scale[v] = hi[v] > lo[v] ? lds.p[w][row][0] / den : 0.0f;
     }
+#pragma unroll
+    for (int part = 0; part < T; ++part) {
+      if (part) __syncthreads();
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        floatx4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = acc[4 * part + i][v] * scale[v];
+        *reinterpret_cast<floatx4*>(&lds.part[w][4 * g + v][4 * r]) = o;
+      }
+      __syncthreads();
+      const int row = tid >> 5, e = 2 * (tid & 31);  // 512 threads x 2 outputs
+      float a = 0.0f, b = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kTileWaves; ++i) {
+        a = a + lds.part[i][row][e];
+        b = b + lds.part[i][row][e + 1];
+      }
+      if (t0 + row < p.n) {
+        float* dst = p.out + ((size_t)(t0 + row) * HEADS + h) * D + 64 * part + e;
+        dst[0] = a;
+        dst[1] = b;
+      }
+    }
+    return false;
+  };
+  // Tokens whose few keys lie far apart go one by one: a row costs about 15 us +
+  // 0.7 a key where the tile costs 3 + 6.5 per 128 keys of the whole reach
+  // (2048 tokens with 8 keys each anywhere: 182 us by keys, 32 by row).
+  const unsigned reach = last - first;
+  bool rows = false;
+  if (reach > 256) {
+    unsigned longest = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      longest = max(longest, (unsigned)__builtin_amdgcn_readlane(hi[i & 3] - lo[i & 3], 16 * (i >> 2)));
+    rows = longest + 17 < 9 * ((reach + 127) / 128);
   }
+  if (!rows)
+    rows = reach <= kFewKeys ? attention_few_keys<D, HEADS, KVS>(p, lds, t0, h, kv, lo, hi, first, last) : by_keys();
+  if (!rows) return;
+  __syncthreads();
+  for (unsigned i = w; i < 16 && t0 + i < p.n; i += kTileWaves)
+    attention_chunked<D, HEADS, KVS, GROUP>(p, (t0 + i) * HEADS + h, reinterpret_cast<floatx4*>(lds.q[w]),
+                                            lds.part[w][0]);
 }
 
 }  // namespace

@@ -138,3 +138,58 @@ def test_scores_of_minus_infinity_weigh_nothing(eg2, gpu, op, n, window):
     assert np.isnan(want[110]).all() and np.isfinite(want[:50]).all() and np.isfinite(want[400:]).all()
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.nanmax(np.abs(got - want)) <= 2e-5
+
+
+def short_lens(seed, total, top):
+    rng, out = np.random.default_rng(seed), []
+    while sum(out) < total:
+        out.append(int(rng.integers(1, top + 1)))
+    return out
+
+
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("lens,window", [([1] * 513, 0), ([3] * 200, 0), ([8] * 70, 2), (short_lens(1, 600, 15), 0),
+                                         (short_lens(2, 600, 15), 4), ([16] * 32, 0), ([17] * 31, 0), ([24, 40] * 9, 0),
+                                         ([32] * 17, 0), ([33] * 16, 0), ([64] * 9, 0), ([65] * 8, 0), ([600], 1),
+                                         ([600], 24), ([600], 25), (short_lens(3, 700, 40), 0)],
+                         ids=lambda v: f"{len(v)}x{v[0]}" if isinstance(v, list) else f"w{v}")
+def test_short_texts_and_narrow_windows(eg2, gpu, op, lens, window):
+    """Tiles that reach few keys: texts shorter than a tile and up to a few
+    blocks, aligned with the tiles and not, and windows that leave as few."""
+    import torch
+
+    heads, d, kvs, group = OPS[op]
+    n = sum(lens)
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    bounds = np.array([(starts[s], starts[s + 1]) for s in range(len(lens)) for _ in range(lens[s])], np.uint32)
+    rng = np.random.default_rng(n + d + window)
+    q = (rng.standard_normal((n, heads, d)) / np.sqrt(d)).astype(np.float32)
+    k, v = (rng.standard_normal((n, kvs)).astype(np.float32) for _ in range(2))
+    y = torch.full((n * heads * d + 64,), 7.0, device=gpu)
+    t = [dev(a, gpu) for a in (q, k, v, bounds.reshape(-1).view(np.int32))]
+    rec = eg2.EgAttention(y.data_ptr(), *(a.data_ptr() for a in t), n, window)
+    eg2.ops.op(op, rec, heads * n, 64)
+    got = host(y)
+    want = softmax_reference(q, k, v, bounds, n, heads, d, kvs, group, window)
+    assert np.abs(got[:-64].reshape(n, heads, d) - want).max() <= 2e-5
+    assert (got[-64:] == 7.0).all()
+
+
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("n,width", [(512, 1), (528, 8), (1100, 8), (1100, 100)])
+def test_scattered_ranges(eg2, gpu, op, n, width):
+    """Neighbouring tokens with key ranges far apart."""
+    import torch
+
+    heads, d, kvs, group = OPS[op]
+    rng = np.random.default_rng(n + width)
+    lo = rng.integers(0, n - width + 1, n)
+    bounds = np.stack([lo, lo + width], 1).astype(np.uint32)
+    q = (rng.standard_normal((n, heads, d)) / np.sqrt(d)).astype(np.float32)
+    k, v = (rng.standard_normal((n, kvs)).astype(np.float32) for _ in range(2))
+    y = torch.full((n * heads * d,), 7.0, device=gpu)
+    t = [dev(a, gpu) for a in (q, k, v, bounds.reshape(-1).view(np.int32))]
+    rec = eg2.EgAttention(y.data_ptr(), *(a.data_ptr() for a in t), n, 0)
+    eg2.ops.op(op, rec, heads * n, 64)
+    want = softmax_reference(q, k, v, bounds, n, heads, d, kvs, group, 0)
+    assert np.abs(host(y).reshape(n, heads, d) - want).max() <= 2e-5
