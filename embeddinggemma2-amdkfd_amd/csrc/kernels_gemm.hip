@@ -407,11 +407,35 @@ inline bool scales_fit(int k, int ld) { return (uint64_t)(k / kQK) * (uint64_t)l
 //   gemm m 768, k 3072:  n 16 17.5 / 5.5, 512 18.5 / 15.6
 // The narrow kernel's time grows with its workgroups (one per 16 x 16 tile,
 // 24 to 48 KB of LDS each), the wide one's hardly until its tiles fill the
-// chip, so the line is a number of tiles.
-constexpr int kNarrowTiles = 1792;
-// gate|up + GeGLU: n 32 8.4 / 5.9, 96 8.7 / 6.1, 192 8.5 / 8.1, 256 8.7 / 10.6
-// (36 workgroups of 53 KB per 16 rows).
-constexpr int kNarrowGegluRows = 192;
+// chip, so the line is a number of tiles. It is in proportion to the blocks, since
+// the wide kernel's time is, while a narrow workgroup takes whole chunks of 24, 36
+// or 48 blocks: m 768, k 32: n 64 2.9 / 2.8, 128 2.9 / 3.2, 512 3.0 / 5.3; k 256:
+// 192 3.9 / 3.8, 320 3.9 / 4.3; k 384: 288 4.7 / 4.4, 320 4.3 / 4.5. Where most of a
+// chunk is filled the line lies higher: k 512: n 512 5.7 / 5.6, 576 5.2 / 6.0; k 896:
+// 512 7.9 / 7.1, 576 6.6 / 7.8; and several chunks of which the last is nearly empty
+// lose earlier: k 3104: 320 15.6 / 14.4, 384 15.9 / 18.1; k 1568: 320 10.2 / 10.1,
+// 384 10.2 / 12.6; hence the bound on the padding.
+constexpr int kNarrowTiles = 1792, kNarrowTilesFilled = 1536, kNarrowPadding = 44000;
+inline bool narrow_gemm(int n, int m, int nb) {
+  const int64_t tiles = (int64_t)((n + 15) / 16) * ((m + 15) / 16);
+  const int64_t padded = nb <= 24 ? 24 : nb <= 36 ? 36 : (nb + 47) / 48 * 48;
+  return (tiles * padded <= (int64_t)kNarrowTiles * nb || (tiles <= kNarrowTilesFilled && 3 * nb >= 2 * padded)) &&
+         tiles * (padded - nb) <= kNarrowPadding;
+}
+// gate|up + GeGLU: ff / 32 workgroups per 16 rows, each over chunks of 24 blocks,
+// in rounds of one per CU (a second workgroup of 53 KB and 512 threads on a CU
+// only shares it), so the time is a number of rounds and chunks, whatever is in
+// them, where the wide kernel's is in proportion to the blocks: k 768, ff 1152:
+// n 112 8.8 / 6.1, 128 8.8 / 8.0, 224 8.9 / 8.1, 256 8.8 / 10.3; ff 4608: 32 8.9 / 8.0,
+// 64 8.9 / 10.3; one round at k 128 5.2 / 5.9, 192 5.6 / 6.0, 256 6.1 / 5.9, 800 7.7 /
+// 8.4 (two chunks, the second for one block), 1152 10.5 / 8.9; two rounds at k 512
+// 7.6 / 8.2, 640 8.2 / 8.1, 1536 12.4 / 13.4. So: one round whose last chunk is at
+// least a third full, or two of one chunk nearly full.
+inline bool narrow_geglu(int n, int ff, int nb) {
+  const int64_t groups = (int64_t)(ff / kQK) * ((n + 15) / 16);
+  const int last = nb % 24 ? nb % 24 : 24;
+  return (groups <= 256 && last >= 8) || (groups <= 512 && nb >= 20 && nb <= 24);
+}
 // Q|K|V in a recorded graph: the fused kernel gives a head's 256 columns to one
 // workgroup, so 32 rows run on 5 CUs; below this the narrow projection (80
 // workgroups per 16 rows) followed by the standalone QK-norm / RoPE in place is
@@ -426,7 +450,7 @@ hipError_t launch_gemm_q8(const int8_t* xq, const float* xd, int ldx, const int8
   if (n <= 0 || m <= 0 || k <= 0 || k % kQK != 0 || ldy < m || ldx < n || ldw < m) return hipErrorInvalidValue;
   if (!scales_fit(k, ldx) || !scales_fit(k, ldw)) return hipErrorInvalidValue;
   const int nb = k / kQK;
-  if ((int64_t)((n + 15) / 16) * ((m + 15) / 16) <= kNarrowTiles) {
+  if (narrow_gemm(n, m, nb)) {
     const dim3 grid((m + 15) / 16, (n + 15) / 16);
     auto* kernel = nb <= 24 ? gemm_q8_narrow_kernel<6> : nb <= 36 ? gemm_q8_narrow_kernel<9> : gemm_q8_narrow_kernel<12>;
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb, ldy);
@@ -442,7 +466,7 @@ hipError_t launch_gemm_q8_geglu(const int8_t* xq, const float* xd, int ldx, cons
   if (n <= 0 || ff <= 0 || ff % kQK != 0 || k <= 0 || k % kQK != 0 || ldx < n || ldw < m || ldg < n)
     return hipErrorInvalidValue;
   if (!scales_fit(k, ldx) || !scales_fit(k, ldw)) return hipErrorInvalidValue;
-  if (n <= kNarrowGegluRows) {
+  if (narrow_geglu(n, ff, k / kQK)) {
     hipLaunchKernelGGL(gemm_q8_geglu_narrow_kernel, dim3(ff / kQK, (n + 15) / 16), dim3(512), 0, st, xq, xd, ldx, wq, wd,
                        ldw, n, ff, k / kQK, gq, gd, ldg);
     return hipGetLastError();

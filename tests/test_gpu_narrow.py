@@ -7,6 +7,7 @@ leave a part of one, and widths that leave a part of a column tile."""
 import numpy as np
 import pytest
 
+import gguf_py
 import oracle_lib as OL
 from oracle_lib import HEAD_DIM, N_EMBD, N_FF, quantize_q8_0
 from test_gpu_ops import (bits, dev, device_q8, device_weights, empty, host, oracle_gelu_q8, oracle_qk_norm_rope,
@@ -24,7 +25,10 @@ def operands(n, m, k, seed, std=0.02):
 @pytest.mark.parametrize("n,m,k", [
     (1, 768, 768), (15, 33, 32), (16, 768, 1152), (17, 40, 800), (31, 100, 1184), (48, 70, 1600),
     (512, 896, 768),    # 32 x 56 tiles: the last narrow size
-    (512, 912, 224), (513, 896, 192), (700, 768, 320)])  # the first wide ones; 7 and 10 blocks take the loop's tail
+    (512, 912, 224), (513, 896, 192), (700, 768, 320),  # wide ones; 7 and 10 blocks take the loop's tail
+    # both sides of the line at one block, a third and two thirds of a chunk, one block in the second and third chunk
+    (64, 288, 32), (80, 288, 32), (192, 768, 256), (208, 768, 256), (512, 768, 512), (513, 768, 512),
+    (304, 768, 1568), (305, 768, 1568), (304, 768, 3104), (321, 768, 3104)])
 def test_gemm_edges(eg2, gpu, n, m, k):
     import torch
 
@@ -37,7 +41,12 @@ def test_gemm_edges(eg2, gpu, n, m, k):
 
 
 @pytest.mark.parametrize("n,ff,k,tied", [(1, N_FF, N_EMBD, False), (15, 64, 416, False), (33, 96, 832, True),
-                                         (192, N_FF, N_EMBD, True), (193, N_FF, N_EMBD, True), (224, 64, 160, False)])
+                                         (192, N_FF, N_EMBD, True), (193, N_FF, N_EMBD, True), (224, 64, 160, False),
+                                         # the last of two rounds and the first past it; one round of other widths
+                                         # and block counts, and what is past it or has too few blocks
+                                         (224, N_FF, N_EMBD, False), (225, N_FF, N_EMBD, False), (2048, 64, 256, True),
+                                         (2049, 64, 256, False), (17, 64, 224, False), (112, N_FF, 1024, False),
+                                         (113, N_FF, 1024, False), (40, 2304, 992, False)])
 def test_geglu_edges(eg2, gpu, n, ff, k, tied):
     """tied: repeated weight rows, so blocks with equal maxima."""
     rng = np.random.default_rng(n + ff)
@@ -57,6 +66,8 @@ def test_geglu_edges(eg2, gpu, n, ff, k, tied):
 
 @pytest.mark.parametrize("n,k", [(1, 768), (17, 224), (256, 768), (257, 768), (260, 224)])
 def test_qkv_rope_edges(eg2, gpu, n, k):
+    """The operator, which is one kernel at every size (a recorded wave's
+    projection changes kernels at 256 rows: test_wave_edges)."""
     import torch
 
     rng = np.random.default_rng(n + k)
@@ -69,3 +80,29 @@ def test_qkv_rope_edges(eg2, gpu, n, k):
     got = host(out)
     assert np.array_equal(bits(got[:n]), bits(oracle_qk_norm_rope(OL.gemm_q8_0(w, xb), qw, kw, pos, 1e4)))
     assert (got[n] == 7.0).all()
+
+
+@pytest.fixture(scope="module")
+def encoder(eg2, gpu, tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("narrow") / "model.gguf")
+    eg2.synth_gguf(path, seed=9, n_layer=2, dense_head=True, sliding_window=64, sliding_window_pattern=2,
+                   rope_base_full=1e6, rope_base_swa=1e4, threads=8)
+    enc = eg2.Encoder(path)
+    yield enc, gguf_py.oracle_model(path)
+    enc.close()
+
+
+@pytest.mark.parametrize("tokens", [50, 64, 65, 192, 193, 224, 225, 256, 257])
+@pytest.mark.parametrize("texts", [1, 7])
+def test_wave_edges(encoder, tokens, texts):
+    """Waves on both sides of the lines where the recorded layers change
+    kernels: the smallest that is not a short wave (64 rows), gate|up (up to
+    224 rows the narrow kernel) and Q|K|V (up to 256 rows two kernels)."""
+    enc, model = encoder
+    rng = np.random.default_rng(tokens + texts)
+    cuts = np.sort(rng.choice(np.arange(1, tokens), texts - 1, replace=False))
+    offsets = np.concatenate([[0], cuts, [tokens]])
+    ids = rng.integers(0, OL.VOCAB, tokens).astype(np.int32)
+    want = OL.forward(model, ids, offsets.astype(np.uint64), threads=8)
+    for _ in range(2):  # the second call replays the graph
+        assert np.array_equal(enc.batch(ids, offsets), want)
