@@ -221,9 +221,11 @@ __device__ __forceinline__ void geglu_epilogue(const floatx16& acc, int tr, int 
 // or (LDS) as plain registers read through a 256-byte ring of the wave's own
 // (dx_ring): a SIMD issues a plain v_mul_f32 in 2.4 cycles and a DPP one in
 // 4.3 (measured, four waves), so block and wave cost 145 cycles instead of
-// 193 when the arithmetic bounds. gate|up, whose 4.5 waves per SIMD do fill
-// it, takes the ring: 18.0 -> 16.9 us at 2048 rows, one 16 x 128 wave 2.26
-// -> 2.21 ms. O, down and Q|K|V, with one or two waves per SIMD, keep the
+// 193 when the arithmetic bounds. gate|up with more than a workgroup per CU
+// takes the ring: 4.5 waves per SIMD at 2048 rows 18.0 -> 16.9 us, one 16 x
+// 128 wave 2.26 -> 2.21 ms, 1024 rows 12.9 -> 11.9, 512 (1.1 workgroups) 10.1 ->
+// 9.8; with one or less its round trip shows (384 rows 8.7 -> 9.0) and the DPP
+// stays. O, down and Q|K|V, with one or two waves per SIMD, keep the
 // DPP: alone they gain 0-5%, but with four waves in flight the step got 1.5%
 // slower (their LDS round trips then sit on the chain and on the LDS that
 // the other waves' attention uses). Operands go straight to registers (the row-tile
@@ -336,7 +338,8 @@ __device__ __forceinline__ floatx16 q8_block_loop(const int8_t* atile, const flo
 // TAIL: nb % kUnroll != 0 (a separate instantiation: the tail code costs
 // registers, and every projection of the model has nb % 4 == 0). GEGLU:
 // the epilogue above replaces the fp32 store (y and ldy unused; m = 2 ff).
-template <bool TAIL, bool GEGLU>
+// RING: the row scales through the LDS ring (q8_block_loop).
+template <bool TAIL, bool GEGLU, bool RING>
 __global__ void __launch_bounds__(256)
 gemm_q8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xd, int ldx, const int8_t* __restrict__ wq,
                const float* __restrict__ wd, int ldw, float* __restrict__ y, int n, int m, int nb, int ldy,
@@ -361,13 +364,13 @@ gemm_q8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xd, int 
   // Row whose scale this lane loads: row lane % 32 for the LDS ring; for the
   // DPP broadcast lane 16r + v carries the scale of output register v for
   // the lanes of 16-lane row r.
-  __shared__ __align__(16) float dx_ring[GEGLU ? 4 : 1][2 * 32];
-  const int srow = GEGLU ? lane & 31 : 8 * ((lane & 15) >> 2) + 4 * g + (lane & 3);
-  const floatx16 acc = q8_block_loop<TAIL, GEGLU>(
+  __shared__ __align__(16) float dx_ring[RING ? 4 : 1][2 * 32];
+  const int srow = RING ? lane & 31 : 8 * ((lane & 15) >> 2) + 4 * g + (lane & 3);
+  const floatx16 acc = q8_block_loop<TAIL, RING>(
       xq + (size_t)min(2 * tr + wr, (n + 31) / 32 - 1) * nb * kTile, xd, ldx, n,
       4u * (uint32_t)min(64 * tr + 32 * wr + srow, n - 1),
       wq + (size_t)min(2 * tc + wc, (m + 31) / 32 - 1) * nb * kTile, wd, ldw, m,
-      4u * (uint32_t)min(64 * tc + 32 * wc + (lane & 31), m - 1), nb, lane, dx_ring[GEGLU ? w : 0]);
+      4u * (uint32_t)min(64 * tc + 32 * wc + (lane & 31), m - 1), nb, lane, dx_ring[RING ? w : 0]);
   if constexpr (GEGLU) {
     geglu_epilogue(acc, tr, tc, wr, wc, n, m / 64, gq, gd, ldy);
   } else {
@@ -381,16 +384,16 @@ gemm_q8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xd, int 
 }
 
 // The kernel for nb blocks (TAIL: nb is not a multiple of kUnroll).
-template <bool GEGLU>
+template <bool GEGLU, bool RING>
 static hipError_t launch_gemm_kernel(dim3 grid, size_t lds, hipStream_t st, const int8_t* xq, const float* xd,
                                      int ldx, const int8_t* wq, const float* wd, int ldw, float* y, int n, int m,
                                      int nb, int ldy, int8_t* gq, float* gd) {
   if (nb % kUnroll == 0)
-    hipLaunchKernelGGL((gemm_q8_kernel<false, GEGLU>), grid, dim3(256), lds, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb,
-                       ldy, gq, gd);
+    hipLaunchKernelGGL((gemm_q8_kernel<false, GEGLU, RING>), grid, dim3(256), lds, st, xq, xd, ldx, wq, wd, ldw, y, n,
+                       m, nb, ldy, gq, gd);
   else
-    hipLaunchKernelGGL((gemm_q8_kernel<true, GEGLU>), grid, dim3(256), lds, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb,
-                       ldy, gq, gd);
+    hipLaunchKernelGGL((gemm_q8_kernel<true, GEGLU, RING>), grid, dim3(256), lds, st, xq, xd, ldx, wq, wd, ldw, y, n, m,
+                       nb, ldy, gq, gd);
   return hipGetLastError();
 }
 
@@ -456,8 +459,8 @@ hipError_t launch_gemm_q8(const int8_t* xq, const float* xd, int ldx, const int8
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb, ldy);
     return hipGetLastError();
   }
-  return launch_gemm_kernel<false>(gemm_grid(n, m, true), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb, ldy, nullptr,
-                                   nullptr);
+  return launch_gemm_kernel<false, false>(gemm_grid(n, m, true), 0, st, xq, xd, ldx, wq, wd, ldw, y, n, m, nb, ldy,
+                                          nullptr, nullptr);
 }
 
 hipError_t launch_gemm_q8_geglu(const int8_t* xq, const float* xd, int ldx, const int8_t* wq, const float* wd, int ldw,
@@ -473,8 +476,10 @@ hipError_t launch_gemm_q8_geglu(const int8_t* xq, const float* xd, int ldx, cons
   }
   // LDS: the epilogue's gate and up tiles
   constexpr size_t lds = 2 * 2 * 32 * kGPitch * sizeof(float);
-  return launch_gemm_kernel<true>(gemm_grid(n, m), lds, st, xq, xd, ldx, wq, wd, ldw, nullptr, n, m, k / kQK, ldg, gq,
-                                  gd);
+  // More than a workgroup per CU: the LDS ring (q8_block_loop).
+  auto* launch = (int64_t)((n + 63) / 64) * (m / 64) > 256 ? launch_gemm_kernel<true, true>
+                                                           : launch_gemm_kernel<true, false>;
+  return launch(gemm_grid(n, m), lds, st, xq, xd, ldx, wq, wd, ldw, nullptr, n, m, k / kQK, ldg, gq, gd);
 }
 
 // ---------------------------------------------------------------------------

@@ -46,7 +46,9 @@ def test_gemm_edges(eg2, gpu, n, m, k):
                                          # and block counts, and what is past it or has too few blocks
                                          (224, N_FF, N_EMBD, False), (225, N_FF, N_EMBD, False), (2048, 64, 256, True),
                                          (2049, 64, 256, False), (17, 64, 224, False), (112, N_FF, 1024, False),
-                                         (113, N_FF, 1024, False), (40, 2304, 992, False)])
+                                         (113, N_FF, 1024, False), (40, 2304, 992, False),
+                                         # the wide kernel up to a workgroup per CU and past it
+                                         (448, N_FF, N_EMBD, True), (449, N_FF, N_EMBD, True), (450, N_FF, 160, False)])
 def test_geglu_edges(eg2, gpu, n, ff, k, tied):
     """tied: repeated weight rows, so blocks with equal maxima."""
     rng = np.random.default_rng(n + ff)
