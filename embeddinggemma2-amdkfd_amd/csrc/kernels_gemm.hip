@@ -433,11 +433,14 @@ inline bool narrow_gemm(int n, int m, int nb) {
 // 64 8.9 / 10.3; one round at k 128 5.2 / 5.9, 192 5.6 / 6.0, 256 6.1 / 5.9, 800 7.7 /
 // 8.4 (two chunks, the second for one block), 1152 10.5 / 8.9; two rounds at k 512
 // 7.6 / 8.2, 640 8.2 / 8.1, 1536 12.4 / 13.4. So: one round whose last chunk is at
-// least a third full, or two of one chunk nearly full.
+// least a third full, or most of two of one chunk nearly full -- not all of the
+// second, since beside other waves' kernels the wide one is the smaller: 224
+// tokens alone 1,571 us a wave instead of 1,612, with four in flight 549 instead
+// of 508 (192 tokens: 503 either way).
 inline bool narrow_geglu(int n, int ff, int nb) {
   const int64_t groups = (int64_t)(ff / kQK) * ((n + 15) / 16);
   const int last = nb % 24 ? nb % 24 : 24;
-  return (groups <= 256 && last >= 8) || (groups <= 512 && nb >= 20 && nb <= 24);
+  return (groups <= 256 && last >= 8) || (groups <= 432 && nb >= 20 && nb <= 24);
 }
 // Q|K|V in a recorded graph: the fused kernel gives a head's 256 columns to one
 // workgroup, so 32 rows run on 5 CUs; below this the narrow projection (80

@@ -42,8 +42,8 @@ def test_gemm_edges(eg2, gpu, n, m, k):
 
 @pytest.mark.parametrize("n,ff,k,tied", [(1, N_FF, N_EMBD, False), (15, 64, 416, False), (33, 96, 832, True),
                                          (192, N_FF, N_EMBD, True), (193, N_FF, N_EMBD, True), (224, 64, 160, False),
-                                         # the last of two rounds and the first past it; one round of other widths
-                                         # and block counts, and what is past it or has too few blocks
+                                         # one round of other widths and block counts, and what is past it or has
+                                         # too few blocks
                                          (224, N_FF, N_EMBD, False), (225, N_FF, N_EMBD, False), (2048, 64, 256, True),
                                          (2049, 64, 256, False), (17, 64, 224, False), (112, N_FF, 1024, False),
                                          (113, N_FF, 1024, False), (40, 2304, 992, False),
@@ -99,7 +99,7 @@ def encoder(eg2, gpu, tmp_path_factory):
 def test_wave_edges(encoder, tokens, texts):
     """Waves on both sides of the lines where the recorded layers change
     kernels: the smallest that is not a short wave (64 rows), gate|up (up to
-    224 rows the narrow kernel) and Q|K|V (up to 256 rows two kernels)."""
+    192 rows the narrow kernel) and Q|K|V (up to 256 rows two kernels)."""
     enc, model = encoder
     rng = np.random.default_rng(tokens + texts)
     cuts = np.sort(rng.choice(np.arange(1, tokens), texts - 1, replace=False))
