@@ -10,8 +10,6 @@
 #include <stddef.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 #include "eg2_libm.hpp"
 
 namespace eg2 {
@@ -134,6 +132,15 @@ __device__ __forceinline__ int32_t q8_value(float v, float id) {
   return id > 3.40282347e38f ? -128 : q8_round(v * id);
 }
 
+// DPP move within 16-lane rows (quad permutations, mirrors, shifts, broadcasts):
+// writes every lane; lanes shifted in from outside the row read 0.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+constexpr int kQuad1032 = 0xB1, kQuad2301 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int kRowMirror = 0x140, kRowHalfMirror = 0x141;
+
 // v combined (op: max or +) with its copies in lanes l ^ 16 and l ^ 32,
 // i.e. over the four 16-lane rows, on the VALU: v_permlane16_swap and
 // v_permlane32_swap of v with itself leave v of lane l and of its partner in
@@ -159,14 +166,10 @@ __device__ __forceinline__ float rows4_sum(float v) {
 // v_permlane16_swap (five LDS shuffles, some 120 cycles each, sat on the
 // chain of the kernels that quantize a value per lane).
 __device__ __forceinline__ float half_wave_max(float v) {
-  auto move = [](float x, auto ctrl) {
-    return __builtin_bit_cast(float,
-                              __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true));
-  };
-  v = fmaxf(v, move(v, std::integral_constant<int, 0xB1>{}));   // quad_perm [1,0,3,2]
-  v = fmaxf(v, move(v, std::integral_constant<int, 0x4E>{}));   // quad_perm [2,3,0,1]
-  v = fmaxf(v, move(v, std::integral_constant<int, 0x141>{}));  // row_half_mirror
-  v = fmaxf(v, move(v, std::integral_constant<int, 0x140>{}));  // row_mirror
+  v = fmaxf(v, dpp<kQuad1032>(v));
+  v = fmaxf(v, dpp<kQuad2301>(v));
+  v = fmaxf(v, dpp<kRowHalfMirror>(v));
+  v = fmaxf(v, dpp<kRowMirror>(v));
   const auto other = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(other[0]), __uint_as_float(other[1]));
 }
@@ -251,8 +254,8 @@ constexpr float kTanhApproxBound = 0x1p-21f;
 // Maximum over each aligned quad of lanes (4i .. 4i+3), on every lane of it,
 // by two DPP quad permutations (all 64 lanes must be active).
 __device__ __forceinline__ float quad_max(float m) {
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0xB1, 0xf, 0xf, true)));
-  return fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0x4E, 0xf, 0xf, true)));
+  m = fmaxf(m, dpp<kQuad1032>(m));
+  return fmaxf(m, dpp<kQuad2301>(m));
 }
 
 // Exact GeGLU values (gelu_mul) of the pending values of each lane (bit i of

@@ -24,7 +24,7 @@ typedef int intx4 __attribute__((ext_vector_type(4)));
 
 constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
 constexpr int kMagicBits = 0x4B400000;
-constexpr int kTileBytes = 1024;       // one 32 x 32 int8 operand block
+constexpr int kTile = 1024;            // bytes of one 32 x 32 int8 operand block
 
 // Operands of one 16 x 16 tile and 32-block: lane 16 g + r holds row r's
 // values 8 g .. 8 g + 7 of both matrices, the weight scale of column r and
@@ -50,13 +50,13 @@ struct NarrowWeights {
   __device__ __forceinline__ NarrowWeights(const int8_t* wq, const float* wd, int ldw, int m, int tc, int blocks)
       : lane_off(narrow_lane_offset()), ldw4(4u * (uint32_t)ldw), nb(blocks) {
     const uint32_t skip = (tc & 1) * 256;
-    rb = buffer_rsrc(wq + (size_t)(tc >> 1) * nb * kTileBytes + skip, (uint32_t)nb * kTileBytes - skip);
+    rb = buffer_rsrc(wq + (size_t)(tc >> 1) * nb * kTile + skip, (uint32_t)nb * kTile - skip);
     rw = buffer_rsrc(wd, 4u * ((uint32_t)(nb - 1) * (uint32_t)ldw + (uint32_t)m));
     woff = 4u * (uint32_t)min(16 * tc + (int)(threadIdx.x & 15), m - 1);
   }
   __device__ __forceinline__ void load(NarrowFrag& f, int kb) const {  // kb uniform; past the end: the last block
     kb = min(kb, nb - 1);
-    f.b = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(rb, lane_off, kb * kTileBytes, 0));
+    f.b = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(rb, lane_off, kb * kTile, 0));
     f.dw = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, woff, (uint32_t)kb * ldw4, 0));
   }
 };
@@ -71,13 +71,13 @@ struct NarrowRows {
       : lane_off(narrow_lane_offset()), ldx4(4u * (uint32_t)ldx), nb(blocks) {
     const int lane = threadIdx.x & 63;
     const uint32_t skip = (tr & 1) * 256;
-    ra = buffer_rsrc(xq + (size_t)(tr >> 1) * nb * kTileBytes + skip, (uint32_t)nb * kTileBytes - skip);
+    ra = buffer_rsrc(xq + (size_t)(tr >> 1) * nb * kTile + skip, (uint32_t)nb * kTile - skip);
     rx = buffer_rsrc(xd, 4u * ((uint32_t)(nb - 1) * (uint32_t)ldx + (uint32_t)n));
     xoff = 4u * (uint32_t)min(16 * tr + 4 * (lane >> 4) + (lane & 3), n - 1);
   }
   __device__ __forceinline__ void load(NarrowFrag& f, int kb) const {
     kb = min(kb, nb - 1);
-    f.a = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(ra, lane_off, kb * kTileBytes, 0));
+    f.a = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(ra, lane_off, kb * kTile, 0));
     f.dx = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, xoff, (uint32_t)kb * ldx4, 0));
   }
 };
@@ -85,7 +85,7 @@ struct NarrowRows {
 // Lane V of each aligned quad, on every lane of the quad.
 template <int V>
 __device__ __forceinline__ float quad_bcast(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), V * 0x55, 0xf, 0xf, true));
+  return dpp<V * 0x55>(x);
 }
 
 // The block's terms (dot * d_w) * d_x: element v is row 4 g + v, column r.

@@ -853,21 +853,17 @@ struct AttentionTileLds {
 };
 
 // Reductions over the 16 lanes of a DPP row, on every lane of it.
-template <int CTRL>
-__device__ __forceinline__ float dpp16(float x) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
-}
 __device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, dpp16<0xB1>(v));
-  v = fmaxf(v, dpp16<0x4E>(v));
-  v = fmaxf(v, dpp16<0x141>(v));
-  return fmaxf(v, dpp16<0x140>(v));
+  v = fmaxf(v, eg2::dpp<eg2::kQuad1032>(v));
+  v = fmaxf(v, eg2::dpp<eg2::kQuad2301>(v));
+  v = fmaxf(v, eg2::dpp<eg2::kRowHalfMirror>(v));
+  return fmaxf(v, eg2::dpp<eg2::kRowMirror>(v));
 }
 __device__ __forceinline__ float row16_sum(float v) {
-  v = v + dpp16<0xB1>(v);
-  v = v + dpp16<0x4E>(v);
-  v = v + dpp16<0x141>(v);
-  return v + dpp16<0x140>(v);
+  v = v + eg2::dpp<eg2::kQuad1032>(v);
+  v = v + eg2::dpp<eg2::kQuad2301>(v);
+  v = v + eg2::dpp<eg2::kRowHalfMirror>(v);
+  return v + eg2::dpp<eg2::kRowMirror>(v);
 }
 
 // A tile whose tokens reach at most kFewKeys keys [first, last) between them:

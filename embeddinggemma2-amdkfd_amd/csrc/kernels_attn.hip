@@ -436,10 +436,6 @@ attention_softmax_kernel(float* __restrict__ scores, const uint4* __restrict__ t
 // waves of longer sequences (fewer pairs per wave hide more latency there).
 constexpr int kGroupPairs = 16;  // pairs per workgroup
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
 // Maximum over each aligned group of LANES lanes, on every lane of it (all
 // 64 lanes active): quad permutations, the other quad of each 8 lanes
 // (row_half_mirror), the other 8 of each 16 (row_mirror), then for 32 the
@@ -447,10 +443,10 @@ __device__ __forceinline__ float dpp_move(float x) {
 template <int LANES>
 __device__ __forceinline__ float group_max(float m) {
   static_assert(LANES == 16 || LANES == 32, "16 or 32 lanes per pair");
-  m = fmaxf(m, dpp_move<0xB1>(m));   // quad_perm [1,0,3,2]
-  m = fmaxf(m, dpp_move<0x4E>(m));   // quad_perm [2,3,0,1]
-  m = fmaxf(m, dpp_move<0x141>(m));  // row_half_mirror
-  m = fmaxf(m, dpp_move<0x140>(m));  // row_mirror
+  m = fmaxf(m, dpp<0xB1>(m));   // quad_perm [1,0,3,2]
+  m = fmaxf(m, dpp<0x4E>(m));   // quad_perm [2,3,0,1]
+  m = fmaxf(m, dpp<0x141>(m));  // row_half_mirror
+  m = fmaxf(m, dpp<0x140>(m));  // row_mirror
   if constexpr (LANES == 32) m = fmaxf(m, __shfl_xor(m, 16, 64));
   return m;
 }

@@ -54,14 +54,13 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 constexpr int kXcds = 8;     // MI355X: 8 XCDs of 32 CUs, each with its own L2
 constexpr int kDepth = 3;    // blocks in flight per wave in gemm_q8_kernel (93 VGPRs: five waves per SIMD)
 constexpr int kUnroll = 6;   // its loop's unrolling: slots rotate mod kDepth, MFMA results mod 2
-constexpr int kTile = 1024;  // one 32 x 32 int8 operand block
 
 extern __shared__ __align__(16) unsigned char gemm_lds[];
 
 // Broadcast of lane V of each 16-lane row to the whole row (row_newbcast).
 template <int V>
 __device__ __forceinline__ float row_bcast(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x150 + V, 0xf, 0xf, true));
+  return dpp<0x150 + V>(x);
 }
 
 // t[v] = (dot[v] * d_w) * d_x(row v) from the biased MFMA result, the

@@ -59,24 +59,18 @@ __device__ __forceinline__ float squares_chain(const TRow* tr, int c) {
   return s;
 }
 
-// DPP moves within 16-lane rows: quad permutation, shift left/right by n
-// lanes. `dpp` writes every lane (lanes shifted in from outside the row
-// read 0 and are not used); `dpp_into` writes only the lanes of the 4-lane
-// banks in BANKS and keeps `old` elsewhere. Choosing lanes by bank mask,
+// DPP moves beside dpp (eg2_device.hpp), which writes every lane: `dpp_into`
+// writes only the lanes of the 4-lane banks in BANKS and keeps `old`
+// elsewhere. Choosing lanes by bank mask,
 // not by a select on the lane index, keeps every source lane active: the
 // compiler may turn a select of two DPP results into an EXEC-masked branch,
 // and a DPP move reads 0 from lanes that EXEC disables.
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
 template <int CTRL, int BANKS>
 __device__ __forceinline__ float dpp_into(float old, float src) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old),
                                                                __builtin_bit_cast(int, src), CTRL, 0xf, BANKS,
                                                                false));
 }
-constexpr int kQuad1032 = 0xB1, kQuad2301 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int kQuad0000 = 0x00, kQuad1111 = 0x55, kQuad2222 = 0xAA, kQuad3333 = 0xFF;
 constexpr int kRowShl4 = 0x104, kRowShr4 = 0x114;  // lane i reads lane i + 4 / i - 4
 constexpr int kBanks02 = 0x5, kBanks13 = 0xA;      // lanes 0-3 and 8-11 / 4-7 and 12-15 of a row

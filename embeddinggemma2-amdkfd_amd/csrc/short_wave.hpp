@@ -328,8 +328,8 @@ short_attention_kernel(const float* __restrict__ qkv, const uint4* __restrict__ 
   float m = -__builtin_inff();
 #pragma unroll
   for (int i = 0; i < KG; ++i) m = fmaxf(m, in(i) ? s[i] : -__builtin_inff());
-  m = fmaxf(m, dpp<0x141>(m));  // row_half_mirror: the other quad of each 8 lanes
-  m = rows4_max(fmaxf(m, dpp<0x140>(m)));  // row_mirror, then the four rows
+  m = fmaxf(m, dpp<kRowHalfMirror>(m));          // the other quad of each 8 lanes
+  m = rows4_max(fmaxf(m, dpp<kRowMirror>(m)));  // the other 8 of the row, then the four rows
 #pragma unroll
   for (int i = 0; i < KG; ++i) {
     const float e = libm::expf_tab(s[i] - m, lds.exp_tab);
