@@ -630,7 +630,7 @@ __device__ __forceinline__ void mm_tile(const EgMM& p) {
         const uintptr_t first = reinterpret_cast<uintptr_t>(p.weight);
         const uintptr_t end = first + (uintptr_t)p.m * (p.k / 32) * 34;
         const bool edge = (blockIdx.x == 0 && first % 4 != 0) || ((blockIdx.x + 1) * TW >= p.m && end % 4 != 0);
-        done = edge ? mm_tile_typed<kQ8Edge, TH, TW>(p, lds.step, lds.part, small, redo)
+        done = __builtin_expect(edge, 0) ? mm_tile_typed<kQ8Edge, TH, TW>(p, lds.step, lds.part, small, redo)
                     : mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, small, redo);
         break;
       }
@@ -1038,7 +1038,6 @@ attention_tile_kernel(EgAttention p) {
     for (int v = 0; v < 4; ++v) m[v] = -__builtin_inff(), l[v] = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4 * T; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    __syncthreads();
     // Rows 4 i + lane / 16 of a key block, dimensions 64 part + 4 (lane % 16) ..
     // (rows past the last repeat it; their scores are masked).
     floatx4 kr[4];
@@ -1050,6 +1049,7 @@ attention_tile_kernel(EgAttention p) {
     };
     bool polluted = false;
     if (first + 16 * w < last) load_k(first + 16 * w, 0);
+    __syncthreads();  // the queries and the exp table are in LDS
     for (unsigned k0 = first + 16 * w; k0 < last; k0 += 16 * kTileWaves) {
       // Scores of keys k0 .. + 15, in four chains.
       floatx4 s[4];
