@@ -29,6 +29,8 @@
 //    then the softmax weights of the chunk (exp through the host libm's
 //    expf restated in eg2_libm.hpp, rescaled by the running maximum between
 //    chunks) go through LDS to the context, where lanes own dimensions.
+//    eg2_op_launch of the whole grid of 512 tokens or more takes tiles of 16
+//    tokens x one head on fp32 MFMA instead (attention_tile_kernel).
 //  - row operators (norm, norm_residual, norm_rope): one wave per row with
 //    the row held in registers as float4s (a single read of the row), the
 //    sum of squares reduced by DPP within 16-lane rows and a 4-way add
@@ -182,11 +184,18 @@ __device__ __forceinline__ void mm_general(const EgMM& p, float* xs, float* ws, 
 // BF16, 1.5e-7 F16, 2.1e-7 F32, where the general form has 4.0e-7.
 //
 // What bounded the general form was its staging: scalar loads, a decode with
-// a branch and a 64-bit address per weight, two barriers per 32 values. On
-// one card, general / this form, Q8_0: eg2_mm 40 x 512 x 512 16.8 / 4.6 us,
-// eg2_mm64 40 x 768 x 1152 63.6 / 7.9, eg2_mm64x64 640 x 512 x 2048 69.7 /
-// 15.4, 2048 x 768 x 1152 159.8 / 29.6 (bf16 weights 14.7 / 4.3, 53.6 / 6.1,
-// 64.0 / 13.1, 153 / 25).
+// a branch and a 64-bit address per weight, two barriers per 32 values. On one
+// card inside a graph, the general form alone / this kernel, us:
+//                               F32           F16           BF16          Q8_0
+//   eg2_mm      40 x 512 x 512   14.4 / 3.9    14.6 / 3.9    14.3 / 3.5    16.4 / 4.1
+//   eg2_mm64    40 x 768 x 1152  87.1 / 8.9    53.8 / 7.1    53.3 / 5.4    63.2 / 6.9
+//   eg2_mm64x64 640 x 512 x 2048 63.4 / 27.1   62.5 / 15.1   63.3 / 12.3   68.6 / 14.5
+//               2048 x 768 x 1152 158 / 62.6   151 / 32.4    152 / 24.5    158 / 28.6
+// Bound by the latency of staging and splitting, F32 weights by the fp32 MFMAs
+// (263 matrix cycles a step and 16 x 16 tile, 74 KB of LDS: two workgroups of 64
+// x 64 per CU). Over one step (k 32) the general form is as fast: 512 x 32 x 512
+// 3.1 / 3.3, 3.2 / 3.3, 3.2 / 3.2, 3.2 / 3.4, 64 x 32 x 64 in 64 x 64 tiles 5.0 / 5.7,
+// 5.2 / 5.1, 5.2 / 4.6, 5.4 / 5.1, but less exact.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));

@@ -29,6 +29,21 @@
  * eg2_gather768 and eg2_attention256x3 are the 768-wide / 3-query-head
  * variants of the embedding-gemma 300M geometry; the others keep the
  * reference kernels' geometry (512-wide gather, 4 query heads).
+ *
+ * What a result depends on, to the last bit:
+ *   eg2_mm*         an output on its own row of x and row of the weights (and
+ *                   on k, the weight type, the tile shape, and whether x lies
+ *                   on 16 bytes and the weights on 16, of Q8_0 on 2): not on
+ *                   the other rows and columns, whatever they hold
+ *   eg2_attention*  below 512 tokens, at another grid, and by symbol a row on
+ *                   its own query, keys and values; eg2_op_launch of the whole
+ *                   grid from 512 tokens on sums a row's keys in an order that
+ *                   follows from where they lie in the packing and from the 15
+ *                   tokens beside it, so the same text in another packing may
+ *                   differ in rounding (both within the 2e-5 of the exact
+ *                   result that the operators are held to). A key whose score
+ *                   is -inf weighs nothing; a row without any other score, and
+ *                   a row with a NaN or +inf score, is NaN.
  */
 #ifndef EG2_OPS_H
 #define EG2_OPS_H

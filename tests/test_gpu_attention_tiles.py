@@ -193,3 +193,31 @@ def test_scattered_ranges(eg2, gpu, op, n, width):
     eg2.ops.op(op, rec, heads * n, 64)
     want = softmax_reference(q, k, v, bounds, n, heads, d, kvs, group, 0)
     assert np.abs(host(y).reshape(n, heads, d) - want).max() <= 2e-5
+
+
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("length", [7, 40, 130])
+def test_packing_moves_rounding_only(eg2, gpu, op, length):
+    """A text alone (the per-row form) and inside a packing of 512 tokens and
+    more, at several places in it: equal but for rounding (each is within 2e-5
+    of the exact result)."""
+    import torch
+
+    heads, d, kvs, _ = OPS[op]
+    rng = np.random.default_rng(length + d)
+    text = [(rng.standard_normal((length, w)) * s).astype(np.float32)
+            for w, s in ((heads * d, d ** -0.5), (kvs, 1), (kvs, 1))]
+    out = []
+    for before, after in ((0, 0), (0, 600), (3, 600), (300, 250), (509, 0)):
+        n = before + length + after
+        q, k, v = (np.concatenate([rng.standard_normal((before, t.shape[1])).astype(np.float32), t,
+                                   rng.standard_normal((after, t.shape[1])).astype(np.float32)]) for t in text)
+        b = np.array([(0, before)] * before + [(before, before + length)] * length +
+                     [(before + length, n)] * after, np.uint32)
+        y = torch.full((n * heads * d,), 7.0, device=gpu)
+        t = [dev(a, gpu) for a in (q, k, v, b.reshape(-1).view(np.int32))]
+        rec = eg2.EgAttention(y.data_ptr(), *(a.data_ptr() for a in t), n, 0)
+        eg2.ops.op(op, rec, heads * n, 64)
+        out.append(host(y).reshape(n, heads * d)[before:before + length])
+    for o in out[1:]:
+        assert np.abs(o - out[0]).max() <= 4e-5
