@@ -1207,14 +1207,8 @@ attention_tile_kernel(EgAttention p) {
   // 0.7 a key where the tile costs 3 + 6.5 per 128 keys of the whole reach
   // (2048 tokens with 8 keys each anywhere: 182 us by keys, 32 by row).
   const unsigned reach = last - first;
-  bool rows = false;
-  if (reach > 256) {
-    unsigned longest = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      longest = max(longest, (unsigned)__builtin_amdgcn_readlane(hi[i & 3] - lo[i & 3], 16 * (i >> 2)));
-    rows = longest + 17 < 9 * ((reach + 127) / 128);
-  }
+  const unsigned longest = max(max(hi[0] - lo[0], hi[1] - lo[1]), max(hi[2] - lo[2], hi[3] - lo[3]));  // of four rows
+  bool rows = reach > 256 && !__any(longest + 17 >= 9 * ((reach + 127) / 128));
   if (!rows)
     rows = reach <= kFewKeys ? attention_few_keys<D, HEADS, KVS>(p, lds, t0, h, kv, lo, hi, first, last) : by_keys();
   if (!rows) return;
