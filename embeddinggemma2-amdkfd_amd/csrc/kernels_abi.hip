@@ -640,7 +640,7 @@ __device__ __forceinline__ void mm_tile(const EgMM& p) {
         const uintptr_t end = first + (uintptr_t)p.m * (p.k / 32) * 34;
         const bool edge = (blockIdx.x == 0 && first % 4 != 0) || ((blockIdx.x + 1) * TW >= p.m && end % 4 != 0);
         done = __builtin_expect(edge, 0) ? mm_tile_typed<kQ8Edge, TH, TW>(p, lds.step, lds.part, small, redo)
-                    : mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, small, redo);
+                                         : mm_tile_typed<8, TH, TW>(p, lds.step, lds.part, small, redo);
         break;
       }
     }
@@ -989,7 +989,8 @@ __device__ __forceinline__ bool attention_few_keys(const EgAttention& p, Attenti
     }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
-    const float inv = hi[v] > lo[v] ? 1.0f / row16_sum(l[v]) : 0.0f;
+    const float den = row16_sum(l[v]);  // every lane active
+    const float inv = hi[v] > lo[v] ? 1.0f / den : 0.0f;
     const unsigned t = t0 + 4 * g + v;
     floatxp o;
 #pragma unroll
