@@ -845,8 +845,9 @@ __device__ __forceinline__ void attention_chunked(const EgAttention& p, unsigned
 // 16 10.3 / 6.3, of 24 12.1 / 10.2, of 64 21.5 / 11.4; window 4 8.7 / 8.1, 16
 // 14.2 / 10.4; at 2048 texts of one token 20.4 / 13.7. (By keys alone 10.0-11.4
 // at 512 whatever the texts, 22 at 2048.) Slower than one wave per row is only
-// what no packing has, neighbours whose few keys lie far apart: 8 keys anywhere,
-// 512 tokens 8.4 / 16.5, 2048 25.8 / 32.6; the rows of a tile share its CU.
+// what no packing has, neighbours whose keys lie far apart: 8 keys anywhere, 512
+// tokens 8.4 / 16.5, 2048 25.8 / 32.6; 100 keys, 1040 tokens 66 / 99, 2048 122 / 165;
+// the rows of a tile share its CU.
 constexpr int kTileWaves = 8;
 // From here the tiles fill half of the CUs; fewer tokens were not looked into.
 constexpr unsigned kTileTokens = 512;
